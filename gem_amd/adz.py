@@ -418,6 +418,7 @@ class BermejoConde:
 L.extra_sigs({
     "adz_ilmc_create": ("i", ["vp", "i", "vp", "vp"]),
     "adz_ilmc_lam": ("i", ["vp", "vp", "vp", "vp"]),
+    "adz_ilmc_set_spin_limit": ("i", ["vp", "i"]),
     "adz_ilmc_free": ("i", ["vp"]),
 })
 
@@ -462,6 +463,9 @@ class IlmcLam:
             raise ValueError("counts needs 3 values per tracer")
         L.check(L.lib().adz_ilmc_lam(self.h, _ptr_at(air_m, self.off), None if counts is None else counts.data_ptr(),
                                      _stream()), "adz_ilmc_lam")
+
+    def set_spin_limit(self, polls):
+        L.check(L.lib().adz_ilmc_set_spin_limit(self.h, int(polls)), "adz_ilmc_set_spin_limit")
 
     def free(self):
         if getattr(self, "h", None) is not None and self.h.value:

@@ -433,8 +433,8 @@ typedef struct adz_ilmc_domain {
 } adz_ilmc_domain;
 
 typedef struct adz_ilmc adz_ilmc;
-/* Register ntr tracers and allocate the visiting lists once (8 bytes per cell of the
- * domain per tracer, the worst case of every cell out of bounds).  Replaces the per-cell
+/* Register ntr tracers and allocate the visiting lists once (8 bytes per 4 cells of a row of
+ * the domain per tracer, the worst case of every cell out of bounds, and a bit per cell).  Replaces the per-cell
  * sweep lists the reference allocates on its first call (ILMC_LAM.F90:138-220); the sweep
  * cells are enumerated in the kernel instead. */
 int adz_ilmc_create(const adz_ilmc_tracer* tr, int ntr, const adz_ilmc_domain* dom, adz_ilmc** out);
@@ -443,9 +443,11 @@ int adz_ilmc_create(const adz_ilmc_tracer* tr, int ntr, const adz_ilmc_domain* d
  * counts (DEVICE int64 [3*ntr] or NULL) receives per tracer: sweeps that moved mass
  * (reset(:,5)), min resets and max resets (reset(:,3:4)).  Tracer arrays must not
  * overlap, and calls on one plan must not overlap (they share its visiting lists).  No host
- * synchronisation: capturable (one launch per hyperplane of the domain, about
- * ni + (2S+1) nj + (2S+1)^2 nk launches). */
+ * synchronisation: capturable (six launches; the visits are one). */
 int adz_ilmc_lam(adz_ilmc* il, const void* air_m, long long* counts, adz_stream stream);
+/* Polls of one wait between visits before it gives up (2^22 by default, some seconds).  The
+ * visits left are then made by one wave in the reference's order: the result is the same. */
+int adz_ilmc_set_spin_limit(adz_ilmc* il, int polls);
 int adz_ilmc_free(adz_ilmc* il);
 
 /* ------------------------------------------------------------------------------------
