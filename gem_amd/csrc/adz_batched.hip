@@ -36,6 +36,9 @@ struct DevItem {
   long minoff;      // lowest source element a stencil may read, from element (1,1,1)
   unsigned span;    // bytes of FP32 source from minoff that stencils may read (0: too large
                     // for 32-bit buffer offsets; global loads are used)
+  long omin;        // lowest destination element of the box, from element (1,1,1)
+  unsigned dspan;   // elements of the destination from omin to the box's last one (0: too many)
+  int pad_;
   long npts, ptiles, ngroups, tile0;
   const void* const* src;
   void* const* dst;
@@ -43,6 +46,12 @@ struct DevItem {
   void* const* mn;
   void* const* mx;
 };
+
+// Can boxes of elements of `size` bytes be staged, and their outputs stored, at 32-bit byte
+// offsets?
+__host__ __device__ inline bool stageable(const DevItem& it, int size) {
+  return it.span && it.dspan && (long)(it.span / 4) * size < 0x7fffffffL && (long)it.dspan * size < 0x7fffffffL;
+}
 
 struct PlanArgs {
   const DevItem* items;
@@ -91,41 +100,41 @@ struct ItemFields {  // field pointer tables of a plan item (device arrays in gl
 #undef ADZ_CONST
 };
 
-// Narrow and store one target's outputs at dst offset o: the value (clipped to [min, max]
-// with ADZ_POST_CLIP) and, with ADZ_POST_STORE, lin clipped to [min, max], min and max.
-// TC is the arithmetic type (FP64 for the reference's arithmetic, FP32 for the mixed form).
-template <class TF, int MATH, int POST, class Fields, class TC>
-__device__ __forceinline__ void store_out(const Fields& F, int f, long o, TC v, TC l, TC mi, TC ma) {
-  typename GPtr<TF>::type d = (typename GPtr<TF>::type)F.d(f);
+// Narrow one target's outputs: the value (clipped to [min, max] with ADZ_POST_CLIP) and, with
+// ADZ_POST_STORE, lin clipped to [min, max], min and max.  TC is the arithmetic type (FP64 for
+// the reference's arithmetic, FP32 for the mixed form).
+template <class TF, int MATH, int POST, class TC>
+__device__ __forceinline__ void narrow_out(TC v, TC l, TC mi, TC ma, TF* vs, TF* ls, TF* mis, TF* mas) {
   if (MATH == ADZ_MATH_REF) {
+    *vs = from_f64<TF>(v);
     if (POST) {
       // adz_interp_hlt.F90:158-160 narrows each to real before clipping lin
-      TF ls = from_f64<TF>(l), mis = from_f64<TF>(mi), mas = from_f64<TF>(ma);
-      TF vs = from_f64<TF>(v);
-      if (POST & ADZ_POST_CLIP) vs = from_f64<TF>(fmax(to_f64(mis), fmin(to_f64(mas), to_f64(vs))));
-      d[o] = vs;
-      if (POST & ADZ_POST_STORE) {
-        ((typename GPtr<TF>::type)F.l(f))[o] = from_f64<TF>(fmax(to_f64(mis), fmin(to_f64(mas), to_f64(ls))));
-        ((typename GPtr<TF>::type)F.n(f))[o] = mis;
-        ((typename GPtr<TF>::type)F.x(f))[o] = mas;
-      }
-    } else {
-      d[o] = from_f64<TF>(v);
+      *mis = from_f64<TF>(mi); *mas = from_f64<TF>(ma);
+      if (POST & ADZ_POST_CLIP) *vs = from_f64<TF>(fmax(to_f64(*mis), fmin(to_f64(*mas), to_f64(*vs))));
+      if (POST & ADZ_POST_STORE)
+        *ls = from_f64<TF>(fmax(to_f64(*mis), fmin(to_f64(*mas), to_f64(from_f64<TF>(l)))));
     }
+  } else if (POST) {
+    *mis = from_f32<TF>(mi); *mas = from_f32<TF>(ma);
+    *vs = from_f32<TF>(snap_to_range(v, mi, ma));
+    if (POST & ADZ_POST_CLIP) *vs = from_f32<TF>(fmaxf(to_f32(*mis), fminf(to_f32(*mas), to_f32(*vs))));
+    if (POST & ADZ_POST_STORE)
+      *ls = from_f32<TF>(fmaxf(to_f32(*mis), fminf(to_f32(*mas), to_f32(from_f32<TF>(l)))));
   } else {
-    if (POST) {
-      TF ls = from_f32<TF>(l), mis = from_f32<TF>(mi), mas = from_f32<TF>(ma);
-      TF vs = from_f32<TF>(snap_to_range(v, mi, ma));
-      if (POST & ADZ_POST_CLIP) vs = from_f32<TF>(fmaxf(to_f32(mis), fminf(to_f32(mas), to_f32(vs))));
-      d[o] = vs;
-      if (POST & ADZ_POST_STORE) {
-        ((typename GPtr<TF>::type)F.l(f))[o] = from_f32<TF>(fmaxf(to_f32(mis), fminf(to_f32(mas), to_f32(ls))));
-        ((typename GPtr<TF>::type)F.n(f))[o] = mis;
-        ((typename GPtr<TF>::type)F.x(f))[o] = mas;
-      }
-    } else {
-      d[o] = from_f32<TF>(v);
-    }
+    *vs = from_f32<TF>(v);
+  }
+}
+
+// Narrow and store one target's outputs at dst offset o.
+template <class TF, int MATH, int POST, class Fields, class TC>
+__device__ __forceinline__ void store_out(const Fields& F, int f, long o, TC v, TC l, TC mi, TC ma) {
+  TF vs, ls, mis, mas;
+  narrow_out<TF, MATH, POST>(v, l, mi, ma, &vs, &ls, &mis, &mas);
+  ((typename GPtr<TF>::type)F.d(f))[o] = vs;
+  if (POST & ADZ_POST_STORE) {
+    ((typename GPtr<TF>::type)F.l(f))[o] = ls;
+    ((typename GPtr<TF>::type)F.n(f))[o] = mis;
+    ((typename GPtr<TF>::type)F.x(f))[o] = mas;
   }
 }
 
@@ -262,6 +271,96 @@ __device__ __forceinline__ void per_lane(const DevItem& it, const Fields& F, int
     if (ok)
       eval_store<TF, MATH, POST, Fields>(F, f, (typename GPtr<TF>::ctype)F.s(f) + x.off, gni, gnij, x.zlinear, cw, o);
     else if (valid) store_nan<TF, MATH, POST>(F, f, o);
+  }
+}
+
+// The same for the few tiles whose box is not staged, one stencil row at a time: each value
+// goes through the operations of the evaluators above in their order, but only one row is
+// held, so that the staged kernels, which contain this path, keep their registers for the
+// staged one.
+template <class TF, int MATH, int POST, class Fields>
+__device__ __forceinline__ void per_lane_rows(const DevItem& it, const Fields& F, int f0, int f1, const Index& x,
+                                              bool ok, bool valid, const double* cw, long o) {
+  typedef typename std::conditional<MATH == ADZ_MATH_REF, double, float>::type TC;
+  typedef typename std::conditional<MATH == ADZ_MATH_REF && sizeof(TF) == 8, double, float>::type TM;
+  const TC* c = (const TC*)cw;
+  const long gni = it.lv.ni, o1 = x.zlinear ? 0 : (long)it.lv.nij, o2 = o1 + it.lv.nij, o3 = o2 + o1;
+  auto wide = [](TF v) -> TC {
+    if constexpr (MATH == ADZ_MATH_REF) return to_f64<TF>(v);
+    else return to_f32<TF>(v);
+  };
+  auto fm = [](TC p, TC q, TC r) -> TC {
+    if constexpr (MATH == ADZ_MATH_REF) return fma(p, q, r);
+    else return fmaf(p, q, r);
+  };
+#pragma unroll 1
+  for (int f = f0; f < f1; f++) {
+    if (!ok) {
+      if (valid) store_nan<TF, MATH, POST>(F, f, o);
+      continue;
+    }
+    const typename GPtr<TF>::ctype s0 = (typename GPtr<TF>::ctype)F.s(f) + x.off;
+    TC ya[4] = {0, 0, 0, 0}, vl[4] = {0, 0, 0, 0};
+    TM vmi[4] = {0, 0, 0, 0}, vma[4] = {0, 0, 0, 0}, lo = 0, hi = 0;
+#pragma unroll 1
+    for (int r = 0; r < 4; r++) {
+      const typename GPtr<TF>::ctype s = s0 + r * gni;
+      const TC cy = r == 0 ? c[4] : (r == 1 ? c[5] : (r == 2 ? c[6] : c[7]));
+      TF p1[4], p2[4];
+#pragma unroll
+      for (int i = 0; i < 4; i++) {
+        p1[i] = s[o1 + i];
+        p2[i] = s[o2 + i];
+        TC za = wide(s[i]) * c[8];
+        za = fm(wide(p1[i]), c[9], za);
+        za = fm(wide(p2[i]), c[10], za);
+        za = fm(wide(s[o3 + i]), c[11], za);
+        ya[i] = r == 0 ? za * cy : fm(za, cy, ya[i]);
+      }
+      if (POST) {
+        if (r == 1 || r == 2)
+#pragma unroll
+          for (int i = 0; i < 4; i++) {
+            TC vz = wide(p1[i]) * c[18];
+            vz = fm(wide(p2[i]), c[19], vz);
+            vl[i] = r == 1 ? vz * c[16] : fm(vz, c[17], vl[i]);
+          }
+        if constexpr (MATH == ADZ_MATH_REF) {
+#pragma unroll
+          for (int i = 1; i < 3; i++) {
+            const TM a = (TM)to_f64<TF>(p1[i]), b = (TM)to_f64<TF>(p2[i]);
+            if (r == 0) { vmi[i] = a; vma[i] = a; }
+            else { vmi[i] = (vmi[i] < a) ? vmi[i] : a; vma[i] = (vma[i] > a) ? vma[i] : a; }
+            vmi[i] = (vmi[i] < b) ? vmi[i] : b;
+            vma[i] = (vma[i] > b) ? vma[i] : b;
+          }
+        } else {
+          const float a1 = to_f32<TF>(p1[1]), a2 = to_f32<TF>(p1[2]), b1 = to_f32<TF>(p2[1]), b2 = to_f32<TF>(p2[2]);
+          if (r == 0) lo = hi = a1;
+          lo = fminf(fminf(lo, a1), fminf(a2, fminf(b1, b2)));
+          hi = fmaxf(fmaxf(hi, a1), fmaxf(a2, fmaxf(b1, b2)));
+        }
+      }
+    }
+    TC v, l = 0, mi = 0, ma = 0;
+    if constexpr (MATH == ADZ_MATH_REF) {
+      const TC y0 = ya[0] * c[0], y1 = ya[1] * c[1], y2 = ya[2] * c[2], y3 = ya[3] * c[3];
+      v = (y0 + y2) + (y1 + y3);
+    } else {
+      v = fm(ya[3], c[3], fm(ya[2], c[2], fm(ya[1], c[1], ya[0] * c[0])));
+    }
+    if (POST) {
+      const TC l0 = vl[0] * c[12], l1 = vl[1] * c[13], l2 = vl[2] * c[14], l3 = vl[3] * c[15];
+      l = (l0 + l2) + (l1 + l3);
+      if constexpr (MATH == ADZ_MATH_REF) {
+        mi = (TC)((vmi[1] < vmi[2]) ? vmi[1] : vmi[2]);
+        ma = (TC)((vma[1] > vma[2]) ? vma[1] : vma[2]);
+      } else {
+        mi = lo;
+        ma = hi;
+      }
+    }
+    store_out<TF, MATH, POST>(F, f, o, v, l, mi, ma);
   }
 }
 
@@ -876,51 +975,171 @@ __device__ __forceinline__ void shared_tile(const DevItem& it, const Fields& F, 
 // into LDS once per field by all four waves with 16-byte buffer-to-LDS DMA, and every lane
 // then reads its 64 stencil values from LDS.  Per-lane loads spend 16 address slots of the
 // texture unit per point-field; the box needs about 2 (a 68 x 7 x 4 box is 28 rows of 18
-// quads for 256 targets).  LDS rows have a fixed pitch of 20 quads (80 floats): the rows of
-// a buffer are dense, each DMA instruction fills 64 consecutive quads of them, and the 16
-// values of one stencil plane lie within 1 KB of one per-lane base, so they are read in
-// pairs at immediate offsets.  The DMA starts each row at a 16-byte boundary, so a field
-// whose base is not 16-byte aligned lands shifted by `sh` floats (0..3), added to the
-// bases.  Two LDS buffers with static roles: field f+1 is in flight while field f is
-// evaluated; one block barrier per field.  Tiles whose box does not fit (more than
-// kMaxRows5 rows or 77 columns), rows not a multiple of 4 floats apart, or sources beyond
-// 32-bit buffer offsets use per-lane loads.  The arithmetic and its order are those of the
-// per-lane path, so both give the same bits.  Staging mode 6 is the same with tiles of 64 x 8
-// targets and blocks of eight waves: a box of 8 target rows spans ~12 source rows against
-// ~7 for 4, so about a fifth fewer DMA bytes per target, and the tile's fixed work (box
-// extents, DMA offsets) is shared by twice the targets.  Staging modes 7 and 8 take tiles of
-// 64 x 4 targets over 2 and 4 consecutive levels (blocks of 8 and 16 waves, one wave per
-// target row and level).  A source plane is read by the stencils of about four levels, so
-// the planes of a box dominate its volume: at c5, a box over 64 x 4 x 4 targets holds ~7
-// rows of ~7 planes against ~11 rows of 4 planes for 64 x 8 x 1, about 14 against 25 DMA
-// bytes per target.
-constexpr int kQRow = 20;                               // 16-byte quads per LDS row
-constexpr int kPitch5 = 4 * kQRow;                      // floats per LDS row
-constexpr int kMaxRows5 = kMaxRows * kPitch / kPitch5;  // rows per buffer (the stage-1 buffers)
-constexpr int kTJ6 = 8;                                 // target rows of a staging-mode-6 tile
-constexpr int kMaxRows8 = 96;                           // rows per buffer of the 16-wave blocks
-// rows per LDS buffer for blocks of W waves: 16-wave blocks run one per CU and take larger
-// buffers (2 x 30 KB); the others keep the stage-1 buffer size, two blocks per CU
-template <int W> constexpr int box_rows() { return W >= 16 ? kMaxRows8 : kMaxRows5; }
-template <int W> constexpr int dma_max() { return (box_rows<W>() * kQRow + 64 * W - 1) / (64 * W); }
-static_assert(4 * dma_max<4>() * 64 >= kMaxRows5 * kQRow && 8 * dma_max<8>() * 64 >= kMaxRows5 * kQRow &&
-                  16 * dma_max<16>() * 64 >= kMaxRows8 * kQRow && dma_max<4>() <= 32,
-              "DMA slots cover a full buffer");
-static_assert(kMaxRows5 < 128 && kMaxRows8 < 128, "row split by a float reciprocal below");
+// quads for 256 targets).
+//   * LDS rows have a fixed pitch of 96 elements: row and plane changes between the lanes of
+//     a wave leave their banks apart (96 floats are three times round the 32 banks; a pitch
+//     of 80 moved each row by 16 banks, and 40 % of the LDS cycles were conflicts: 16
+//     subdomains x 6 fields 6.1 ms against 5.3), and a stencil plane is read in pairs at
+//     immediate offsets from its base and from its base three rows on.
+//   * The quads start at the box's first column: a 16-byte DMA takes any 4-byte-aligned
+//     address, so rows of any length and fields at any element are staged (an aligned start
+//     would shift each row by its own 0..3 floats; layouts with rows not a multiple of 4
+//     floats apart, as the extended ones of halo 5, took per-lane loads: 6.96 -> 6.3 ms).
+//   * Field f + 1 is in flight while field f is evaluated from the other of two buffers, one
+//     block barrier per field, and no wave waits for its own stores (dma_tile).
+//   * A field's pointers are loaded a step ahead, outside the LDS reads.
+// Tiles whose box does not fit (more than box_rows rows or 96 columns) or reaches the end of
+// 32-bit buffer offsets use per-lane loads, in the same arithmetic and order: the same bits.
+// Staging mode 6 has tiles of 64 x 8 targets and blocks of eight waves, modes 7 and 8 tiles
+// of 64 x 4 targets over 2 and 4 consecutive levels (blocks of 8 and 16 waves, one wave per
+// target row and level).  A source plane is read by the stencils of about four levels, so the
+// planes of a box dominate its volume: DMA bytes per target and field on 512 x 384 x 84 are
+// 39.7 for 64 x 4 x 1, 29.9 for 64 x 8 x 1, 24.5 for 64 x 4 x 2 and 16.9 for 64 x 4 x 4.
+// What bounds it: 6 fields, no lin/min/max (stage 7): LDS reads (256 B per point-field, 58 %
+// of the cycles, a quarter of those still bank conflicts), FP32 arithmetic (100 instructions
+// per field and 40 per field for the tile's indexes, weights and box: 54 %) and the texture
+// unit's DMA (41 %), none hidden completely behind another with 16 waves per CU.
+constexpr int kPitch5 = 96;                // elements per LDS row
+constexpr int kTJ6 = 8;                    // target rows of a staging-mode-6 tile
+template <class TF> constexpr int quads_per_row() { return kPitch5 * (int)sizeof(TF) / 16; }
+// rows per LDS buffer for blocks of W waves
+template <int W> constexpr int box_rows() { return W >= 8 ? 85 : 64; }
+// DMA instructions per wave and field: all are issued for every field (lanes without a quad
+// ask for one out of range and get zeros), so that a wave can count what is outstanding
+template <class TF, int W> constexpr int dma_per_wave() {
+  return (box_rows<W>() * quads_per_row<TF>() + 64 * W - 1) / (64 * W);
+}
+template <class TF, int W> constexpr int box_elems() { return dma_per_wave<TF, W>() * W * 1024 / (int)sizeof(TF); }
+static_assert(box_rows<4>() < 128 && box_rows<16>() < 128, "row split by a float reciprocal below");
 
-template <int MATH, int POST, class TP, int TH, int TL, class Fields>
-__device__ __forceinline__ void dma_tile(const DevItem& it, const Fields& F, long ptile, int f0, int f1,
-                                         float* boxA, float* boxB, int* red, int level_inner) {
+// s_waitcnt immediate (gfx9): at most n vector-memory operations outstanding, the other
+// counters not waited for
+constexpr int vmcnt_imm(int n) { return (n & 15) | (7 << 4) | (15 << 8) | ((n >> 4) << 14); }
+
+template <class TF>
+__device__ __forceinline__ void buf_store(TF v, __amdgpu_buffer_rsrc_t rs, int off) {
+  if constexpr (sizeof(TF) == 8) {
+    typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), rs, off, 0, 0);
+  } else if constexpr (sizeof(TF) == 4) {
+    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), rs, off, 0, 0);
+  } else {
+    __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(unsigned short, v), rs, off, 0, 0);
+  }
+}
+
+// Block-wide minimum of 6 values, returned as scalars, with one barrier and no reading of
+// other waves' words: each wave reduces by DPP moves (pairs, quads, half-rows, rows of 16, then
+// the row broadcasts of 15 and 31 leave the minimum in lane 63), lanes 0..5 of the wave put
+// the six into LDS with one min each, and after the barrier lanes 0..5 read them back.  `red`
+// holds three sets of 6 words, all `kFar` at first; tile number t uses set t % 3 and clears
+// set (t + 1) % 3, which was last read before the barrier of tile t - 1.
+constexpr int kFar = 1 << 30;
+template <int CTRL, int ROWS = 0xF>
+__device__ __forceinline__ int dpp_min(int v) {
+  if constexpr (ROWS == 0xF) return min(v, __builtin_amdgcn_mov_dpp(v, CTRL, 0xF, 0xF, true));
+  else return min(v, __builtin_amdgcn_update_dpp(0x7fffffff, v, CTRL, ROWS, 0xF, false));
+}
+__device__ __forceinline__ void tile_min6(int* v, int* red, unsigned t) {
+  const int lane = threadIdx.x & 63;
+  int mine = kFar;
+#pragma unroll
+  for (int q = 0; q < 6; q++) {
+    int m = v[q];
+    m = dpp_min<0xB1>(m);        // quad_perm [1,0,3,2]
+    m = dpp_min<0x4E>(m);        // quad_perm [2,3,0,1]
+    m = dpp_min<0x141>(m);       // row_half_mirror
+    m = dpp_min<0x140>(m);       // row_mirror
+    m = dpp_min<0x142, 0xA>(m);  // row_bcast:15 into rows 1 and 3
+    m = dpp_min<0x143, 0xC>(m);  // row_bcast:31 into rows 2 and 3
+    int w = __builtin_amdgcn_readlane(m, 63);
+    asm volatile("" : "+s"(w));  // here, by every lane: the reduction must not sink into a branch
+    mine = lane == q ? w : mine;
+  }
+  int* set = red + 6 * (t % 3);
+  if (lane < 6) atomicMin(set + lane, mine);
+  if (threadIdx.x < 6) red[6 * ((t + 1) % 3) + threadIdx.x] = kFar;
+  __syncthreads();
+  const int r = set[min(lane, 5)];
+#pragma unroll
+  for (int q = 0; q < 6; q++) v[q] = __builtin_amdgcn_readlane(r, q);
+}
+
+// The outputs of one target in the reference's arithmetic from LDS, a stencil row at a time
+// with the next row's values on their way: the operations of tricub_ref_a and mono_extra_a in
+// their order, but with two rows held instead of as many as the compiler would read ahead, so
+// that the kernel fits 128 registers (four waves per SIMD; reading ahead took 182 and two).
+template <class TF, int POST, class Acc>
+__device__ __forceinline__ void eval_rows(Acc at, const double* c, double* v, double* l, double* mi, double* ma) {
+  typedef typename std::conditional<sizeof(TF) == 8, double, float>::type TM;
+  double ya[4], vl[4] = {0, 0, 0, 0};
+  TM vmi[4], vma[4];
+  TF row[2][4][4];
+  auto load = [&](int r) {
+#pragma unroll
+    for (int z = 0; z < 4; z++)
+#pragma unroll
+      for (int i = 0; i < 4; i++) row[r & 1][z][i] = at(r, z, i);
+  };
+  load(0);
+#pragma unroll
+  for (int r = 0; r < 4; r++) {
+    if (r < 3) load(r + 1);
+    const TF(&q)[4][4] = row[r & 1];
+    double w1[4], w2[4];
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      w1[i] = to_f64<TF>(q[1][i]);
+      w2[i] = to_f64<TF>(q[2][i]);
+      double za = to_f64<TF>(q[0][i]) * c[8];
+      za = fma(w1[i], c[9], za);
+      za = fma(w2[i], c[10], za);
+      za = fma(to_f64<TF>(q[3][i]), c[11], za);
+      ya[i] = (r == 0) ? za * c[4] : fma(za, c[4 + r], ya[i]);
+    }
+    if (POST) {
+#pragma unroll
+      for (int i = 1; i < 3; i++) {
+        const TM a = (TM)q[1][i], b = (TM)q[2][i];
+        if (r == 0) { vmi[i] = a; vma[i] = a; }
+        else { vmi[i] = (vmi[i] < a) ? vmi[i] : a; vma[i] = (vma[i] > a) ? vma[i] : a; }
+        vmi[i] = (vmi[i] < b) ? vmi[i] : b;
+        vma[i] = (vma[i] > b) ? vma[i] : b;
+      }
+      if (r == 1 || r == 2)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          double vz = w1[i] * c[18];
+          vz = fma(w2[i], c[19], vz);
+          vl[i] = r == 1 ? vz * c[16] : fma(vz, c[17], vl[i]);
+        }
+    }
+    // the row is done with here, and no further one is read before
+    asm volatile("" : "+v"(ya[0]), "+v"(ya[1]), "+v"(ya[2]), "+v"(ya[3])::"memory");
+    if (POST) asm volatile("" : "+v"(vl[0]), "+v"(vl[1]), "+v"(vl[2]), "+v"(vl[3]));
+  }
+  const double y0 = ya[0] * c[0], y1 = ya[1] * c[1], y2 = ya[2] * c[2], y3 = ya[3] * c[3];
+  *v = (y0 + y2) + (y1 + y3);
+  if (POST) {
+    *mi = (double)((vmi[1] < vmi[2]) ? vmi[1] : vmi[2]);
+    *ma = (double)((vma[1] > vma[2]) ? vma[1] : vma[2]);
+    const double l0 = vl[0] * c[12], l1 = vl[1] * c[13], l2 = vl[2] * c[14], l3 = vl[3] * c[15];
+    *l = (l0 + l2) + (l1 + l3);
+  }
+}
+
+template <class TF, int MATH, int POST, class TP, int TH, int TL, class Fields>
+__device__ __forceinline__ void dma_tile(const DevItem& it, const Fields& F, long ptile, int f0, int f1, TF* boxA,
+                                         TF* boxB, int* red, unsigned nth, int level_inner) {
   constexpr int W = TH * TL;                  // waves of the block: one per target row and level
-  constexpr int kRows = box_rows<W>();
-  constexpr int kDmaMax = dma_max<W>();       // DMA instructions per wave and field
+  constexpr int kRows = box_rows<W>(), kN = dma_per_wave<TF, W>();
+  constexpr int kQ = quads_per_row<TF>(), kE = 16 / (int)sizeof(TF), SZ = (int)sizeof(TF);
+  constexpr int kSt = POST & ADZ_POST_STORE ? 4 : 1;  // stores per field
   const int lane = threadIdx.x & (kTI - 1), wv = threadIdx.x / kTI;
   const TileXY tc = tile_at(it, ptile, level_inner, kTI, TH, TL);
   const int ii = tc.ib * kTI + lane, jj = tc.jb * TH + wv % TH, kk = tc.kk * TL + wv / TH;
   const bool valid = ii < it.nx && jj < it.ny && kk < it.nz;
-  const int i = it.i0 + ii, j = it.j0 + jj, k = it.k0 + kk;
   const long p = (long)ii + (long)it.nx * (jj + (long)it.ny * kk);
-  const long o = (long)(i - 1) + (long)it.dni * ((j - 1) + (long)it.dnj * (k - 1));
   Index x;
   bool ok = false;
   if (valid) {
@@ -933,52 +1152,47 @@ __device__ __forceinline__ void dma_tile(const DevItem& it, const Fields& F, lon
     if (MATH == ADZ_MATH_REF) weights_ref(x, it.lv, cw);
     else weights_f32(x, it.lv, (float*)cw);
   }
-  const int big = 1 << 30;
-  int ext[6] = {ok ? x.ix - 1 : big, ok ? -(x.ix + 2) : big, ok ? x.iy - 1 : big, ok ? -(x.iy + 2) : big,
-                ok ? x.pz : big, ok ? -(x.pz + (x.zlinear ? 1 : 3)) : big};
-  block_min6<W>(ext, red);
-#pragma unroll
-  for (int q = 0; q < 6; q++) ext[q] = __builtin_amdgcn_readfirstlane(ext[q]);  // block-uniform
+  int ext[6] = {ok ? x.ix - 1 : kFar, ok ? -(x.ix + 2) : kFar, ok ? x.iy - 1 : kFar, ok ? -(x.iy + 2) : kFar,
+                ok ? x.pz : kFar, ok ? -(x.pz + (x.zlinear ? 1 : 3)) : kFar};
+  tile_min6(ext, red, nth);
   const int x0 = ext[0], y0 = ext[2], z0 = ext[4];
-  if (x0 == big) {  // no target of the tile has an in-range stencil
+  const long od = (long)ii + (long)it.dni * (jj + (long)it.dnj * kk);  // destination element from omin
+  if (x0 == kFar) {  // no target of the tile has an in-range stencil
     if (valid)
-      for (int f = f0; f < f1; f++) store_nan<float, MATH, POST>(F, f, o);
+      for (int f = f0; f < f1; f++) store_nan<TF, MATH, POST>(F, f, od + it.omin);
     return;
   }
   const int nxb = -ext[1] - x0 + 1, nyb = -ext[3] - y0 + 1, nzb = -ext[5] - z0 + 1;
-  const int nrows = nyb * nzb, cpr = (nxb + 3 + 3) / 4;  // quads per row, room for the shift
+  const int nrows = nyb * nzb, cpr = (nxb + kE - 1) / kE;  // quads per row
   const long gni = it.lv.ni, gnij = it.lv.nij;
-  // every quad the DMA reads, for any shift 0..3, inside the buffer's range [minoff,
-  // minoff + span): a quad reaching outside would read zeros for its in-range floats too
-  const long first = (long)(x0 - 1 - 3) + (long)(y0 - 1) * gni + (long)z0 * gnij - it.minoff;
-  const long last = (long)(x0 - 1) + 4L * cpr - 1 + (long)(y0 + nyb - 2) * gni + (long)(z0 + nzb - 1) * gnij -
+  // every quad the DMA reads inside the buffer's range [minoff, minoff + span): a quad
+  // reaching outside would read zeros for its in-range elements too
+  const long first = (long)(x0 - 1) + (long)(y0 - 1) * gni + (long)z0 * gnij - it.minoff;
+  const long last = (long)(x0 - 1) + (long)kE * cpr - 1 + (long)(y0 + nyb - 2) * gni + (long)(z0 + nzb - 1) * gnij -
                     it.minoff;
-  if (nrows > kRows || cpr > kQRow || !it.span || (gni & 3) || (gnij & 3) || first < 0 ||
-      (last + 1) * 4 > (long)it.span) {
-    per_lane<float, MATH, POST>(it, F, f0, f1, x, ok, valid, cw, o);
+  const unsigned span = it.span / 4 * SZ;  // (it.span is in bytes of FP32)
+  if (nrows > kRows || cpr > kQ || !stageable(it, SZ) || first < 0 || (last + 1) * 4 > (long)it.span) {
+    per_lane_rows<TF, MATH, POST>(it, F, f0, f1, x, ok, valid, cw, od + it.omin);
     return;
   }
   // this lane's DMA slots: instruction q of wave wv fills the 64 quads g*64 .. g*64+63 of
-  // the buffer (g = wv + W q), quad Q = row Q / kQRow, column quad Q % kQRow; element
-  // offsets from minoff of the lane's quad (before the field's shift)
-  // (32-bit arithmetic: every offset is below span < 2^31 bytes; R / nyb by a float
-  // reciprocal, exact since R < 128 and nyb < 128 keep (R + 0.5) / nyb >= 1/256 from an
-  // integer, far above the float product's error; slots with R >= nrows are inactive)
-  const int rel0 = (int)__builtin_amdgcn_readfirstlane((int)((long)(x0 - 1) + (long)(y0 - 1) * gni +
-                                                             (long)z0 * gnij - it.minoff));
+  // the buffer (g = wv + W q), quad Q = row Q / kQ, column quad Q % kQ; byte offsets from
+  // minoff of the lane's quad, or `span` (out of range) where the box has none
+  // (32-bit arithmetic: every offset is below 2^31; R / nyb by a float reciprocal, exact
+  // since R < 128 and nyb < 128 keep (R + 0.5) / nyb >= 1/256 from an integer, far above the
+  // float product's error)
+  const int rel0 = (int)__builtin_amdgcn_readfirstlane((int)first);
   const int ni32 = (int)gni, nij32 = (int)gnij;
   const float rnyb = 1.0f / (float)nyb;
-  int rel[kDmaMax];
-  unsigned act = 0;
+  int rel[kN];
 #pragma unroll
-  for (int q = 0; q < kDmaMax; q++) {
+  for (int q = 0; q < kN; q++) {
     const int Q = (wv + W * q) * 64 + lane;
-    const int R = Q / kQRow, cq = Q - R * kQRow;
+    const int R = Q / kQ, cq = Q - R * kQ;
     const int zz = (int)(((float)R + 0.5f) * rnyb), yy = R - zz * nyb;
-    rel[q] = rel0 + 4 * cq + yy * ni32 + zz * nij32;
-    if (R < nrows && cq < cpr) act |= 1u << q;
+    rel[q] = R < nrows && cq < cpr ? SZ * (rel0 + kE * cq + yy * ni32 + zz * nij32) : (int)span;
   }
-  // plane bases of this lane's stencil in a buffer (floats, before the field's shift)
+  // plane bases of this lane's stencil in a buffer (elements)
   int lb[4] = {0, 0, 0, 0};
   if (ok) {
     const int r0 = x.iy - 1 - y0, pz0 = x.pz - z0, c0 = x.ix - 1 - x0;
@@ -988,56 +1202,91 @@ __device__ __forceinline__ void dma_tile(const DevItem& it, const Fields& F, lon
       lb[z] = (r0 + nyb * (pz0 + dz)) * kPitch5 + c0;
     }
   }
-  auto shift = [&](int f) {  // floats between the field's 16-byte boundary and column x0
-    const unsigned long long b = (unsigned long long)F.s(f);
-    return (int)(((b >> 2) + (unsigned)(x0 - 1)) & 3);
+  const int so = valid ? (int)od * SZ : (int)it.dspan * SZ;  // invalid lanes store out of range (dropped)
+  // A field's pointers, loaded a step ahead and held in scalar registers: a scalar load in the
+  // middle of a step would share its counter with the LDS reads and make them all wait.
+  struct Ptr {
+    const void* s;
+    void *d, *l, *n, *x;
   };
-  auto issue = [&](int f, float* buf) {
-    const int sh = shift(f);
-    const __amdgpu_buffer_rsrc_t rs = field_rsrc((const float*)F.s(f) + it.minoff, it.span);
-#pragma unroll
-    for (int q = 0; q < kDmaMax; q++) {
-      if (act & (1u << q))
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(
-            rs, (__attribute__((address_space(3))) void*)(buf + (wv + W * q) * 256), 16,
-            (rel[q] - sh) * 4, 0, 0, 0);
+  auto source = [&](int f, Ptr* q) {  // (past the last field: any source, nothing is in range)
+    q->s = F.s(f < f1 ? f : f0);
+    asm volatile("" : "+s"(q->s));
+  };
+  auto target = [&](int f, Ptr* q) {
+    q->d = F.d(f < f1 ? f : f0);
+    asm volatile("" : "+s"(q->d));
+    if (POST & ADZ_POST_STORE) {
+      q->l = F.l(f < f1 ? f : f0); q->n = F.n(f < f1 ? f : f0); q->x = F.x(f < f1 ? f : f0);
+      asm volatile("" : "+s"(q->l), "+s"(q->n), "+s"(q->x));
     }
   };
-  // Every lane evaluates (one without a stencil reads its buffer's first values and stores
-  // NaN where valid): with one store site the field index and output pointers stay scalar.
+  auto issue = [&](const void* src, bool on, TF* buf) {
+    const __amdgpu_buffer_rsrc_t rs = field_rsrc((const TF*)src + it.minoff, on ? span : 0u);
+#pragma unroll
+    for (int q = 0; q < kN; q++)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rs, (__attribute__((address_space(3))) void*)(buf + (wv + W * q) * (1024 / SZ)), 16, rel[q], 0, 0, 0);
+  };
+  auto dst = [&](void* base) { return field_rsrc((TF*)base + it.omin, it.dspan * SZ); };
+  // Every lane evaluates (one without a stencil reads its buffer's first values and stores NaN
+  // where valid): with one store site the field index and output pointers stay scalar.
   typedef typename std::conditional<MATH == ADZ_MATH_REF, double, float>::type TC;
-  auto eval = [&](int f, const float* buf) {
-    const int sh = shift(f);
-    const float* b0 = buf + lb[0] + sh;
-    const float* b1 = buf + lb[1] + sh;
-    const float* b2 = buf + lb[2] + sh;
-    const float* b3 = buf + lb[3] + sh;
-    auto at = [&](int r, int z, int c) -> float {
-      const float* bz = z == 0 ? b0 : (z == 1 ? b1 : (z == 2 ? b2 : b3));
+  auto eval = [&](const Ptr& P, const TF* buf) {
+    const TF* b0 = buf + lb[0];
+    const TF* b1 = buf + lb[1];
+    const TF* b2 = buf + lb[2];
+    const TF* b3 = buf + lb[3];
+    auto at = [&](int r, int z, int c) -> TF {
+      const TF* bz = z == 0 ? b0 : (z == 1 ? b1 : (z == 2 ? b2 : b3));
       return bz[r * kPitch5 + c];
     };
     TC v = 0, l = 0, mi = 0, ma = 0;
-    eval_vals<float, MATH, POST>(at, cw, &v, &l, &mi, &ma);
+    if constexpr (MATH == ADZ_MATH_REF) eval_rows<TF, POST>(at, cw, &v, &l, &mi, &ma);
+    else eval_vals<TF, MATH, POST>(at, cw, &v, &l, &mi, &ma);
     if (!ok) {
       const TC nan = (TC)__builtin_nanf("");
       v = nan; l = nan; mi = nan; ma = nan;
     }
-    if (valid) store_out<float, MATH, POST>(F, f, o, v, l, mi, ma);
+    TF vs, ls, mis, mas;
+    narrow_out<TF, MATH, POST>(v, l, mi, ma, &vs, &ls, &mis, &mas);
+    buf_store<TF>(vs, dst(P.d), so);
+    if (POST & ADZ_POST_STORE) {
+      buf_store<TF>(ls, dst(P.l), so);
+      buf_store<TF>(mis, dst(P.n), so);
+      buf_store<TF>(mas, dst(P.x), so);
+    }
   };
-  issue(f0, boxA);
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __syncthreads();
-  for (int f = f0; f < f1; f += 2) {
-    if (f + 1 < f1) issue(f + 1, boxB);
-    eval(f, boxA);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    if (f + 1 >= f1) break;
-    if (f + 2 < f1) issue(f + 2, boxA);
-    eval(f + 1, boxB);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
+  // Field f is evaluated from one buffer while field f + 1 is on its way into the other.  A
+  // wave's vector-memory operations retire in order, and every field adds kN loads and then
+  // kSt stores, so at the wait for field f only the stores of field f - 1 may be outstanding:
+  // no wave waits for its stores.  (The first field has none before it: as many, out of range
+  // and therefore dropped, keep the count.)
+  Ptr P;
+  auto step = [&](int f, const TF* cur, TF* next) {
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(kSt));
+    __syncthreads();  // every wave's part of field f has landed, and nobody reads `next` any more
+    issue(P.s, f + 1 < f1, next);
+    eval(P, cur);
+    source(f + 2, &P);
+    target(f + 1, &P);
+  };
+  source(f0, &P);
+  target(f0, &P);
+  issue(P.s, true, boxA);
+  {
+    const __amdgpu_buffer_rsrc_t none = field_rsrc(P.d, 0u);
+#pragma unroll
+    for (int q = 0; q < kSt; q++) buf_store<TF>((TF)0, none, 0);
   }
+  source(f0 + 1, &P);
+  for (int f = f0;;) {
+    step(f, boxA, boxB);
+    if (++f >= f1) break;
+    step(f, boxB, boxA);
+    if (++f >= f1) break;
+  }
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm(kSt));  // no load into LDS is left behind
 }
 
 // Persistent loop over the tile list of a plan.
@@ -1052,6 +1301,7 @@ __device__ __forceinline__ void plan_loop(const PlanArgs& A, TF* boxA, TF* boxB,
     step = nb;
     t0 = lo + l;
   }
+  unsigned nth = 0;
   for (long t = t0; t < hi; t += step) {
     int q = 0;
     // The item table does not change during a launch: read through the constant address
@@ -1082,14 +1332,14 @@ __device__ __forceinline__ void plan_loop(const PlanArgs& A, TF* boxA, TF* boxB,
     ItemFields F{it.src, it.dst, it.lin, it.mn, it.mx};
     if constexpr (STAGE == 4 && std::is_same<TF, float>::value)
       shared_tile<MATH, POST, TP>(it, F, ptile, f0, f1, A.level_inner);
-    else if constexpr (STAGE == 5 && std::is_same<TF, float>::value)
-      dma_tile<MATH, POST, TP, kTJ, 1>(it, F, ptile, f0, f1, (float*)boxA, (float*)boxB, red, A.level_inner);
-    else if constexpr (STAGE == 6 && std::is_same<TF, float>::value)
-      dma_tile<MATH, POST, TP, kTJ6, 1>(it, F, ptile, f0, f1, (float*)boxA, (float*)boxB, red, A.level_inner);
-    else if constexpr (STAGE == 7 && std::is_same<TF, float>::value)
-      dma_tile<MATH, POST, TP, kTJ, 2>(it, F, ptile, f0, f1, (float*)boxA, (float*)boxB, red, A.level_inner);
-    else if constexpr (STAGE == 8 && std::is_same<TF, float>::value)
-      dma_tile<MATH, POST, TP, kTJ, 4>(it, F, ptile, f0, f1, (float*)boxA, (float*)boxB, red, A.level_inner);
+    else if constexpr (STAGE == 5)
+      dma_tile<TF, MATH, POST, TP, kTJ, 1>(it, F, ptile, f0, f1, boxA, boxB, red, nth++, A.level_inner);
+    else if constexpr (STAGE == 6)
+      dma_tile<TF, MATH, POST, TP, kTJ6, 1>(it, F, ptile, f0, f1, boxA, boxB, red, nth++, A.level_inner);
+    else if constexpr (STAGE == 7)
+      dma_tile<TF, MATH, POST, TP, kTJ, 2>(it, F, ptile, f0, f1, boxA, boxB, red, nth++, A.level_inner);
+    else if constexpr (STAGE == 8)
+      dma_tile<TF, MATH, POST, TP, kTJ, 4>(it, F, ptile, f0, f1, boxA, boxB, red, nth++, A.level_inner);
     else
       run_tile<TF, TP, MATH, POST, ItemFields>(it, F, ptile, f0, f1, boxA, boxB, red, rowoff, STAGE, A.level_inner);
   }
@@ -1116,12 +1366,16 @@ __global__ __launch_bounds__(kTile) void k_plan(PlanArgs A) {
 // blocks its two LDS buffers allow per CU keep four waves on every SIMD; the reference
 // arithmetic needs more registers than that without spilling (and has no 16-wave form).
 template <int TH, int TL> constexpr int dma_stage() { return TL == 4 ? 8 : TL == 2 ? 7 : TH == kTJ ? 5 : 6; }
-template <class TP, int MATH, int POST, int TH, int TL>
-__global__ __launch_bounds__(64 * TH * TL, MATH == ADZ_MATH_F32 ? 4 : 1) void k_plan5(PlanArgs A) {
-  __shared__ float boxA[box_rows<TH * TL>() * kPitch5];
-  __shared__ float boxB[box_rows<TH * TL>() * kPitch5];
-  __shared__ int red[6 * TH * TL];
-  plan_loop<float, TP, MATH, POST, dma_stage<TH, TL>()>(A, boxA, boxB, red, nullptr);
+#define ADZ_BOXES(TF, W)                                                              \
+  __shared__ TF boxA[box_elems<TF, W>()];                                             \
+  __shared__ TF boxB[box_elems<TF, W>()];                                             \
+  __shared__ int red[18];                                                             \
+  if (threadIdx.x < 18) red[threadIdx.x] = kFar;                                      \
+  __syncthreads();
+template <class TF, class TP, int MATH, int POST, int TH, int TL>
+__global__ __launch_bounds__(64 * TH * TL, 4) void k_plan5(PlanArgs A) {
+  ADZ_BOXES(TF, TH * TL)
+  plan_loop<TF, TP, MATH, POST, dma_stage<TH, TL>()>(A, boxA, boxB, red, nullptr);
 }
 
 // One item with inline field pointers (the adz_tricub_hlt entry point).
@@ -1131,27 +1385,25 @@ __global__ __launch_bounds__(kTile) void k_hlt(DevItem it, InlineFields F) {
                                              nullptr, 2, 0);
 }
 
-// The same for FP32 sources with LDS-staged boxes (staging mode 6: tiles of 64 x 8 targets,
-// blocks of eight waves): every field of the call in one pass per tile, tiles in
-// super-columns of kHltOrder tile rows, and block b on tile
-// (b % 8) * per + b / 8, so that each XCD (blocks go round-robin over the 8 XCDs) walks one
-// contiguous eighth of the tile list and its L2 sees neighbouring tiles.  One tile per
-// block: without lin/min/max the kernel needs 72 VGPRs, so seven waves share each SIMD.
-// (The 16-wave form of 64 x 4 x 4 tiles moves fewer bytes, but one such block is resident per
-// CU and its per-field DMA waits are not covered: at c5 with 16 fields and no lin/min/max it
-// gave 150-154 against 200 G point-fields/s.)
-constexpr int kHltOrder = 3;
+// The same with LDS-staged boxes (tiles of 64 x 4 targets x 2 levels, blocks of eight waves):
+// every field of the call in one pass per tile, and block b on tile (b % 8) * per + b / 8, so
+// that each XCD (blocks go round-robin over the 8 XCDs) walks one contiguous eighth of the
+// tile list.  One tile per block: the hardware fills a CU with the next ones as blocks end.
+// Measured against 64 x 8 x 1 tiles with 62 rows per box, where a third of the tiles of a
+// 200 x 150 grid and four fifths of a 512 x 384 one fitted: 3 fields of 200 x 150 x 60 in the
+// reference's arithmetic 63.7 -> 54.8 us; in FP32, 4 fields of 512 x 384 x 84 681 -> 550 us,
+// 8 of 2048 x 1024 x 84 13.4 -> 8.2 ms.  Super-columns of 3 tile rows in place of rows, then
+// levels: 8.2 and 55 against 8.3 and 52 us (3 fields of 200 x 150 x 60, FP32).
+constexpr int kHltOrder = 0;
+constexpr int kHltTH = kTJ, kHltTL = 2;
 
-template <class TP, int MATH, int POST>
-__global__ __launch_bounds__(64 * kTJ6, MATH == ADZ_MATH_F32 ? 4 : 1) void k_hlt5(DevItem it, InlineFields F,
-                                                                                   long ntiles) {
-  __shared__ float boxA[box_rows<kTJ6>() * kPitch5];
-  __shared__ float boxB[box_rows<kTJ6>() * kPitch5];
-  __shared__ int red[6 * kTJ6];
+template <class TF, class TP, int MATH, int POST>
+__global__ __launch_bounds__(64 * kHltTH * kHltTL, 4) void k_hlt5(DevItem it, InlineFields F, long ntiles) {
+  ADZ_BOXES(TF, kHltTH * kHltTL)
   const long per = (ntiles + 7) / 8;
   const long t = (long)(blockIdx.x % 8) * per + blockIdx.x / 8;
   if (t >= ntiles) return;  // the whole block leaves: no barrier is reached
-  dma_tile<MATH, POST, TP, kTJ6, 1>(it, F, t, 0, it.nf, boxA, boxB, red, kHltOrder);
+  dma_tile<TF, MATH, POST, TP, kHltTH, kHltTL>(it, F, t, 0, it.nf, boxA, boxB, red, 0, kHltOrder);
 }
 
 }  // namespace adz
@@ -1192,6 +1444,11 @@ bool fill_item(DevItem* d, const adz_ztab* geom, const void* xyz, int i0, int in
     long bytes = (maxoff - d->minoff + 1) * 4;
     d->span = (bytes > 0 && bytes < 0x7fffffffL) ? (unsigned)bytes : 0u;
   }
+  {
+    d->omin = (long)(i0 - 1) + (long)d->dni * ((long)(j0 - 1) + (long)d->dnj * (k0 - 1));
+    const long n = (long)(d->nx - 1) + (long)d->dni * ((d->ny - 1) + (long)d->dnj * (d->nz - 1)) + 1;
+    d->dspan = n < 0x7fffffffL ? (unsigned)n : 0u;
+  }
   d->npts = (long)d->nx * d->ny * d->nz;
   d->ptiles = (long)((d->nx + kTI - 1) / kTI) * ((d->ny + kTJ - 1) / kTJ) * d->nz;
   return true;
@@ -1211,35 +1468,35 @@ void* pick_plan(int post, int stage) {
     }
     if (stage == 5) {
       switch (post) {
-        case 0: return (void*)&k_plan5<TP, M, 0, kTJ, 1>;
-        case 1: return (void*)&k_plan5<TP, M, 1, kTJ, 1>;
-        case 2: return (void*)&k_plan5<TP, M, 2, kTJ, 1>;
-        default: return (void*)&k_plan5<TP, M, 3, kTJ, 1>;
+        case 0: return (void*)&k_plan5<TF, TP, M, 0, kTJ, 1>;
+        case 1: return (void*)&k_plan5<TF, TP, M, 1, kTJ, 1>;
+        case 2: return (void*)&k_plan5<TF, TP, M, 2, kTJ, 1>;
+        default: return (void*)&k_plan5<TF, TP, M, 3, kTJ, 1>;
       }
     }
     if (stage == 6) {
       switch (post) {
-        case 0: return (void*)&k_plan5<TP, M, 0, kTJ6, 1>;
-        case 1: return (void*)&k_plan5<TP, M, 1, kTJ6, 1>;
-        case 2: return (void*)&k_plan5<TP, M, 2, kTJ6, 1>;
-        default: return (void*)&k_plan5<TP, M, 3, kTJ6, 1>;
+        case 0: return (void*)&k_plan5<TF, TP, M, 0, kTJ6, 1>;
+        case 1: return (void*)&k_plan5<TF, TP, M, 1, kTJ6, 1>;
+        case 2: return (void*)&k_plan5<TF, TP, M, 2, kTJ6, 1>;
+        default: return (void*)&k_plan5<TF, TP, M, 3, kTJ6, 1>;
       }
     }
     if (stage == 7) {
       switch (post) {
-        case 0: return (void*)&k_plan5<TP, M, 0, kTJ, 2>;
-        case 1: return (void*)&k_plan5<TP, M, 1, kTJ, 2>;
-        case 2: return (void*)&k_plan5<TP, M, 2, kTJ, 2>;
-        default: return (void*)&k_plan5<TP, M, 3, kTJ, 2>;
+        case 0: return (void*)&k_plan5<TF, TP, M, 0, kTJ, 2>;
+        case 1: return (void*)&k_plan5<TF, TP, M, 1, kTJ, 2>;
+        case 2: return (void*)&k_plan5<TF, TP, M, 2, kTJ, 2>;
+        default: return (void*)&k_plan5<TF, TP, M, 3, kTJ, 2>;
       }
     }
     if constexpr (M == ADZ_MATH_F32) {
       if (stage == 8) {
         switch (post) {
-          case 0: return (void*)&k_plan5<TP, M, 0, kTJ, 4>;
-          case 1: return (void*)&k_plan5<TP, M, 1, kTJ, 4>;
-          case 2: return (void*)&k_plan5<TP, M, 2, kTJ, 4>;
-          default: return (void*)&k_plan5<TP, M, 3, kTJ, 4>;
+          case 0: return (void*)&k_plan5<TF, TP, M, 0, kTJ, 4>;
+          case 1: return (void*)&k_plan5<TF, TP, M, 1, kTJ, 4>;
+          case 2: return (void*)&k_plan5<TF, TP, M, 2, kTJ, 4>;
+          default: return (void*)&k_plan5<TF, TP, M, 3, kTJ, 4>;
         }
       }
     }
@@ -1268,13 +1525,13 @@ void* pick_plan(int post, int stage) {
   }
 }
 template <class TF, class TP, int M>
-void* pick_hlt(int post) {
+void* pick_hlt(int post, bool staged) {
   if constexpr (std::is_same<TF, float>::value) {
-    switch (post) {
-      case 0: return (void*)&k_hlt5<TP, M, 0>;
-      case 1: return (void*)&k_hlt5<TP, M, 1>;
-      case 2: return (void*)&k_hlt5<TP, M, 2>;
-      default: return (void*)&k_hlt5<TP, M, 3>;
+    if (staged) switch (post) {
+      case 0: return (void*)&k_hlt5<TF, TP, M, 0>;
+      case 1: return (void*)&k_hlt5<TF, TP, M, 1>;
+      case 2: return (void*)&k_hlt5<TF, TP, M, 2>;
+      default: return (void*)&k_hlt5<TF, TP, M, 3>;
     }
   }
   switch (post) {
@@ -1287,7 +1544,7 @@ void* pick_hlt(int post) {
 
 template <bool PLAN>
 void* pick(int fdt, int pdt, int math, int post, int stage = 2) {
-#define P_(TF, TP, M) return PLAN ? pick_plan<TF, TP, M>(post, stage) : pick_hlt<TF, TP, M>(post)
+#define P_(TF, TP, M) return PLAN ? pick_plan<TF, TP, M>(post, stage) : pick_hlt<TF, TP, M>(post, stage != 2)
   if (math == ADZ_MATH_REF) {
     if (fdt == ADZ_F64 && pdt == ADZ_F64) P_(double, double, ADZ_MATH_REF);
     if (fdt == ADZ_F64 && pdt == ADZ_F32) P_(double, float, ADZ_MATH_REF);
@@ -1303,13 +1560,37 @@ void* pick(int fdt, int pdt, int math, int post, int stage = 2) {
   return nullptr;
 }
 
-// Built-in tile parameters, ten fields per pass: for FP32 fields in the FP32 arithmetic,
-// LDS-staged boxes over tiles of 64 x 4 targets x 4 levels (stage 8) with one 16-wave block
-// per CU, the levels of a tile column walked first; otherwise LDS-staged boxes over 64 x 4
-// tiles (stage 5; other field types fall back to per-lane loads) in super-columns of three
-// tile rows.
-adz_tune default_tune(int fdtype, int math) {
-  return fdtype == ADZ_F32 && math == ADZ_MATH_F32 ? adz_tune{10, 0, 1, 1, 8, 1} : adz_tune{10, 0, 4, 1, 5, 3};
+// Built-in tile parameters of FP32 fields, ten fields per pass, LDS-staged boxes:
+//   * FP32 arithmetic with lin/min/max: tiles of 64 x 4 targets x 4 levels (stage 8; the
+//     fewest DMA bytes per target, and the stores leave no room for more).  10 fields of
+//     1024 x 512 x 84 3.61 ms (64 x 4 x 2: 3.8 to 4.5; before 4.15), rows, then levels,
+//     with 8 blocks per CU to even out the ends; where a plane outgrows an XCD's L2 (2048 x
+//     1024: 13.6 ms) super-columns of 3 tile rows with one block per CU (rows, then levels:
+//     15.8 ms; 1024 x 512 in super-columns: 3.9 ms);
+//   * otherwise tiles of 64 x 4 targets x 2 levels (stage 7): two blocks per CU, one
+//     evaluates while the other waits.  16 subdomains x 6 fields in FP32 4.48 ms (stage 8:
+//     5.1; before 6.96), 6 fields of 512 x 384 x 84 in the reference's arithmetic with
+//     lin/min/max 1.33 ms (stage 5: 1.40; before 1.82).
+// Other field types, and items beyond 32-bit offsets: per-lane loads (stage 2).
+adz_tune default_tune(int fdtype, int math, int post, bool staged, long plane_bytes) {
+  if (!staged) return adz_tune{10, 0, 4, 1, 2, 3};
+  if (math != ADZ_MATH_F32) return adz_tune{10, 0, 16, 1, 7, 0};
+  if (!(post & ADZ_POST_STORE)) return adz_tune{10, 0, 32, 1, 7, 3};
+  return plane_bytes <= (4L << 20) ? adz_tune{10, 0, 8, 1, 8, 0} : adz_tune{10, 0, 1, 1, 8, 3};
+}
+adz_tune default_tune(const adz_item* items, int nitems, int fdtype, int math, int post) {
+  bool staged = fdtype == ADZ_F32;
+  long plane = 0;
+  for (int q = 0; q < nitems && items; q++) {
+    const adz_item& a = items[q];
+    DevItem d;
+    if (fill_item(&d, a.geom, a.xyz, a.i0, a.in, a.j0, a.jn, a.k0, a.nk, a.dminx, a.dmaxx, a.dminy, a.dmaxy, a.ext,
+                  a.nptr)) {
+      staged = staged && stageable(d, 4);
+      plane = std::max(plane, (long)d.lv.nij * 4);
+    }
+  }
+  return default_tune(fdtype, math, post, staged, plane);
 }
 // targets per tile along i: kSW for the shared-column staging of FP32 sources, else kTI
 
@@ -1345,8 +1626,8 @@ int adz_tricub_hlt(const adz_field* fld, int nptr, const void* xyz, int pdtype, 
   if (!fld || nptr < 0) return fail(ADZ_EINVAL, "adz_tricub_hlt: bad field list");
   if (nptr == 0 || in < i0 || jn < j0) return ADZ_OK;  // nij <= 0: nothing to do (:61)
   if (post < 0 || post > 3) return fail(ADZ_EINVAL, "adz_tricub_hlt: post must be 0..3");
-  void* kern = pick<false>(fdtype, pdtype, math, post);
-  if (!kern) return fail(ADZ_EINVAL, "adz_tricub_hlt: unsupported (field dtype, position dtype, math)");
+  if (!pick<false>(fdtype, pdtype, math, post))
+    return fail(ADZ_EINVAL, "adz_tricub_hlt: unsupported (field dtype, position dtype, math)");
   for (int f = 0; f < nptr; f++) {
     if (!fld[f].src || !fld[f].dst) return fail(ADZ_EINVAL, "adz_tricub_hlt: null src/dst");
     if ((post & ADZ_POST_STORE) && (!fld[f].lin || !fld[f].mn || !fld[f].mx))
@@ -1365,11 +1646,13 @@ int adz_tricub_hlt(const adz_field* fld, int nptr, const void* xyz, int pdtype, 
       const adz_field& a = fld[f0 + f];
       F.src[f] = a.src; F.dst[f] = a.dst; F.lin[f] = a.lin; F.mn[f] = a.mn; F.mx[f] = a.mx;
     }
-    if (fdtype == ADZ_F32) {  // k_hlt5: LDS-staged boxes, an eighth of the tile list per XCD
-      long ntiles = item_ptiles(it.nx, it.ny, it.nz, kHltOrder, kTI, kTJ6);
+    const bool staged = fdtype == ADZ_F32 && stageable(it, 4);
+    void* kern = pick<false>(fdtype, pdtype, math, post, staged ? 7 : 2);
+    if (staged) {  // k_hlt5: LDS-staged boxes, an eighth of the tile list per XCD
+      long ntiles = item_ptiles(it.nx, it.ny, it.nz, kHltOrder, kTI, kHltTH, kHltTL);
       long grid = 8 * ((ntiles + 7) / 8);  // one block per tile
       void* args[] = {&it, &F, &ntiles};
-      ADZ_HIP_CHECK(hipLaunchKernel(kern, dim3((unsigned)grid), dim3(64 * kTJ6), args, 0, (hipStream_t)stream));
+      ADZ_HIP_CHECK(hipLaunchKernel(kern, dim3((unsigned)grid), dim3(64 * kHltTH * kHltTL), args, 0, (hipStream_t)stream));
     } else {
       void* args[] = {&it, &F};
       ADZ_HIP_CHECK(hipLaunchKernel(kern, dim3((unsigned)it.ptiles), dim3(kTile), args, 0, (hipStream_t)stream));
@@ -1391,7 +1674,7 @@ int adz_plan_create(const adz_item* items, int nitems, int fdtype, int math, int
     return fail(ADZ_EINVAL, "adz_plan_create: stage 8 needs the FP32 arithmetic");
   if (tune && (tune->xcd_chunks < 0 || tune->xcd_chunks > 1))
     return fail(ADZ_EINVAL, "adz_plan_create: xcd_chunks must be 0 or 1");
-  adz_tune T = default_tune(fdtype, math);
+  adz_tune T = default_tune(items, nitems, fdtype, math, post);
   if (tune) {
     if (tune->fields_per_pass > 0) T.fields_per_pass = std::min(64, tune->fields_per_pass);
     T.points_outer = tune->points_outer;
@@ -1530,12 +1813,12 @@ int adz_plan_autotune(const adz_item* items, int nitems, int fdtype, int math, i
     int rf = adz_plan_free(p);
     return rc != ADZ_OK ? rc : rf;
   };
-  adz_tune cur = default_tune(fdtype, math);
+  adz_tune cur = default_tune(items, nitems, fdtype, math, post);
   cur.fields_per_pass = std::min(cur.fields_per_pass, maxf);
   float cur_ms = 0.f;
   int rc = time_one(cur, &cur_ms);
   const int stages[] = {1, 2, 3, 4, 5, 6, 7, 8}, fpps[] = {2, 3, 4, 5, 8, 10, 16, 20, 32, 40, 64},
-            bpcs[] = {1, 2, 4, 8, 16}, flags[] = {0, 1}, orders[] = {0, 1, 2, 3, 4, 6, 8};
+            bpcs[] = {1, 2, 4, 8, 16, 32}, flags[] = {0, 1}, orders[] = {0, 1, 2, 3, 4, 6, 8};
   const int nst = fdtype != ADZ_F32 ? 2 : math == ADZ_MATH_F32 ? 8 : 7, nor = 7;
   // staging and tile order together first: the LDS-staged forms depend on the L2 reuse the
   // tile order gives, so one is not searched at the other's best value.  Each staging is
@@ -1557,7 +1840,7 @@ int adz_plan_autotune(const adz_item* items, int nitems, int fdtype, int math, i
   for (int ci = 0; ci < 5 && rc == ADZ_OK; ci++) {
     const int coord = coords[ci];
     const int* vals = coord == 1 ? orders : coord == 2 ? fpps : coord == 3 ? bpcs : flags;
-    int nv = coord == 1 ? nor : coord == 2 ? 11 : coord == 3 ? 5 : 2;
+    int nv = coord == 1 ? nor : coord == 2 ? 11 : coord == 3 ? 6 : 2;
     for (int v = 0; v < nv && rc == ADZ_OK; v++) {
       adz_tune t = cur;
       int* slot = coord == 1 ? &t.level_inner : coord == 2 ? &t.fields_per_pass

@@ -69,20 +69,22 @@ __device__ __forceinline__ void mono_extra_a(Acc at, const TC* c, TC* lin, TC* m
     *mi = lo;
     *ma = hi;
   } else {
-    TC vmi[4], vma[4];
+    // FP32 values compare in FP32 as they do widened: the same selection, at half the registers
+    typedef typename std::conditional<std::is_same<TF, float>::value, float, TC>::type TM;
+    TM vmi[4], vma[4];
 #pragma unroll
     for (int r = 0; r < 4; r++) {
 #pragma unroll
       for (int i = 1; i < 3; i++) {
-        TC a = (TC)to_f64<TF>(at(r, 1, i)), b = (TC)to_f64<TF>(at(r, 2, i));
+        TM a = (TM)to_f64<TF>(at(r, 1, i)), b = (TM)to_f64<TF>(at(r, 2, i));
         if (r == 0) { vmi[i] = a; vma[i] = a; }
         else { vmi[i] = (vmi[i] < a) ? vmi[i] : a; vma[i] = (vma[i] > a) ? vma[i] : a; }
         vmi[i] = (vmi[i] < b) ? vmi[i] : b;
         vma[i] = (vma[i] > b) ? vma[i] : b;
       }
     }
-    *mi = (vmi[1] < vmi[2]) ? vmi[1] : vmi[2];
-    *ma = (vma[1] > vma[2]) ? vma[1] : vma[2];
+    *mi = (TC)((vmi[1] < vmi[2]) ? vmi[1] : vmi[2]);
+    *ma = (TC)((vma[1] > vma[2]) ? vma[1] : vma[2]);
   }
   TC vyl[4];
 #pragma unroll

@@ -227,9 +227,10 @@ typedef struct adz_item {
 } adz_item;
 
 /* Tile parameters of the persistent kernel; zero fields_per_pass / blocks_per_cu take the
-   built-in default, {10, 0, 1, 1, 8, 1} for FP32 fields in the FP32 arithmetic and
-   {10, 0, 4, 1, 5, 3} otherwise, and stage 0 takes the built-in staging together with its
-   level_inner; adz_plan_autotune searches them on the actual plan. */
+   built-in default: ten fields per pass, and for FP32 fields stage 8 in the FP32 arithmetic
+   with lin/min/max, stage 7 otherwise (other field types, and arrays beyond 32-bit byte
+   offsets: stage 2).  Stage 0 takes the built-in staging together with its level_inner;
+   adz_plan_autotune searches them on the actual plan. */
 typedef struct adz_tune {
   int fields_per_pass; /* fields interpolated per pass over the points (1..64)          */
   int points_outer;    /* 1: a block runs every field group of a point tile; 0: a pass
@@ -249,7 +250,7 @@ typedef struct adz_tune {
                           (FP32 sources): tiles of 64 x 4 targets over 2 and 4
                           consecutive levels, blocks of 8 and 16 waves (8: the FP32
                           arithmetic only, ADZ_EINVAL otherwise; one block per CU is
-                          resident; the fastest form at c5)                             */
+                          resident)                                                     */
   int level_inner;     /* tile order. 0: i, j, then k; 1: consecutive tiles walk the
                           levels of one tile column; S >= 2: super-columns of S tile
                           rows walked level by level (source planes and rows reused
