@@ -48,8 +48,9 @@ struct DevItem {
 };
 
 // Can boxes of elements of `size` bytes be staged, and their outputs stored, at 32-bit byte
-// offsets?
+// offsets?  (2-byte elements: every row must begin at the same half of a 4-byte word.)
 __host__ __device__ inline bool stageable(const DevItem& it, int size) {
+  if (size == 2 && ((it.lv.ni | it.lv.nij) & 1)) return false;
   return it.span && it.dspan && (long)(it.span / 4) * size < 0x7fffffffL && (long)it.dspan * size < 0x7fffffffL;
 }
 
@@ -174,6 +175,15 @@ struct RegStencil {
   __device__ __forceinline__ float operator()(int r, int z, int i) const { return v[r][z][i]; }
 };
 
+// Four 2-byte values of a stencil row as one 8-byte load.
+typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
+struct HalfStencil {
+  const u32x2 (*v)[4];
+  __device__ __forceinline__ bf16 operator()(int r, int z, int i) const {
+    return __builtin_bit_cast(bf16, (uint16_t)(v[r][z][i >> 1] >> (16 * (i & 1))));
+  }
+};
+
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t field_rsrc(const void* base, unsigned bytes) {
   // the field pointer is uniform across the wave: keep the descriptor in SGPRs
   unsigned long long a = (unsigned long long)base;
@@ -266,6 +276,25 @@ __device__ __forceinline__ void per_lane(const DevItem& it, const Fields& F, int
       }
       return;
     }
+  }
+  if constexpr (sizeof(TF) == 2) {
+    const long o1 = x.zlinear ? 0 : gnij, o2 = o1 + gnij, o3 = o2 + o1;
+    for (int f = f0; f < f1; f++) {
+      if (ok) {
+        typedef ADZ_GLOBAL u32x2 __attribute__((aligned(2))) Quad;
+        const ADZ_GLOBAL char* s = (const ADZ_GLOBAL char*)F.s(f) + 2 * x.off;
+        u32x2 v[4][4];
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+          for (int z = 0; z < 4; z++)
+            v[r][z] = *(const Quad*)(s + 2 * (r * gni + (z == 0 ? 0 : (z == 1 ? o1 : (z == 2 ? o2 : o3)))));
+        eval_store_a<TF, MATH, POST>(F, f, HalfStencil{v}, cw, o);
+      } else if (valid) {
+        store_nan<TF, MATH, POST>(F, f, o);
+      }
+    }
+    return;
   }
   for (int f = f0; f < f1; f++) {
     if (ok)
@@ -971,7 +1000,7 @@ __device__ __forceinline__ void shared_tile(const DevItem& it, const Fields& F, 
 }
 
 // ---------------------------------------------------------------------------------
-// Staging mode 5 (FP32 sources): the tile's box (the union of its 256 stencils) is copied
+// Staging mode 5: the tile's box (the union of its 256 stencils) is copied
 // into LDS once per field by all four waves with 16-byte buffer-to-LDS DMA, and every lane
 // then reads its 64 stencil values from LDS.  Per-lane loads spend 16 address slots of the
 // texture unit per point-field; the box needs about 2 (a 68 x 7 x 4 box is 28 rows of 18
@@ -988,29 +1017,36 @@ __device__ __forceinline__ void shared_tile(const DevItem& it, const Fields& F, 
 //   * Field f + 1 is in flight while field f is evaluated from the other of two buffers, one
 //     block barrier per field, and no wave waits for its own stores (dma_tile).
 //   * A field's pointers are loaded a step ahead, outside the LDS reads.
-// Tiles whose box does not fit (more than box_rows rows or 96 columns) or reaches the end of
+// Tiles whose box does not fit (more than box_rows rows or box_pitch columns) or reaches the end of
 // 32-bit buffer offsets use per-lane loads, in the same arithmetic and order: the same bits.
 // Staging mode 6 has tiles of 64 x 8 targets and blocks of eight waves, modes 7 and 8 tiles
 // of 64 x 4 targets over 2 and 4 consecutive levels (blocks of 8 and 16 waves, one wave per
 // target row and level).  A source plane is read by the stencils of about four levels, so the
 // planes of a box dominate its volume: DMA bytes per target and field on 512 x 384 x 84 are
 // 39.7 for 64 x 4 x 1, 29.9 for 64 x 8 x 1, 24.5 for 64 x 4 x 2 and 16.9 for 64 x 4 x 4.
-// What bounds it: 6 fields, no lin/min/max (stage 7): LDS reads (256 B per point-field, 58 %
+//   * FP64 fields: rows of 80 elements (five times round the banks), 62 per buffer, so that
+//     two blocks of eight waves fit a CU.  BF16 fields: rows of 128 elements; the quads begin
+//     at the word that holds the box's first column, a lane reads the three words that hold
+//     its four columns and shifts them (reading 2-byte values took 190 us where this takes
+//     72, and per-lane loads 115).
+// What bounds it: 6 FP32 fields, no lin/min/max (stage 7): LDS reads (256 B per point-field, 58 %
 // of the cycles, a quarter of those still bank conflicts), FP32 arithmetic (100 instructions
 // per field and 40 per field for the tile's indexes, weights and box: 54 %) and the texture
 // unit's DMA (41 %), none hidden completely behind another with 16 waves per CU.
-constexpr int kPitch5 = 96;                // elements per LDS row
+
+// elements per LDS row: whole rounds of the 32 banks
+template <class TF> constexpr int box_pitch() { return sizeof(TF) == 8 ? 80 : sizeof(TF) == 4 ? 96 : 128; }
 constexpr int kTJ6 = 8;                    // target rows of a staging-mode-6 tile
-template <class TF> constexpr int quads_per_row() { return kPitch5 * (int)sizeof(TF) / 16; }
+template <class TF> constexpr int quads_per_row() { return box_pitch<TF>() * (int)sizeof(TF) / 16; }
 // rows per LDS buffer for blocks of W waves
-template <int W> constexpr int box_rows() { return W >= 8 ? 85 : 64; }
-// DMA instructions per wave and field: all are issued for every field (lanes without a quad
-// ask for one out of range and get zeros), so that a wave can count what is outstanding
-template <class TF, int W> constexpr int dma_per_wave() {
-  return (box_rows<W>() * quads_per_row<TF>() + 64 * W - 1) / (64 * W);
-}
-template <class TF, int W> constexpr int box_elems() { return dma_per_wave<TF, W>() * W * 1024 / (int)sizeof(TF); }
-static_assert(box_rows<4>() < 128 && box_rows<16>() < 128, "row split by a float reciprocal below");
+// (8-byte elements: 62 rows, so that two blocks of two buffers fit a CU's 160 KB)
+template <class TF, int W> constexpr int box_rows() { return sizeof(TF) == 8 ? 62 : W >= 8 ? 85 : 64; }
+// DMA instructions (1 KB each) that fill a buffer, dealt out to the waves in turn.  Lanes
+// without a quad ask for one out of range and get zeros.
+template <class TF, int W> constexpr int box_dma() { return (box_rows<TF, W>() * quads_per_row<TF>() + 63) / 64; }
+template <class TF, int W> constexpr int dma_per_wave() { return (box_dma<TF, W>() + W - 1) / W; }
+template <class TF, int W> constexpr int box_elems() { return box_dma<TF, W>() * 1024 / (int)sizeof(TF); }
+static_assert(box_rows<float, 8>() < 128 && box_rows<double, 8>() < 128, "row split by a float reciprocal below");
 
 // s_waitcnt immediate (gfx9): at most n vector-memory operations outstanding, the other
 // counters not waited for
@@ -1019,7 +1055,6 @@ constexpr int vmcnt_imm(int n) { return (n & 15) | (7 << 4) | (15 << 8) | ((n >>
 template <class TF>
 __device__ __forceinline__ void buf_store(TF v, __amdgpu_buffer_rsrc_t rs, int off) {
   if constexpr (sizeof(TF) == 8) {
-    typedef unsigned u32x2 __attribute__((ext_vector_type(2)));
     __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), rs, off, 0, 0);
   } else if constexpr (sizeof(TF) == 4) {
     __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), rs, off, 0, 0);
@@ -1132,8 +1167,8 @@ template <class TF, int MATH, int POST, class TP, int TH, int TL, class Fields>
 __device__ __forceinline__ void dma_tile(const DevItem& it, const Fields& F, long ptile, int f0, int f1, TF* boxA,
                                          TF* boxB, int* red, unsigned nth, int level_inner) {
   constexpr int W = TH * TL;                  // waves of the block: one per target row and level
-  constexpr int kRows = box_rows<W>(), kN = dma_per_wave<TF, W>();
-  constexpr int kQ = quads_per_row<TF>(), kE = 16 / (int)sizeof(TF), SZ = (int)sizeof(TF);
+  constexpr int kRows = box_rows<TF, W>(), kN = dma_per_wave<TF, W>();
+  constexpr int kPitch = box_pitch<TF>(), kQ = quads_per_row<TF>(), kE = 16 / (int)sizeof(TF), SZ = (int)sizeof(TF);
   constexpr int kSt = POST & ADZ_POST_STORE ? 4 : 1;  // stores per field
   const int lane = threadIdx.x & (kTI - 1), wv = threadIdx.x / kTI;
   const TileXY tc = tile_at(it, ptile, level_inner, kTI, TH, TL);
@@ -1163,7 +1198,8 @@ __device__ __forceinline__ void dma_tile(const DevItem& it, const Fields& F, lon
     return;
   }
   const int nxb = -ext[1] - x0 + 1, nyb = -ext[3] - y0 + 1, nzb = -ext[5] - z0 + 1;
-  const int nrows = nyb * nzb, cpr = (nxb + kE - 1) / kE;  // quads per row
+  // quads per row (2-byte elements: room for a row that begins in the middle of a word)
+  const int nrows = nyb * nzb, cpr = (nxb + (SZ == 2) + kE - 1) / kE;
   const long gni = it.lv.ni, gnij = it.lv.nij;
   // every quad the DMA reads inside the buffer's range [minoff, minoff + span): a quad
   // reaching outside would read zeros for its in-range elements too
@@ -1181,7 +1217,7 @@ __device__ __forceinline__ void dma_tile(const DevItem& it, const Fields& F, lon
   // (32-bit arithmetic: every offset is below 2^31; R / nyb by a float reciprocal, exact
   // since R < 128 and nyb < 128 keep (R + 0.5) / nyb >= 1/256 from an integer, far above the
   // float product's error)
-  const int rel0 = (int)__builtin_amdgcn_readfirstlane((int)first);
+  const int rel0 = (int)__builtin_amdgcn_readfirstlane((int)first) & (SZ == 2 ? ~1 : ~0);
   const int ni32 = (int)gni, nij32 = (int)gnij;
   const float rnyb = 1.0f / (float)nyb;
   int rel[kN];
@@ -1199,7 +1235,7 @@ __device__ __forceinline__ void dma_tile(const DevItem& it, const Fields& F, lon
 #pragma unroll
     for (int z = 0; z < 4; z++) {
       const int dz = x.zlinear ? (z >> 1) : z;
-      lb[z] = (r0 + nyb * (pz0 + dz)) * kPitch5 + c0;
+      lb[z] = (r0 + nyb * (pz0 + dz)) * kPitch + c0;
     }
   }
   const int so = valid ? (int)od * SZ : (int)it.dspan * SZ;  // invalid lanes store out of range (dropped)
@@ -1221,29 +1257,54 @@ __device__ __forceinline__ void dma_tile(const DevItem& it, const Fields& F, lon
       asm volatile("" : "+s"(q->l), "+s"(q->n), "+s"(q->x));
     }
   };
+  // 2-byte elements: the quads begin at the 4-byte word that holds the box's first column, one
+  // element early (half_of = 1) where that is the word's second half; with `first` odd, rel0
+  // is one element early already.
+  auto half_of = [&](const void* src) -> int {
+    if constexpr (SZ != 2) return 0;
+    return (int)((((unsigned long long)src >> 1) + (unsigned long long)(it.minoff + first)) & 1);
+  };
+  const int wu = box_dma<TF, W>() % W ? (int)__builtin_amdgcn_readfirstlane(wv) : 0;
   auto issue = [&](const void* src, bool on, TF* buf) {
-    const __amdgpu_buffer_rsrc_t rs = field_rsrc((const TF*)src + it.minoff, on ? span : 0u);
+    const int d = SZ == 2 ? ((int)first & 1) - half_of(src) : 0;  // elements from rel0's to the quads' begin
+    const __amdgpu_buffer_rsrc_t rs = field_rsrc((const TF*)src + it.minoff + d, on ? span - SZ * d : 0u);
 #pragma unroll
     for (int q = 0; q < kN; q++)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(
+      if (box_dma<TF, W>() % W == 0 || wu + W * q < box_dma<TF, W>()) __builtin_amdgcn_raw_ptr_buffer_load_lds(
           rs, (__attribute__((address_space(3))) void*)(buf + (wv + W * q) * (1024 / SZ)), 16, rel[q], 0, 0, 0);
   };
   auto dst = [&](void* base) { return field_rsrc((TF*)base + it.omin, it.dspan * SZ); };
   // Every lane evaluates (one without a stencil reads its buffer's first values and stores NaN
   // where valid): with one store site the field index and output pointers stay scalar.
   typedef typename std::conditional<MATH == ADZ_MATH_REF, double, float>::type TC;
-  auto eval = [&](const Ptr& P, const TF* buf) {
-    const TF* b0 = buf + lb[0];
-    const TF* b1 = buf + lb[1];
-    const TF* b2 = buf + lb[2];
-    const TF* b3 = buf + lb[3];
-    auto at = [&](int r, int z, int c) -> TF {
-      const TF* bz = z == 0 ? b0 : (z == 1 ? b1 : (z == 2 ? b2 : b3));
-      return bz[r * kPitch5 + c];
-    };
+  auto eval = [&](const Ptr& P, int half, const TF* buf) {
     TC v = 0, l = 0, mi = 0, ma = 0;
-    if constexpr (MATH == ADZ_MATH_REF) eval_rows<TF, POST>(at, cw, &v, &l, &mi, &ma);
-    else eval_vals<TF, MATH, POST>(at, cw, &v, &l, &mi, &ma);
+    if constexpr (SZ == 2) {
+      // a stencil row from the three words that hold it
+      u32x2 q[4][4];
+      const unsigned sh = 16 * ((lb[0] + half) & 1);
+#pragma unroll
+      for (int z = 0; z < 4; z++) {
+        const unsigned* b = (const unsigned*)buf + ((lb[z] + half) >> 1);
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+          const unsigned w0 = b[r * (kPitch / 2)], w1 = b[r * (kPitch / 2) + 1], w2 = b[r * (kPitch / 2) + 2];
+          q[r][z] = u32x2{__builtin_amdgcn_alignbit(w1, w0, sh), __builtin_amdgcn_alignbit(w2, w1, sh)};
+        }
+      }
+      eval_vals<TF, MATH, POST>(HalfStencil{q}, cw, &v, &l, &mi, &ma);
+    } else {
+      const TF* b0 = buf + lb[0];
+      const TF* b1 = buf + lb[1];
+      const TF* b2 = buf + lb[2];
+      const TF* b3 = buf + lb[3];
+      auto at = [&](int r, int z, int c) -> TF {
+        const TF* bz = z == 0 ? b0 : (z == 1 ? b1 : (z == 2 ? b2 : b3));
+        return bz[r * kPitch + c];
+      };
+      if constexpr (MATH == ADZ_MATH_REF) eval_rows<TF, POST>(at, cw, &v, &l, &mi, &ma);
+      else eval_vals<TF, MATH, POST>(at, cw, &v, &l, &mi, &ma);
+    }
     if (!ok) {
       const TC nan = (TC)__builtin_nanf("");
       v = nan; l = nan; mi = nan; ma = nan;
@@ -1258,7 +1319,7 @@ __device__ __forceinline__ void dma_tile(const DevItem& it, const Fields& F, lon
     }
   };
   // Field f is evaluated from one buffer while field f + 1 is on its way into the other.  A
-  // wave's vector-memory operations retire in order, and every field adds kN loads and then
+  // wave's vector-memory operations retire in order, and every field adds its loads and then
   // kSt stores, so at the wait for field f only the stores of field f - 1 may be outstanding:
   // no wave waits for its stores.  (The first field has none before it: as many, out of range
   // and therefore dropped, keep the count.)
@@ -1266,8 +1327,9 @@ __device__ __forceinline__ void dma_tile(const DevItem& it, const Fields& F, lon
   auto step = [&](int f, const TF* cur, TF* next) {
     __builtin_amdgcn_s_waitcnt(vmcnt_imm(kSt));
     __syncthreads();  // every wave's part of field f has landed, and nobody reads `next` any more
+    const int half = half_of(SZ == 2 ? F.s(f) : nullptr);
     issue(P.s, f + 1 < f1, next);
-    eval(P, cur);
+    eval(P, half, cur);
     source(f + 2, &P);
     target(f + 1, &P);
   };
@@ -1361,14 +1423,14 @@ __global__ __launch_bounds__(kTile) void k_plan(PlanArgs A) {
   }
 }
 
-// Staging modes 5 to 8 (FP32 sources, tiles of TH target rows x TL levels, one wave per row
+// Staging modes 5 to 8 (tiles of TH target rows x TL levels, one wave per row
 // and level): their own kernel.  In the FP32 arithmetic it is held to 128 VGPRs, so that the
 // blocks its two LDS buffers allow per CU keep four waves on every SIMD; the reference
 // arithmetic needs more registers than that without spilling (and has no 16-wave form).
 template <int TH, int TL> constexpr int dma_stage() { return TL == 4 ? 8 : TL == 2 ? 7 : TH == kTJ ? 5 : 6; }
 #define ADZ_BOXES(TF, W)                                                              \
-  __shared__ TF boxA[box_elems<TF, W>()];                                             \
-  __shared__ TF boxB[box_elems<TF, W>()];                                             \
+  __shared__ __attribute__((aligned(16))) TF boxA[box_elems<TF, W>()];                                             \
+  __shared__ __attribute__((aligned(16))) TF boxB[box_elems<TF, W>() + 2];                                           \
   __shared__ int red[18];                                                             \
   if (threadIdx.x < 18) red[threadIdx.x] = kFar;                                      \
   __syncthreads();
@@ -1466,40 +1528,42 @@ void* pick_plan(int post, int stage) {
         default: return (void*)&k_plan<TF, TP, M, 3, 4>;
       }
     }
-    if (stage == 5) {
+  }
+  if (stage == 5) {
+    switch (post) {
+      case 0: return (void*)&k_plan5<TF, TP, M, 0, kTJ, 1>;
+      case 1: return (void*)&k_plan5<TF, TP, M, 1, kTJ, 1>;
+      case 2: return (void*)&k_plan5<TF, TP, M, 2, kTJ, 1>;
+      default: return (void*)&k_plan5<TF, TP, M, 3, kTJ, 1>;
+    }
+  }
+  if (stage == 6) {
+    switch (post) {
+      case 0: return (void*)&k_plan5<TF, TP, M, 0, kTJ6, 1>;
+      case 1: return (void*)&k_plan5<TF, TP, M, 1, kTJ6, 1>;
+      case 2: return (void*)&k_plan5<TF, TP, M, 2, kTJ6, 1>;
+      default: return (void*)&k_plan5<TF, TP, M, 3, kTJ6, 1>;
+    }
+  }
+  if (stage == 7) {
+    switch (post) {
+      case 0: return (void*)&k_plan5<TF, TP, M, 0, kTJ, 2>;
+      case 1: return (void*)&k_plan5<TF, TP, M, 1, kTJ, 2>;
+      case 2: return (void*)&k_plan5<TF, TP, M, 2, kTJ, 2>;
+      default: return (void*)&k_plan5<TF, TP, M, 3, kTJ, 2>;
+    }
+  }
+  if constexpr (M == ADZ_MATH_F32) {
+    if (stage == 8) {
       switch (post) {
-        case 0: return (void*)&k_plan5<TF, TP, M, 0, kTJ, 1>;
-        case 1: return (void*)&k_plan5<TF, TP, M, 1, kTJ, 1>;
-        case 2: return (void*)&k_plan5<TF, TP, M, 2, kTJ, 1>;
-        default: return (void*)&k_plan5<TF, TP, M, 3, kTJ, 1>;
+        case 0: return (void*)&k_plan5<TF, TP, M, 0, kTJ, 4>;
+        case 1: return (void*)&k_plan5<TF, TP, M, 1, kTJ, 4>;
+        case 2: return (void*)&k_plan5<TF, TP, M, 2, kTJ, 4>;
+        default: return (void*)&k_plan5<TF, TP, M, 3, kTJ, 4>;
       }
     }
-    if (stage == 6) {
-      switch (post) {
-        case 0: return (void*)&k_plan5<TF, TP, M, 0, kTJ6, 1>;
-        case 1: return (void*)&k_plan5<TF, TP, M, 1, kTJ6, 1>;
-        case 2: return (void*)&k_plan5<TF, TP, M, 2, kTJ6, 1>;
-        default: return (void*)&k_plan5<TF, TP, M, 3, kTJ6, 1>;
-      }
-    }
-    if (stage == 7) {
-      switch (post) {
-        case 0: return (void*)&k_plan5<TF, TP, M, 0, kTJ, 2>;
-        case 1: return (void*)&k_plan5<TF, TP, M, 1, kTJ, 2>;
-        case 2: return (void*)&k_plan5<TF, TP, M, 2, kTJ, 2>;
-        default: return (void*)&k_plan5<TF, TP, M, 3, kTJ, 2>;
-      }
-    }
-    if constexpr (M == ADZ_MATH_F32) {
-      if (stage == 8) {
-        switch (post) {
-          case 0: return (void*)&k_plan5<TF, TP, M, 0, kTJ, 4>;
-          case 1: return (void*)&k_plan5<TF, TP, M, 1, kTJ, 4>;
-          case 2: return (void*)&k_plan5<TF, TP, M, 2, kTJ, 4>;
-          default: return (void*)&k_plan5<TF, TP, M, 3, kTJ, 4>;
-        }
-      }
-    }
+  }
+  if constexpr (std::is_same<TF, float>::value) {
     if (stage == 3) {
       switch (post) {
         case 0: return (void*)&k_plan_pc<TP, M, 0>;
@@ -1526,8 +1590,8 @@ void* pick_plan(int post, int stage) {
 }
 template <class TF, class TP, int M>
 void* pick_hlt(int post, bool staged) {
-  if constexpr (std::is_same<TF, float>::value) {
-    if (staged) switch (post) {
+  if (staged) {
+    switch (post) {
       case 0: return (void*)&k_hlt5<TF, TP, M, 0>;
       case 1: return (void*)&k_hlt5<TF, TP, M, 1>;
       case 2: return (void*)&k_hlt5<TF, TP, M, 2>;
@@ -1560,48 +1624,62 @@ void* pick(int fdt, int pdt, int math, int post, int stage = 2) {
   return nullptr;
 }
 
-// Built-in tile parameters of FP32 fields, ten fields per pass, LDS-staged boxes:
-//   * FP32 arithmetic with lin/min/max: tiles of 64 x 4 targets x 4 levels (stage 8; the
+int field_bytes(int fdtype) { return fdtype == ADZ_F64 ? 8 : fdtype == ADZ_F32 ? 4 : 2; }
+
+// Built-in tile parameters, ten fields per pass, LDS-staged boxes:
+//   * FP32 fields in FP32 arithmetic with lin/min/max: tiles of 64 x 4 targets x 4 levels (stage 8; the
 //     fewest DMA bytes per target, and the stores leave no room for more).  10 fields of
 //     1024 x 512 x 84 3.61 ms (64 x 4 x 2: 3.8 to 4.5; before 4.15), rows, then levels,
 //     with 8 blocks per CU to even out the ends; where a plane outgrows an XCD's L2 (2048 x
 //     1024: 13.6 ms) super-columns of 3 tile rows with one block per CU (rows, then levels:
 //     15.8 ms; 1024 x 512 in super-columns: 3.9 ms);
-//   * otherwise tiles of 64 x 4 targets x 2 levels (stage 7): two blocks per CU, one
+//   * FP32 fields otherwise, tiles of 64 x 4 targets x 2 levels (stage 7): two blocks per CU, one
 //     evaluates while the other waits.  16 subdomains x 6 fields in FP32 4.48 ms (stage 8:
 //     5.1; before 6.96), 6 fields of 512 x 384 x 84 in the reference's arithmetic with
 //     lin/min/max 1.33 ms (stage 5: 1.40; before 1.82).
-// Other field types, and items beyond 32-bit offsets: per-lane loads (stage 2).
+//   * FP64 fields: the same tiles in super-columns of two tile rows, since only two such
+//     blocks fit a CU's LDS.  4 fields of 511 x 385 x 84 0.75 ms (stage 5: 1.02; per-lane
+//     loads 1.30), with clipping 1.16 (1.42; 2.21);
+//   * BF16 fields: tiles of 64 x 4 targets (stage 5), whose boxes are small in bytes, with
+//     four blocks per CU.  4 clipped fields of 200 x 150 x 60 72 us (stage 7: 77; per-lane
+//     loads 115), of 600 x 400 x 60 0.62 ms (0.65; 1.09).
+// Items beyond 32-bit offsets, and BF16 ones with rows or planes of odd length: per-lane
+// loads (stage 2).
 adz_tune default_tune(int fdtype, int math, int post, bool staged, long plane_bytes) {
   if (!staged) return adz_tune{10, 0, 4, 1, 2, 3};
+  if (fdtype == ADZ_F64) return adz_tune{10, 0, 32, 1, 7, 2};
+  if (fdtype == ADZ_BF16) return adz_tune{10, 0, 16, 1, 5, 0};
   if (math != ADZ_MATH_F32) return adz_tune{10, 0, 16, 1, 7, 0};
   if (!(post & ADZ_POST_STORE)) return adz_tune{10, 0, 32, 1, 7, 3};
   return plane_bytes <= (4L << 20) ? adz_tune{10, 0, 8, 1, 8, 0} : adz_tune{10, 0, 1, 1, 8, 3};
 }
 adz_tune default_tune(const adz_item* items, int nitems, int fdtype, int math, int post) {
-  bool staged = fdtype == ADZ_F32;
+  bool staged = true;
   long plane = 0;
   for (int q = 0; q < nitems && items; q++) {
     const adz_item& a = items[q];
     DevItem d;
     if (fill_item(&d, a.geom, a.xyz, a.i0, a.in, a.j0, a.jn, a.k0, a.nk, a.dminx, a.dmaxx, a.dminy, a.dmaxy, a.ext,
                   a.nptr)) {
-      staged = staged && stageable(d, 4);
-      plane = std::max(plane, (long)d.lv.nij * 4);
+      staged = staged && stageable(d, field_bytes(fdtype));
+      plane = std::max(plane, (long)d.lv.nij * field_bytes(fdtype));
     }
   }
   return default_tune(fdtype, math, post, staged, plane);
 }
 // targets per tile along i: kSW for the shared-column staging of FP32 sources, else kTI
 
-int tile_width(int stage, int fdtype) { return (stage == 4 && fdtype == ADZ_F32) ? kSW : kTI; }
-int tile_height(int stage, int fdtype) { return (stage == 6 && fdtype == ADZ_F32) ? kTJ6 : kTJ; }
-int tile_levels(int stage, int fdtype) {
-  return fdtype != ADZ_F32 ? 1 : stage == 7 ? 2 : stage == 8 ? 4 : 1;
+// the staging a plan of this field type runs: modes that only FP32 sources have (3, 4), and
+// the 16-wave blocks in the reference's arithmetic, stand for per-lane loads
+int run_stage(int stage, int fdtype) {
+  if (fdtype == ADZ_F32) return stage;
+  return stage == 3 || stage == 4 || (stage == 8 && fdtype == ADZ_F64) ? 2 : stage;
 }
+int tile_width(int stage) { return stage == 4 ? kSW : kTI; }
+int tile_height(int stage) { return stage == 6 ? kTJ6 : kTJ; }
+int tile_levels(int stage) { return stage == 7 ? 2 : stage == 8 ? 4 : 1; }
 // threads per block of a plan's kernel
-unsigned plan_threads(int stage, int fdtype) {
-  if (fdtype != ADZ_F32) return kTile;
+unsigned plan_threads(int stage) {
   return stage == 3 ? kPCThreads : stage == 6 || stage == 7 ? 512 : stage == 8 ? 1024 : kTile;
 }
 
@@ -1646,7 +1724,7 @@ int adz_tricub_hlt(const adz_field* fld, int nptr, const void* xyz, int pdtype, 
       const adz_field& a = fld[f0 + f];
       F.src[f] = a.src; F.dst[f] = a.dst; F.lin[f] = a.lin; F.mn[f] = a.mn; F.mx[f] = a.mx;
     }
-    const bool staged = fdtype == ADZ_F32 && stageable(it, 4);
+    const bool staged = stageable(it, field_bytes(fdtype));
     void* kern = pick<false>(fdtype, pdtype, math, post, staged ? 7 : 2);
     if (staged) {  // k_hlt5: LDS-staged boxes, an eighth of the tile list per XCD
       long ntiles = item_ptiles(it.nx, it.ny, it.nz, kHltOrder, kTI, kHltTH, kHltTL);
@@ -1707,8 +1785,9 @@ int adz_plan_create(const adz_item* items, int nitems, int fdtype, int math, int
       ptrs[4 * nptr_total + pofs + f] = a.fld[f].mx;
     }
     dv[q].ngroups = (a.nptr + T.fields_per_pass - 1) / T.fields_per_pass;
-    dv[q].ptiles = item_ptiles(dv[q].nx, dv[q].ny, dv[q].nz, T.level_inner, tile_width(T.stage, fdtype),
-                               tile_height(T.stage, fdtype), tile_levels(T.stage, fdtype));
+    const int rs = run_stage(T.stage, fdtype);
+    dv[q].ptiles = item_ptiles(dv[q].nx, dv[q].ny, dv[q].nz, T.level_inner, tile_width(rs), tile_height(rs),
+                               tile_levels(rs));
     if (dv[q].ptiles >= (1L << 31)) return fail(ADZ_EINVAL, "adz_plan_create: an item of 2^31 tiles or more");
     dv[q].tile0 = tiles;
     tiles += dv[q].ptiles * dv[q].ngroups;
@@ -1751,10 +1830,11 @@ int adz_plan_create(const adz_item* items, int nitems, int fdtype, int math, int
 
 int adz_plan_execute(const adz_plan* p, adz_stream stream) {
   if (!p) return fail(ADZ_EINVAL, "adz_plan_execute: null plan");
-  void* kern = pick<true>(p->fdtype, p->pdtype, p->math, p->post, p->tune.stage);
+  const int rs = run_stage(p->tune.stage, p->fdtype);
+  void* kern = pick<true>(p->fdtype, p->pdtype, p->math, p->post, rs);
   PlanArgs a = p->args;
   void* args[] = {&a};
-  const unsigned nthr = plan_threads(p->tune.stage, p->fdtype);
+  const unsigned nthr = plan_threads(rs);
   ADZ_HIP_CHECK(hipLaunchKernel(kern, dim3(p->grid), dim3(nthr), args, 0, (hipStream_t)stream));
   return ADZ_OK;
 }
@@ -1817,9 +1897,11 @@ int adz_plan_autotune(const adz_item* items, int nitems, int fdtype, int math, i
   cur.fields_per_pass = std::min(cur.fields_per_pass, maxf);
   float cur_ms = 0.f;
   int rc = time_one(cur, &cur_ms);
-  const int stages[] = {1, 2, 3, 4, 5, 6, 7, 8}, fpps[] = {2, 3, 4, 5, 8, 10, 16, 20, 32, 40, 64},
+  const int f32s[] = {1, 2, 3, 4, 5, 6, 7, 8}, others[] = {1, 2, 5, 6, 7, 8};
+  const int* stages = fdtype == ADZ_F32 ? f32s : others;
+  const int fpps[] = {2, 3, 4, 5, 8, 10, 16, 20, 32, 40, 64},
             bpcs[] = {1, 2, 4, 8, 16, 32}, flags[] = {0, 1}, orders[] = {0, 1, 2, 3, 4, 6, 8};
-  const int nst = fdtype != ADZ_F32 ? 2 : math == ADZ_MATH_F32 ? 8 : 7, nor = 7;
+  const int nst = (fdtype == ADZ_F32 ? 8 : 6) - (math != ADZ_MATH_F32), nor = 7;
   // staging and tile order together first: the LDS-staged forms depend on the L2 reuse the
   // tile order gives, so one is not searched at the other's best value.  Each staging is
   // timed at 4 blocks per CU, blocks of 16 waves at 1 (one of them is resident per CU).
@@ -1828,7 +1910,7 @@ int adz_plan_autotune(const adz_item* items, int nitems, int fdtype, int math, i
       adz_tune t = cur;
       t.stage = stages[s];
       t.level_inner = orders[v];
-      t.blocks_per_cu = plan_threads(t.stage, fdtype) >= 1024 ? 1 : 4;
+      t.blocks_per_cu = plan_threads(run_stage(t.stage, fdtype)) >= 1024 ? 1 : 4;
       if (t.stage == cur.stage && t.level_inner == cur.level_inner && t.blocks_per_cu == cur.blocks_per_cu) continue;
       float ms = 0.f;
       rc = time_one(t, &ms);

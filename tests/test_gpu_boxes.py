@@ -13,7 +13,7 @@ pytestmark = pytest.mark.gpu
 MH = 2
 
 
-def _setup(torch, A, L, ni, nj, nk, halo, fdt, pdt, nf, ext, seed, deform, special):
+def _setup(torch, A, L, ni, nj, nk, halo, fdt, pdt, nf, ext, seed, deform, special, lead=0):
     from gem_amd import tricublin as TC
 
     H = halo if ext else MH
@@ -42,7 +42,8 @@ def _setup(torch, A, L, ni, nj, nk, halo, fdt, pdt, nf, ext, seed, deform, speci
             f[rng.integers(0, f.size, 5)] = np.inf
             f[rng.integers(0, f.size, 5)] = np.nan
             f[rng.integers(0, f.size, 200)] = -0.0
-        src.append(torch.from_numpy(f).to(fdt).cuda())
+        first = lead * (len(src) % 2)  # element its first value is at, in an allocation of its own
+        src.append(torch.cat([torch.zeros(first, dtype=fdt), torch.from_numpy(f).to(fdt)]).cuda()[first:])
     return geom, box, xyz, src, H + nx * H
 
 
@@ -95,4 +96,44 @@ def test_staged_f32_equals_per_lane(cuda, ni, nj, nk, halo, nf, ext, deform, spe
             same = (a.view(np.uint32) == b.view(np.uint32)) | (np.isnan(a) & np.isnan(b))
             if not math_ref:  # minNum / maxNum do not tell +0 from -0
                 same |= (a == 0) & (b == 0)
+            assert same.all(), (stage, q, int((~same).sum()))
+
+
+@pytest.mark.parametrize("post", [0, 1, 3])
+@pytest.mark.parametrize("ni,nj,nk,halo,nf,ext,deform,special", CASES)
+def test_staged_f64_equals_per_lane(cuda, ni, nj, nk, halo, nf, ext, deform, special, post):
+    import torch
+
+    from gem_amd import _lib as L
+    from gem_amd import adz as A
+
+    pdt = torch.float64 if ni % 2 else torch.float32
+    s = _setup(torch, A, L, ni, nj, nk, halo, torch.float64, pdt, nf, ext, ni + nk, deform, special, lead=1)
+    print(f"[boxes] f64 {ni}x{nj}x{nk} nf={nf} ext={ext} deform={deform} post={post}", flush=True)
+    want = _run(torch, A, L, s, torch.float64, L.ADZ_MATH_REF, post, ext, ni, nj, nk, 2)
+    for stage in (3, 4, 5, 6, 7, 8, None, "call"):
+        got = _run(torch, A, L, s, torch.float64, L.ADZ_MATH_REF, post, ext, ni, nj, nk, stage)
+        for q, (a, b) in enumerate(zip(got, want)):
+            same = (a.view(np.uint64) == b.view(np.uint64)) | (np.isnan(a) & np.isnan(b))
+            assert same.all(), (stage, q, int((~same).sum()))
+
+
+@pytest.mark.parametrize("post", [0, 1, 3])
+@pytest.mark.parametrize("lead", [0, 1])  # 1: every other field begins in the middle of a word
+@pytest.mark.parametrize("ni,nj,nk,halo,nf,ext,deform,special", CASES)
+def test_staged_bf16_equals_per_lane(cuda, ni, nj, nk, halo, nf, ext, deform, special, lead, post):
+    import torch
+
+    from gem_amd import _lib as L
+    from gem_amd import adz as A
+
+    pdt = torch.float32 if ni % 2 else torch.float64
+    s = _setup(torch, A, L, ni, nj, nk, halo, torch.bfloat16, pdt, nf, ext, ni + nk, deform, special, lead=lead)
+    print(f"[boxes] bf16 {ni}x{nj}x{nk} nf={nf} ext={ext} lead={lead} deform={deform} post={post}", flush=True)
+    want = _run(torch, A, L, s, torch.bfloat16, L.ADZ_MATH_F32, post, ext, ni, nj, nk, 2)
+    for stage in (3, 4, 5, 6, 7, 8, None, "call"):
+        got = _run(torch, A, L, s, torch.bfloat16, L.ADZ_MATH_F32, post, ext, ni, nj, nk, stage)
+        for q, (a, b) in enumerate(zip(got, want)):
+            # minNum / maxNum do not tell +0 from -0
+            same = (a.view(np.uint32) == b.view(np.uint32)) | (np.isnan(a) & np.isnan(b)) | ((a == 0) & (b == 0))
             assert same.all(), (stage, q, int((~same).sum()))
