@@ -48,9 +48,8 @@ struct DevItem {
 };
 
 // Can boxes of elements of `size` bytes be staged, and their outputs stored, at 32-bit byte
-// offsets?  (2-byte elements: every row must begin at the same half of a 4-byte word.)
+// offsets?
 __host__ __device__ inline bool stageable(const DevItem& it, int size) {
-  if (size == 2 && ((it.lv.ni | it.lv.nij) & 1)) return false;
   return it.span && it.dspan && (long)(it.span / 4) * size < 0x7fffffffL && (long)it.dspan * size < 0x7fffffffL;
 }
 
@@ -276,25 +275,6 @@ __device__ __forceinline__ void per_lane(const DevItem& it, const Fields& F, int
       }
       return;
     }
-  }
-  if constexpr (sizeof(TF) == 2) {
-    const long o1 = x.zlinear ? 0 : gnij, o2 = o1 + gnij, o3 = o2 + o1;
-    for (int f = f0; f < f1; f++) {
-      if (ok) {
-        typedef ADZ_GLOBAL u32x2 __attribute__((aligned(2))) Quad;
-        const ADZ_GLOBAL char* s = (const ADZ_GLOBAL char*)F.s(f) + 2 * x.off;
-        u32x2 v[4][4];
-#pragma unroll
-        for (int r = 0; r < 4; r++)
-#pragma unroll
-          for (int z = 0; z < 4; z++)
-            v[r][z] = *(const Quad*)(s + 2 * (r * gni + (z == 0 ? 0 : (z == 1 ? o1 : (z == 2 ? o2 : o3)))));
-        eval_store_a<TF, MATH, POST>(F, f, HalfStencil{v}, cw, o);
-      } else if (valid) {
-        store_nan<TF, MATH, POST>(F, f, o);
-      }
-    }
-    return;
   }
   for (int f = f0; f < f1; f++) {
     if (ok)
@@ -1025,28 +1005,47 @@ __device__ __forceinline__ void shared_tile(const DevItem& it, const Fields& F, 
 // planes of a box dominate its volume: DMA bytes per target and field on 512 x 384 x 84 are
 // 39.7 for 64 x 4 x 1, 29.9 for 64 x 8 x 1, 24.5 for 64 x 4 x 2 and 16.9 for 64 x 4 x 4.
 //   * FP64 fields: rows of 80 elements (five times round the banks), 62 per buffer, so that
-//     two blocks of eight waves fit a CU.  BF16 fields: rows of 128 elements; the quads begin
-//     at the word that holds the box's first column, a lane reads the three words that hold
-//     its four columns and shifts them (reading 2-byte values took 190 us where this takes
-//     72, and per-lane loads 115).
-// What bounds it: 6 FP32 fields, no lin/min/max (stage 7): LDS reads (256 B per point-field, 58 %
-// of the cycles, a quarter of those still bank conflicts), FP32 arithmetic (100 instructions
-// per field and 40 per field for the tile's indexes, weights and box: 54 %) and the texture
-// unit's DMA (41 %), none hidden completely behind another with 16 waves per CU.
+//     two blocks of eight waves fit a CU.  BF16 fields: rows of 128 elements; the quads of a
+//     row begin at the word that holds the box's first column, a lane reads the three words
+//     that hold its four columns and shifts them (reading 2-byte values took 190 us where
+//     this takes 72, and per-lane loads 115).
+// What bounds it: 6 FP32 fields, no lin/min/max (stage 7): LDS reads (256 B per point-field),
+// FP32 arithmetic (100 instructions per field and 40 per field for the tile's indexes, weights
+// and box) and the texture unit's DMA, 58, 54 and 41 % of the cycles with 16 waves per CU,
+// none hidden completely behind another; with 24 waves 0.85 of that time.
 
 // elements per LDS row: whole rounds of the 32 banks
 template <class TF> constexpr int box_pitch() { return sizeof(TF) == 8 ? 80 : sizeof(TF) == 4 ? 96 : 128; }
 constexpr int kTJ6 = 8;                    // target rows of a staging-mode-6 tile
 template <class TF> constexpr int quads_per_row() { return box_pitch<TF>() * (int)sizeof(TF) / 16; }
-// rows per LDS buffer for blocks of W waves
-// (8-byte elements: 62 rows, so that two blocks of two buffers fit a CU's 160 KB)
-template <class TF, int W> constexpr int box_rows() { return sizeof(TF) == 8 ? 62 : W >= 8 ? 85 : 64; }
+// How the blocks of staging modes 5 to 8 fill a CU:
+//   * One tile per block for blocks of four and eight waves: the hardware fills a CU with the
+//     next ones as blocks end.  In a persistent loop over the tiles the loop's state went to
+//     memory (one clipped FP32 field of 800 x 500 x 84 in the reference's arithmetic 1151 ->
+//     860 us).  Blocks of 16 waves, of which a CU holds one, loop: the waves that are done
+//     start on the next tile (10 fields of 1024 x 512 x 84 with lin/min/max 3.6 ms, 4.4 with
+//     one tile per block).
+//   * Six waves per SIMD, three blocks of eight waves per CU, for 4- and 2-byte fields, which
+//     nothing hides the tile's extents and its first box from but other blocks: 16
+//     subdomains x 6 fields 4.49 -> 3.82 ms, 2 fields of 800 x 500 x 84 716 -> 605 us.  Not in
+//     the reference's arithmetic with clipping or lin/min/max, which does not fit 80 VGPRs
+//     (one field of 304 x 227 x 84 127 -> 317 us); there, and for FP64 boxes, four.
+constexpr bool one_tile(int waves) { return waves <= 8; }
+constexpr int dma_waves(int size, int waves, int math, int post) {
+  return waves == 8 && size <= 4 && (math == ADZ_MATH_F32 || !post) ? 6 : 4;
+}
+
+// rows per LDS buffer for blocks of W waves, S waves per SIMD: as many as fit the CU's 160 KB
+// (FP32, eight waves: two blocks with S = 4, three with S = 6, in whole rounds of the waves)
+template <class TF, int W, int S> constexpr int box_rows() {
+  return sizeof(TF) == 8 ? 62 : W == 4 || (sizeof(TF) == 4 && S == 6) ? 64 : 85;
+}
 // DMA instructions (1 KB each) that fill a buffer, dealt out to the waves in turn.  Lanes
 // without a quad ask for one out of range and get zeros.
-template <class TF, int W> constexpr int box_dma() { return (box_rows<TF, W>() * quads_per_row<TF>() + 63) / 64; }
-template <class TF, int W> constexpr int dma_per_wave() { return (box_dma<TF, W>() + W - 1) / W; }
-template <class TF, int W> constexpr int box_elems() { return box_dma<TF, W>() * 1024 / (int)sizeof(TF); }
-static_assert(box_rows<float, 8>() < 128 && box_rows<double, 8>() < 128, "row split by a float reciprocal below");
+template <class TF, int W, int S> constexpr int box_dma() { return (box_rows<TF, W, S>() * quads_per_row<TF>() + 63) / 64; }
+template <class TF, int W, int S> constexpr int dma_per_wave() { return (box_dma<TF, W, S>() + W - 1) / W; }
+template <class TF, int W, int S> constexpr int box_elems() { return box_dma<TF, W, S>() * 1024 / (int)sizeof(TF); }
+static_assert(box_rows<float, 8, 4>() < 128 && box_rows<double, 8, 4>() < 128, "row split by a float reciprocal below");
 
 // s_waitcnt immediate (gfx9): at most n vector-memory operations outstanding, the other
 // counters not waited for
@@ -1167,7 +1166,8 @@ template <class TF, int MATH, int POST, class TP, int TH, int TL, class Fields>
 __device__ __forceinline__ void dma_tile(const DevItem& it, const Fields& F, long ptile, int f0, int f1, TF* boxA,
                                          TF* boxB, int* red, unsigned nth, int level_inner) {
   constexpr int W = TH * TL;                  // waves of the block: one per target row and level
-  constexpr int kRows = box_rows<TF, W>(), kN = dma_per_wave<TF, W>();
+  constexpr int S = dma_waves(sizeof(TF), W, MATH, POST);  // waves per SIMD
+  constexpr int kRows = box_rows<TF, W, S>(), kN = dma_per_wave<TF, W, S>();
   constexpr int kPitch = box_pitch<TF>(), kQ = quads_per_row<TF>(), kE = 16 / (int)sizeof(TF), SZ = (int)sizeof(TF);
   constexpr int kSt = POST & ADZ_POST_STORE ? 4 : 1;  // stores per field
   const int lane = threadIdx.x & (kTI - 1), wv = threadIdx.x / kTI;
@@ -1213,11 +1213,11 @@ __device__ __forceinline__ void dma_tile(const DevItem& it, const Fields& F, lon
   }
   // this lane's DMA slots: instruction q of wave wv fills the 64 quads g*64 .. g*64+63 of
   // the buffer (g = wv + W q), quad Q = row Q / kQ, column quad Q % kQ; byte offsets from
-  // minoff of the lane's quad, or `span` (out of range) where the box has none
+  // minoff of the lane's quad, or one out of range where the box has none
   // (32-bit arithmetic: every offset is below 2^31; R / nyb by a float reciprocal, exact
   // since R < 128 and nyb < 128 keep (R + 0.5) / nyb >= 1/256 from an integer, far above the
   // float product's error)
-  const int rel0 = (int)__builtin_amdgcn_readfirstlane((int)first) & (SZ == 2 ? ~1 : ~0);
+  const int rel0 = (int)__builtin_amdgcn_readfirstlane((int)first);
   const int ni32 = (int)gni, nij32 = (int)gnij;
   const float rnyb = 1.0f / (float)nyb;
   int rel[kN];
@@ -1226,16 +1226,17 @@ __device__ __forceinline__ void dma_tile(const DevItem& it, const Fields& F, lon
     const int Q = (wv + W * q) * 64 + lane;
     const int R = Q / kQ, cq = Q - R * kQ;
     const int zz = (int)(((float)R + 0.5f) * rnyb), yy = R - zz * nyb;
-    rel[q] = R < nrows && cq < cpr ? SZ * (rel0 + kE * cq + yy * ni32 + zz * nij32) : (int)span;
+    rel[q] = R < nrows && cq < cpr ? SZ * (rel0 + kE * cq + yy * ni32 + zz * nij32) : (int)span + 4;
   }
   // plane bases of this lane's stencil in a buffer (elements)
-  int lb[4] = {0, 0, 0, 0};
+  int lb[4] = {0, 0, 0, 0}, odd[4] = {0, 0, 0, 0};  // odd: parity of the source row of the stencil's first row
   if (ok) {
     const int r0 = x.iy - 1 - y0, pz0 = x.pz - z0, c0 = x.ix - 1 - x0;
 #pragma unroll
     for (int z = 0; z < 4; z++) {
       const int dz = x.zlinear ? (z >> 1) : z;
       lb[z] = (r0 + nyb * (pz0 + dz)) * kPitch + c0;
+      if constexpr (SZ == 2) odd[z] = (rel0 + r0 * ni32 + (pz0 + dz) * nij32) & 1;
     }
   }
   const int so = valid ? (int)od * SZ : (int)it.dspan * SZ;  // invalid lanes store out of range (dropped)
@@ -1257,21 +1258,23 @@ __device__ __forceinline__ void dma_tile(const DevItem& it, const Fields& F, lon
       asm volatile("" : "+s"(q->l), "+s"(q->n), "+s"(q->x));
     }
   };
-  // 2-byte elements: the quads begin at the 4-byte word that holds the box's first column, one
-  // element early (half_of = 1) where that is the word's second half; with `first` odd, rel0
-  // is one element early already.
+  // 2-byte elements: the quads of a row begin at the 4-byte word that holds the box's first
+  // column in that row, one element early where that is the word's second half: where the
+  // row's element offset from minoff and the element that minoff is in its word (half_of, of
+  // each field) sum up odd.
   auto half_of = [&](const void* src) -> int {
     if constexpr (SZ != 2) return 0;
-    return (int)((((unsigned long long)src >> 1) + (unsigned long long)(it.minoff + first)) & 1);
+    return (int)(((unsigned long long)src / 2 + (unsigned long long)it.minoff) & 1);
   };
-  const int wu = box_dma<TF, W>() % W ? (int)__builtin_amdgcn_readfirstlane(wv) : 0;
+  const int wu = box_dma<TF, W, S>() % W ? (int)__builtin_amdgcn_readfirstlane(wv) : 0;
   auto issue = [&](const void* src, bool on, TF* buf) {
-    const int d = SZ == 2 ? ((int)first & 1) - half_of(src) : 0;  // elements from rel0's to the quads' begin
-    const __amdgpu_buffer_rsrc_t rs = field_rsrc((const TF*)src + it.minoff + d, on ? span - SZ * d : 0u);
+    const int h = half_of(src);
+    const __amdgpu_buffer_rsrc_t rs = field_rsrc((const TF*)src + it.minoff - h, on ? span + SZ * h : 0u);
 #pragma unroll
     for (int q = 0; q < kN; q++)
-      if (box_dma<TF, W>() % W == 0 || wu + W * q < box_dma<TF, W>()) __builtin_amdgcn_raw_ptr_buffer_load_lds(
-          rs, (__attribute__((address_space(3))) void*)(buf + (wv + W * q) * (1024 / SZ)), 16, rel[q], 0, 0, 0);
+      if (box_dma<TF, W, S>() % W == 0 || wu + W * q < box_dma<TF, W, S>()) __builtin_amdgcn_raw_ptr_buffer_load_lds(
+          rs, (__attribute__((address_space(3))) void*)(buf + (wv + W * q) * (1024 / SZ)), 16,
+          SZ == 2 ? (rel[q] + 2 * h) & ~3 : rel[q], 0, 0, 0);
   };
   auto dst = [&](void* base) { return field_rsrc((TF*)base + it.omin, it.dspan * SZ); };
   // Every lane evaluates (one without a stencil reads its buffer's first values and stores NaN
@@ -1280,16 +1283,20 @@ __device__ __forceinline__ void dma_tile(const DevItem& it, const Fields& F, lon
   auto eval = [&](const Ptr& P, int half, const TF* buf) {
     TC v = 0, l = 0, mi = 0, ma = 0;
     if constexpr (SZ == 2) {
-      // a stencil row from the three words that hold it
+      // a stencil row from the three words that hold it; with rows of odd length every other
+      // one begins at the other half of a word
       u32x2 q[4][4];
-      const unsigned sh = 16 * ((lb[0] + half) & 1);
+      const int other = ni32 & 1;
 #pragma unroll
       for (int z = 0; z < 4; z++) {
-        const unsigned* b = (const unsigned*)buf + ((lb[z] + half) >> 1);
+        const int h = odd[z] ^ half, e0 = lb[z] + h, e1 = lb[z] + (h ^ other);
+        const unsigned* b0 = (const unsigned*)buf + (e0 >> 1);
+        const unsigned* b1 = (const unsigned*)buf + (e1 >> 1);
 #pragma unroll
         for (int r = 0; r < 4; r++) {
-          const unsigned w0 = b[r * (kPitch / 2)], w1 = b[r * (kPitch / 2) + 1], w2 = b[r * (kPitch / 2) + 2];
-          q[r][z] = u32x2{__builtin_amdgcn_alignbit(w1, w0, sh), __builtin_amdgcn_alignbit(w2, w1, sh)};
+          const unsigned* b = (r & 1 ? b1 : b0) + r * (kPitch / 2);
+          const unsigned sh = (unsigned)(r & 1 ? e1 : e0) << 4;  // 16 where odd (a shift of 32 bits or more is taken modulo 32)
+          q[r][z] = u32x2{__builtin_amdgcn_alignbit(b[1], b[0], sh), __builtin_amdgcn_alignbit(b[2], b[1], sh)};
         }
       }
       eval_vals<TF, MATH, POST>(HalfStencil{q}, cw, &v, &l, &mi, &ma);
@@ -1351,9 +1358,49 @@ __device__ __forceinline__ void dma_tile(const DevItem& it, const Fields& F, lon
   __builtin_amdgcn_s_waitcnt(vmcnt_imm(kSt));  // no load into LDS is left behind
 }
 
+// Entry t of a plan's tile list: its item, tile and fields [f0, f1).
+struct PlanTile {
+  DevItem it;
+  long ptile;
+  int f0, f1;
+  __device__ __forceinline__ ItemFields fields() const { return ItemFields{it.src, it.dst, it.lin, it.mn, it.mx}; }
+};
+__device__ __forceinline__ PlanTile plan_tile(const PlanArgs& A, long t) {
+  PlanTile P;
+  DevItem& it = P.it;
+  int q = 0;
+  // The item table does not change during a launch: read through the constant address
+  // space, the (uniform) item's fields come in with scalar loads.
+  typedef const DevItem __attribute__((address_space(4))) CItem;
+  const CItem* items = (const CItem*)A.items;
+  while (q + 1 < A.nitems && items[q + 1].tile0 <= t) q++;
+  {
+    static_assert(sizeof(DevItem) % 8 == 0, "DevItem is copied in 8-byte words");
+    typedef const unsigned long long __attribute__((address_space(4))) CWord;
+    const CWord* w = (const CWord*)(A.items + q);
+    unsigned long long* d = (unsigned long long*)&it;
+#pragma unroll
+    for (int e = 0; e < (int)(sizeof(DevItem) / 8); e++) d[e] = w[e];
+  }
+  const long local = t - it.tile0;
+  long ptile, grp;
+  if (local < (1L << 31)) {  // 32-bit division (the usual case)
+    const unsigned lo32 = (unsigned)local;
+    if (A.points_outer) { const unsigned q = lo32 / (unsigned)it.ngroups; ptile = q; grp = lo32 - q * (unsigned)it.ngroups; }
+    else { const unsigned q = lo32 / (unsigned)it.ptiles; grp = q; ptile = lo32 - q * (unsigned)it.ptiles; }
+  } else {
+    if (A.points_outer) { ptile = local / it.ngroups; grp = local % it.ngroups; }
+    else { grp = local / it.ptiles; ptile = local % it.ptiles; }
+  }
+  P.ptile = ptile;
+  P.f0 = (int)grp * A.g;
+  P.f1 = min(it.nf, P.f0 + A.g);
+  return P;
+}
+
 // Persistent loop over the tile list of a plan.
-template <class TF, class TP, int MATH, int POST, int STAGE>
-__device__ __forceinline__ void plan_loop(const PlanArgs& A, TF* boxA, TF* boxB, int* red, int* rowoff) {
+template <class Body>
+__device__ __forceinline__ void each_tile(const PlanArgs& A, Body body) {
   long lo = 0, hi = A.ntiles, step = gridDim.x, t0 = blockIdx.x;
   if (A.xcd_chunks) {
     int nb = gridDim.x / 8;                 // blocks per XCD (grid is a multiple of 8)
@@ -1363,48 +1410,20 @@ __device__ __forceinline__ void plan_loop(const PlanArgs& A, TF* boxA, TF* boxB,
     step = nb;
     t0 = lo + l;
   }
-  unsigned nth = 0;
   for (long t = t0; t < hi; t += step) {
-    int q = 0;
-    // The item table does not change during a launch: read through the constant address
-    // space, the (uniform) item's fields come in with scalar loads.
-    typedef const DevItem __attribute__((address_space(4))) CItem;
-    const CItem* items = (const CItem*)A.items;
-    while (q + 1 < A.nitems && items[q + 1].tile0 <= t) q++;
-    DevItem it;
-    {
-      static_assert(sizeof(DevItem) % 8 == 0, "DevItem is copied in 8-byte words");
-      typedef const unsigned long long __attribute__((address_space(4))) CWord;
-      const CWord* w = (const CWord*)(A.items + q);
-      unsigned long long* d = (unsigned long long*)&it;
-#pragma unroll
-      for (int e = 0; e < (int)(sizeof(DevItem) / 8); e++) d[e] = w[e];
-    }
-    const long local = t - it.tile0;
-    long ptile, grp;
-    if (local < (1L << 31)) {  // 32-bit division (the usual case)
-      const unsigned lo32 = (unsigned)local;
-      if (A.points_outer) { const unsigned q = lo32 / (unsigned)it.ngroups; ptile = q; grp = lo32 - q * (unsigned)it.ngroups; }
-      else { const unsigned q = lo32 / (unsigned)it.ptiles; grp = q; ptile = lo32 - q * (unsigned)it.ptiles; }
-    } else {
-      if (A.points_outer) { ptile = local / it.ngroups; grp = local % it.ngroups; }
-      else { grp = local / it.ptiles; ptile = local % it.ptiles; }
-    }
-    int f0 = (int)grp * A.g, f1 = min(it.nf, f0 + A.g);
-    ItemFields F{it.src, it.dst, it.lin, it.mn, it.mx};
-    if constexpr (STAGE == 4 && std::is_same<TF, float>::value)
-      shared_tile<MATH, POST, TP>(it, F, ptile, f0, f1, A.level_inner);
-    else if constexpr (STAGE == 5)
-      dma_tile<TF, MATH, POST, TP, kTJ, 1>(it, F, ptile, f0, f1, boxA, boxB, red, nth++, A.level_inner);
-    else if constexpr (STAGE == 6)
-      dma_tile<TF, MATH, POST, TP, kTJ6, 1>(it, F, ptile, f0, f1, boxA, boxB, red, nth++, A.level_inner);
-    else if constexpr (STAGE == 7)
-      dma_tile<TF, MATH, POST, TP, kTJ, 2>(it, F, ptile, f0, f1, boxA, boxB, red, nth++, A.level_inner);
-    else if constexpr (STAGE == 8)
-      dma_tile<TF, MATH, POST, TP, kTJ, 4>(it, F, ptile, f0, f1, boxA, boxB, red, nth++, A.level_inner);
-    else
-      run_tile<TF, TP, MATH, POST, ItemFields>(it, F, ptile, f0, f1, boxA, boxB, red, rowoff, STAGE, A.level_inner);
+    const PlanTile P = plan_tile(A, t);
+    body(P);
   }
+}
+template <class TF, class TP, int MATH, int POST, int STAGE>
+__device__ __forceinline__ void plan_loop(const PlanArgs& A, TF* boxA, TF* boxB, int* red, int* rowoff) {
+  each_tile(A, [&](const PlanTile& P) {
+    if constexpr (STAGE == 4 && std::is_same<TF, float>::value)
+      shared_tile<MATH, POST, TP>(P.it, P.fields(), P.ptile, P.f0, P.f1, A.level_inner);
+    else
+      run_tile<TF, TP, MATH, POST, ItemFields>(P.it, P.fields(), P.ptile, P.f0, P.f1, boxA, boxB, red, rowoff, STAGE,
+                                               A.level_inner);
+  });
 }
 
 // Persistent kernel: STAGE 1 stages each tile's source box in LDS, STAGE 2 reads per lane,
@@ -1423,21 +1442,41 @@ __global__ __launch_bounds__(kTile) void k_plan(PlanArgs A) {
   }
 }
 
-// Staging modes 5 to 8 (tiles of TH target rows x TL levels, one wave per row
-// and level): their own kernel.  In the FP32 arithmetic it is held to 128 VGPRs, so that the
-// blocks its two LDS buffers allow per CU keep four waves on every SIMD; the reference
-// arithmetic needs more registers than that without spilling (and has no 16-wave form).
-template <int TH, int TL> constexpr int dma_stage() { return TL == 4 ? 8 : TL == 2 ? 7 : TH == kTJ ? 5 : 6; }
-#define ADZ_BOXES(TF, W)                                                              \
-  __shared__ __attribute__((aligned(16))) TF boxA[box_elems<TF, W>()];                                             \
-  __shared__ __attribute__((aligned(16))) TF boxB[box_elems<TF, W>() + 2];                                           \
+// Tile of this block, >= n where it has none: in the order of the blocks, or (chunks) an
+// eighth of the list for each of the 8 XCDs, to which the hardware deals blocks in turn.
+// The grid has two dimensions, since one holds less than 2^32 threads.
+constexpr long kGridX = 1L << 21;  // blocks per row of the grid: a multiple of 8
+__device__ __forceinline__ long tile_of_block(long n, int chunks) {
+  const long b = (long)blockIdx.y * kGridX + blockIdx.x;
+  if (!chunks) return b;
+  const long per = (n + 7) / 8, l = b / 8;
+  return l < per ? b % 8 * per + l : n;
+}
+inline dim3 tile_grid(long n) {
+  const long b = 8 * ((n + 7) / 8);
+  return dim3((unsigned)(b < kGridX ? b : kGridX), (unsigned)((b + kGridX - 1) / kGridX));
+}
+#define ADZ_BOXES(TF, W, S)                                                              \
+  __shared__ __attribute__((aligned(16))) TF boxA[box_elems<TF, W, S>()];                                             \
+  __shared__ __attribute__((aligned(16))) TF boxB[box_elems<TF, W, S>() + 2];                                           \
   __shared__ int red[18];                                                             \
   if (threadIdx.x < 18) red[threadIdx.x] = kFar;                                      \
   __syncthreads();
 template <class TF, class TP, int MATH, int POST, int TH, int TL>
-__global__ __launch_bounds__(64 * TH * TL, 4) void k_plan5(PlanArgs A) {
-  ADZ_BOXES(TF, TH * TL)
-  plan_loop<TF, TP, MATH, POST, dma_stage<TH, TL>()>(A, boxA, boxB, red, nullptr);
+__global__ __launch_bounds__(64 * TH * TL, dma_waves(sizeof(TF), TH * TL, MATH, POST)) void k_plan5(PlanArgs A) {
+  ADZ_BOXES(TF, TH * TL, dma_waves(sizeof(TF), TH * TL, MATH, POST))
+  if constexpr (one_tile(TH * TL)) {
+    const long t = tile_of_block(A.ntiles, A.xcd_chunks);
+    if (t >= A.ntiles) return;  // the whole block leaves: no barrier is reached
+    const PlanTile P = plan_tile(A, t);
+    dma_tile<TF, MATH, POST, TP, TH, TL>(P.it, P.fields(), P.ptile, P.f0, P.f1, boxA, boxB, red, 0, A.level_inner);
+  } else {
+    unsigned nth = 0;
+    each_tile(A, [&](const PlanTile& P) {
+      dma_tile<TF, MATH, POST, TP, TH, TL>(P.it, P.fields(), P.ptile, P.f0, P.f1, boxA, boxB, red, nth++,
+                                           A.level_inner);
+    });
+  }
 }
 
 // One item with inline field pointers (the adz_tricub_hlt entry point).
@@ -1460,10 +1499,10 @@ constexpr int kHltOrder = 0;
 constexpr int kHltTH = kTJ, kHltTL = 2;
 
 template <class TF, class TP, int MATH, int POST>
-__global__ __launch_bounds__(64 * kHltTH * kHltTL, 4) void k_hlt5(DevItem it, InlineFields F, long ntiles) {
-  ADZ_BOXES(TF, kHltTH * kHltTL)
-  const long per = (ntiles + 7) / 8;
-  const long t = (long)(blockIdx.x % 8) * per + blockIdx.x / 8;
+__global__ __launch_bounds__(64 * kHltTH * kHltTL,
+                                  dma_waves(sizeof(TF), kHltTH * kHltTL, MATH, POST)) void k_hlt5(DevItem it, InlineFields F, long ntiles) {
+  ADZ_BOXES(TF, kHltTH * kHltTL, dma_waves(sizeof(TF), kHltTH * kHltTL, MATH, POST))
+  const long t = tile_of_block(ntiles, 1);
   if (t >= ntiles) return;  // the whole block leaves: no barrier is reached
   dma_tile<TF, MATH, POST, TP, kHltTH, kHltTL>(it, F, t, 0, it.nf, boxA, boxB, red, 0, kHltOrder);
 }
@@ -1626,46 +1665,51 @@ void* pick(int fdt, int pdt, int math, int post, int stage = 2) {
 
 int field_bytes(int fdtype) { return fdtype == ADZ_F64 ? 8 : fdtype == ADZ_F32 ? 4 : 2; }
 
-// Built-in tile parameters, ten fields per pass, LDS-staged boxes:
-//   * FP32 fields in FP32 arithmetic with lin/min/max: tiles of 64 x 4 targets x 4 levels (stage 8; the
-//     fewest DMA bytes per target, and the stores leave no room for more).  10 fields of
-//     1024 x 512 x 84 3.61 ms (64 x 4 x 2: 3.8 to 4.5; before 4.15), rows, then levels,
-//     with 8 blocks per CU to even out the ends; where a plane outgrows an XCD's L2 (2048 x
-//     1024: 13.6 ms) super-columns of 3 tile rows with one block per CU (rows, then levels:
-//     15.8 ms; 1024 x 512 in super-columns: 3.9 ms);
-//   * FP32 fields otherwise, tiles of 64 x 4 targets x 2 levels (stage 7): two blocks per CU, one
-//     evaluates while the other waits.  16 subdomains x 6 fields in FP32 4.48 ms (stage 8:
-//     5.1; before 6.96), 6 fields of 512 x 384 x 84 in the reference's arithmetic with
-//     lin/min/max 1.33 ms (stage 5: 1.40; before 1.82).
-//   * FP64 fields: the same tiles in super-columns of two tile rows, since only two such
-//     blocks fit a CU's LDS.  4 fields of 511 x 385 x 84 0.75 ms (stage 5: 1.02; per-lane
-//     loads 1.30), with clipping 1.16 (1.42; 2.21);
-//   * BF16 fields: tiles of 64 x 4 targets (stage 5), whose boxes are small in bytes, with
-//     four blocks per CU.  4 clipped fields of 200 x 150 x 60 72 us (stage 7: 77; per-lane
-//     loads 115), of 600 x 400 x 60 0.62 ms (0.65; 1.09).
-// Items beyond 32-bit offsets, and BF16 ones with rows or planes of odd length: per-lane
-// loads (stage 2).
-adz_tune default_tune(int fdtype, int math, int post, bool staged, long plane_bytes) {
+// Too few fields to pay for a tile's extents and its first box?  One FP32 or unclipped FP64
+// field below 2^24 targets, or one clipped FP32 field in the reference's arithmetic.  Per-lane
+// loads (staged boxes), us, 304 x 227 x 84 and 800 x 500 x 84: FP32 arithmetic, one field 65
+// (78) and 427 (458), clipped 84 (88) and 595 (530), two 105 (98) and 750 (601); reference
+// arithmetic, one field 83 (96) and 575 (553), clipped 107 (134) and 737 (855), two clipped 183
+// (183) and 1257 (1135); FP64, one field 115 (120) and 803 (748), clipped 181 (150) and 1278
+// (946); BF16, one field 90 (93) and 585 (570).
+bool few_fields(int fdtype, int math, int post, long targets, int fields) {
+  if (fields > 1 || fdtype == ADZ_BF16 || (fdtype == ADZ_F64 && post)) return false;
+  return targets < (1L << 24) || (math != ADZ_MATH_F32 && post);
+}
+
+// Built-in tile parameters: ten fields per pass, LDS-staged boxes of tiles of 64 x 4 targets x
+// 2 levels (stage 7; its eight-wave blocks leave the most of them on a CU).  Times of stage 7
+// (of stage 5, stage 8, per-lane loads), ms:
+//   16 subdomains to 512 x 384 x 6 FP32 fields, FP32 arithmetic  3.84 (4.94, 5.09, 6.22)
+//   10 fields with lin/min/max, 1024 x 512 x 84                  3.51 (4.30, 3.70, 6.87)
+//   10 fields with lin/min/max, 2048 x 1024 x 84                14.2 (17.4, 14.7, 30.1)
+//   4 clipped FP32 fields, reference arithmetic, the same grid   8.73 (8.99, -, 11.1)
+//   4 FP64 fields, 511 x 385 x 84                                0.71 (1.02, -, 1.29)
+//   4 clipped BF16 fields, 600 x 400 x 60                        0.57 (0.65, 0.73, 1.07)
+// Tiles walk rows, then levels, where lin/min/max are stored (levels first, 3.95 and 15.5 ms
+// in lines two and three), else the levels of a column first (rows first 3.95 ms in line
+// one); FP64 fields super-columns of two tile rows (line five; rows first 0.77).
+// Items beyond 32-bit offsets, and too few fields (few_fields): per-lane loads (stage 2).
+adz_tune default_tune(int fdtype, int math, int post, bool staged, long targets, int fields) {
   if (!staged) return adz_tune{10, 0, 4, 1, 2, 3};
-  if (fdtype == ADZ_F64) return adz_tune{10, 0, 32, 1, 7, 2};
-  if (fdtype == ADZ_BF16) return adz_tune{10, 0, 16, 1, 5, 0};
-  if (math != ADZ_MATH_F32) return adz_tune{10, 0, 16, 1, 7, 0};
-  if (!(post & ADZ_POST_STORE)) return adz_tune{10, 0, 32, 1, 7, 3};
-  return plane_bytes <= (4L << 20) ? adz_tune{10, 0, 8, 1, 8, 0} : adz_tune{10, 0, 1, 1, 8, 3};
+  if (few_fields(fdtype, math, post, targets, fields)) return adz_tune{10, 0, 32, 1, 2, targets < (1L << 24) ? 1 : 0};
+  return adz_tune{10, 0, 8, 1, 7, fdtype == ADZ_F64 ? 2 : post & ADZ_POST_STORE ? 0 : 1};
 }
 adz_tune default_tune(const adz_item* items, int nitems, int fdtype, int math, int post) {
   bool staged = true;
-  long plane = 0;
+  long targets = 0;
+  int fields = 0;
   for (int q = 0; q < nitems && items; q++) {
     const adz_item& a = items[q];
     DevItem d;
     if (fill_item(&d, a.geom, a.xyz, a.i0, a.in, a.j0, a.jn, a.k0, a.nk, a.dminx, a.dmaxx, a.dminy, a.dmaxy, a.ext,
                   a.nptr)) {
       staged = staged && stageable(d, field_bytes(fdtype));
-      plane = std::max(plane, (long)d.lv.nij * field_bytes(fdtype));
+      targets += (long)d.nx * d.ny * d.nz;
+      fields = std::max(fields, a.nptr);
     }
   }
-  return default_tune(fdtype, math, post, staged, plane);
+  return default_tune(fdtype, math, post, staged, targets, fields);
 }
 // targets per tile along i: kSW for the shared-column staging of FP32 sources, else kTI
 
@@ -1724,13 +1768,13 @@ int adz_tricub_hlt(const adz_field* fld, int nptr, const void* xyz, int pdtype, 
       const adz_field& a = fld[f0 + f];
       F.src[f] = a.src; F.dst[f] = a.dst; F.lin[f] = a.lin; F.mn[f] = a.mn; F.mx[f] = a.mx;
     }
-    const bool staged = stageable(it, field_bytes(fdtype));
+    const bool staged = stageable(it, field_bytes(fdtype)) &&
+                        !few_fields(fdtype, math, post, (long)it.nx * it.ny * it.nz, nf);
     void* kern = pick<false>(fdtype, pdtype, math, post, staged ? 7 : 2);
     if (staged) {  // k_hlt5: LDS-staged boxes, an eighth of the tile list per XCD
       long ntiles = item_ptiles(it.nx, it.ny, it.nz, kHltOrder, kTI, kHltTH, kHltTL);
-      long grid = 8 * ((ntiles + 7) / 8);  // one block per tile
       void* args[] = {&it, &F, &ntiles};
-      ADZ_HIP_CHECK(hipLaunchKernel(kern, dim3((unsigned)grid), dim3(64 * kHltTH * kHltTL), args, 0, (hipStream_t)stream));
+      ADZ_HIP_CHECK(hipLaunchKernel(kern, tile_grid(ntiles), dim3(64 * kHltTH * kHltTL), args, 0, (hipStream_t)stream));
     } else {
       void* args[] = {&it, &F};
       ADZ_HIP_CHECK(hipLaunchKernel(kern, dim3((unsigned)it.ptiles), dim3(kTile), args, 0, (hipStream_t)stream));
@@ -1835,7 +1879,7 @@ int adz_plan_execute(const adz_plan* p, adz_stream stream) {
   PlanArgs a = p->args;
   void* args[] = {&a};
   const unsigned nthr = plan_threads(rs);
-  ADZ_HIP_CHECK(hipLaunchKernel(kern, dim3(p->grid), dim3(nthr), args, 0, (hipStream_t)stream));
+  ADZ_HIP_CHECK(hipLaunchKernel(kern, rs >= 5 && one_tile(nthr / 64) ? tile_grid(a.ntiles) : dim3(p->grid), dim3(nthr), args, 0, (hipStream_t)stream));
   return ADZ_OK;
 }
 

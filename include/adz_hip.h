@@ -227,15 +227,16 @@ typedef struct adz_item {
 } adz_item;
 
 /* Tile parameters of the persistent kernel; zero fields_per_pass / blocks_per_cu take the
-   built-in default: ten fields per pass, stage 8 for FP32 fields in the FP32 arithmetic
-   with lin/min/max, stage 5 for BF16 fields, stage 7 otherwise (arrays beyond 32-bit byte
-   offsets, and BF16 ones with rows or planes of odd length: stage 2).  Stage 0 takes the built-in staging together with its level_inner;
-   adz_plan_autotune searches them on the actual plan. */
+   built-in default: ten fields per pass, stage 7 (stage 2 for arrays beyond 32-bit byte
+   offsets, and for one field where that is too few to stage).  Stage 0 takes the built-in
+   staging together with its level_inner; adz_plan_autotune searches them on the actual
+   plan. */
 typedef struct adz_tune {
   int fields_per_pass; /* fields interpolated per pass over the points (1..64)          */
   int points_outer;    /* 1: a block runs every field group of a point tile; 0: a pass
                           over all points per field group                               */
-  int blocks_per_cu;   /* persistent grid = blocks_per_cu * CUs                         */
+  int blocks_per_cu;   /* persistent grid = blocks_per_cu * CUs (stages 5 to 7: a block
+                          per tile)                                                     */
   int xcd_chunks;      /* 1: each XCD takes a contiguous range of tiles                 */
   int stage;           /* 1: stage each tile's source box in LDS; 2: per-lane loads;
                           3 (FP32 sources): one producer wave per block streams the
@@ -243,15 +244,14 @@ typedef struct adz_tune {
                           waves evaluate from LDS; 4 (FP32 sources): each lane loads one
                           stencil column, reduces it for its own and its three left
                           neighbours' targets, partials shared by lane shifts (61-wide
-                          tiles); 5: all four waves copy each field's
-                          box into LDS with 16-byte DMA, double-buffered, and every
-                          lane evaluates from LDS; 6: the same with
-                          tiles of 64 x 8 targets and blocks of eight waves; 7 and 8:
-                          tiles of 64 x 4 targets over 2 and 4 consecutive levels,
-                          blocks of 8 and 16 waves (8: FP32 fields in the reference's
-                          arithmetic ADZ_EINVAL; one block per CU is resident).  FP64
-                          and BF16 sources run stages 3 and 4, and FP64 ones stage 8,
-                          as stage 2                                                    */
+                          tiles); 5: all four waves copy each field's box into LDS
+                          with 16-byte DMA, double-buffered, and every lane evaluates
+                          from LDS; 6: the same with tiles of 64 x 8 targets and blocks
+                          of eight waves; 7 and 8: tiles of 64 x 4 targets over 2 and 4
+                          consecutive levels, blocks of 8 and 16 waves (8: FP32 fields
+                          in the reference's arithmetic ADZ_EINVAL; one block per CU is
+                          resident).  FP64 and BF16 sources run stages 3 and 4, and
+                          FP64 ones stage 8, as stage 2                                 */
   int level_inner;     /* tile order. 0: i, j, then k; 1: consecutive tiles walk the
                           levels of one tile column; S >= 2: super-columns of S tile
                           rows walked level by level (source planes and rows reused
