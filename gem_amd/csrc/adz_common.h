@@ -189,14 +189,16 @@ __device__ __forceinline__ void weights_f32(const Index& x, const ZtabDev& lv, f
 // rows folded by fma, and the x stage accumulated column by column with fma
 // (Tricublin_zyxf3_inline AVX2 path, turbo_tricublin.c:1142-1257).  f points at the
 // stencil corner; ni3/nij3 are the element strides of a row / plane (3*ni, 3*nij).
-template <class TF>
-__device__ __forceinline__ void tricub3_ref(const TF* __restrict__ f, const double* c, long ni3, long nij3,
+template <class TF, class I>
+__device__ __forceinline__ void tricub3_ref(const TF* __restrict__ f, const double* c, I ni3, I nij3,
                                             int zlinear, double* out) {
-  const long o1 = zlinear ? 0 : nij3;
-  const long o2 = o1 + nij3, o3 = o2 + o1;
+  const I o1 = zlinear ? 0 : nij3;
+  const I o2 = o1 + nij3, o3 = o2 + o1;
   // rows outer, the 12 interleaved values of a row inner: only one row's values and the
   // 12 running sums are live at a time (each element keeps the same operation order)
   double dst[12];
+#pragma unroll
+  for (int e = 0; e < 12; e++) dst[e] = -0.0;  // fma(a, b, -0.0) is a * b, signs of zeros included
 #pragma unroll 1
   for (int r = 0; r < 4; r++) {
     const TF* s = f + r * ni3;
@@ -211,7 +213,7 @@ __device__ __forceinline__ void tricub3_ref(const TF* __restrict__ f, const doub
     for (int e = 0; e < 12; e++) za[e] = fma(to_f64(s[e + o3]), c[11], za[e]);
     const double cyr = r == 0 ? c[4] : (r == 1 ? c[5] : (r == 2 ? c[6] : c[7]));  // no dynamic index into c
 #pragma unroll
-    for (int e = 0; e < 12; e++) dst[e] = (r == 0) ? za[e] * cyr : fma(za[e], cyr, dst[e]);
+    for (int e = 0; e < 12; e++) dst[e] = fma(za[e], cyr, dst[e]);
   }
 #pragma unroll
   for (int q = 0; q < 3; q++) {

@@ -15,6 +15,7 @@
 
 #include "adz_common.h"
 #include "adz_qv.h"
+#include "adz_tile.h"
 
 using namespace adz;
 
@@ -139,56 +140,188 @@ __global__ void k_prep_arr(S* __restrict__ uarr, S* __restrict__ varr, S* __rest
 }
 
 // ---------------------------------------------------------------- adz_traject
-// adz_traject.F90:66-104: niter fixed-point updates of one arrival point (i,j,k).
+// adz_traject.F90:66-104: niter fixed-point updates of one arrival point (i,j,k) per lane.
+//
+// A block takes a tile of tw x tr points, at most 256, on kTrajLevels levels (four waves per
+// level; 64 x 4 on wide grids, see traj_tile) and copies the box of the derived winds (three interleaved components) that its points read
+// into LDS; every iteration reduces the box it needs over the block and stages a new one only
+// where that leaves the one in LDS, which has a margin of one element on every side where that
+// fits.  The stencil of a point is 192 values, of which the lanes of a tile read few that
+// differ; as per-lane loads they were 48 16-byte loads per lane and iteration.
+// Rows of the box begin kWindPitch elements apart (a row is one 1 KB DMA instruction of a
+// wave, two in FP64): lanes are three words apart, free of bank conflicts, and rows a multiple
+// of the banks.  A tile whose box does not fit reads per lane, in the same arithmetic and order.
+//
+// What bounds it: FP64 arithmetic.  1024 x 512 x 84 points, three iterations: 4.5 ms as
+// per-lane loads with 70 % of the cycles issuing vector instructions (880 per iteration, 192
+// of them selects and copies for the first row's missing sum, 192 conversions); 3.6 ms now
+// (780 of them, 76 %), where 2.3 ms would be arithmetic alone.  Held to 128 registers, without
+// spills (which cost more than the boxes gain), for two blocks per CU; in FP64 one block fits.
+constexpr int kTrajLevels = 2, kTrajWaves = 4 * kTrajLevels, kTrajRows = 78;
+constexpr int kWindPitch = 256;  // elements
+
+// tricub3_ref (its operations and their order): columns 0 and 1 of the stencil, then 2 and 3,
+// and of each a row of a plane (6 values) at a time with the next one on its way; read(h, r, z,
+// v) gives the values of columns 2h and 2h + 1, row r, plane z.  More values at a time would
+// cost the registers that keep four waves on a SIMD.
+template <class S, class Read>
+__device__ __forceinline__ void tricub3_steps(Read read, const double* c, double* out) {
+  S v[2][6];
+  double dst[6], za[6];
+  auto load = [&](int q) { read(q / 16, q / 4 % 4, q % 4, v[q & 1]); };
+  load(0);
+#pragma unroll
+  for (int q = 0; q < 32; q++) {
+    if (q < 31) load(q + 1);
+#pragma unroll
+    for (int e = 0; e < 6; e++) {
+      const double x = to_f64(v[q & 1][e]);
+      za[e] = q % 4 == 0 ? x * c[8] : fma(x, c[8 + q % 4], za[e]);
+    }
+    // the sums are formed here, and the values of step q + 2 are not read before
+    asm volatile("" : "+v"(za[0]), "+v"(za[1]), "+v"(za[2]), "+v"(za[3]), "+v"(za[4]), "+v"(za[5]) : : "memory");
+    if (q % 4 == 3) {
+      const int r = q / 4 % 4;
+#pragma unroll
+      for (int e = 0; e < 6; e++) dst[e] = r == 0 ? za[e] * c[4] : fma(za[e], c[4 + r], dst[e]);
+      asm volatile("" : "+v"(dst[0]), "+v"(dst[1]), "+v"(dst[2]), "+v"(dst[3]), "+v"(dst[4]), "+v"(dst[5]));
+    }
+    if (q % 16 == 15) {
+#pragma unroll
+      for (int e = 0; e < 3; e++)
+        out[e] = q == 15 ? fma(dst[e + 3], c[1], dst[e] * c[0]) : fma(dst[e + 3], c[3], fma(dst[e], c[2], out[e]));
+    }
+  }
+}
+
 template <class S>
-__global__ __launch_bounds__(256) void k_traject(S* __restrict__ pxyzm, double* __restrict__ wpxyz,
-                                                  S* __restrict__ uvw_dep, const S* __restrict__ uvw_d,
-                                                  const S* __restrict__ uarr, const S* __restrict__ varr,
-                                                  const S* __restrict__ warr, ZtabDev lv, TrajParams P, int niter,
-                                                  double dtA, double dtD, double dtzA, double dtzD) {
-  // 32-bit point index (adz_set refuses tiles of 2^31 points or more)
-  const unsigned a = blockIdx.x * blockDim.x + threadIdx.x;
-  const unsigned nxy = (unsigned)P.ni * (unsigned)P.nj;
-  if (a >= nxy * (unsigned)(P.nk - P.k00 + 1)) return;
-  const unsigned kq = a / nxy, rem = a - kq * nxy, jq = rem / (unsigned)P.ni;
-  const int k = (int)kq + P.k00;
-  const int j = (int)jq + 1;
-  const int i = (int)(rem - jq * (unsigned)P.ni) + 1;
-  long p = p3_idx(P, i, j, k);
-  long aw = (long)(i - 1) + (long)P.ni * (j - 1) + (long)nxy * (k - 1);
-  S px = pxyzm[p], py = pxyzm[p + 1], pz = pxyzm[p + 2];
-  S ud = (S)0, vd = (S)0, wd = (S)0;
-  double xm = 0.0, ym = 0.0, pzm = 0.0;
-  const double ua = (double)uarr[aw], va = (double)varr[aw], wa = (double)warr[aw];
+__global__ __launch_bounds__(64 * kTrajWaves, sizeof(S) == 4 ? 4 : 2) void k_traject(
+    S* __restrict__ pxyzm, double* __restrict__ wpxyz, S* __restrict__ uvw_dep, const S* __restrict__ uvw_d,
+    const S* __restrict__ uarr, const S* __restrict__ varr, const S* __restrict__ warr, ZtabDev lv, TrajParams P,
+    int niter, double dtA, double dtD, double dtzA, double dtzD, unsigned tw, unsigned tr) {
+  __shared__ __attribute__((aligned(16))) S box[kTrajRows * kWindPitch];
+  __shared__ int red[18], moved[3];
+  if (threadIdx.x < 18) red[threadIdx.x] = kFar;
+  if (threadIdx.x < 3) moved[threadIdx.x] = 0;
+  __syncthreads();
+  const unsigned nbi = (P.ni + tw - 1) / tw, nbj = (P.nj + tr - 1) / tr;
+  const unsigned nbk = (P.nk - P.k00 + kTrajLevels) / kTrajLevels;
+  const long ntiles = (long)nbi * nbj * nbk, t = tile_of_block(ntiles, 1);
+  if (t >= ntiles) return;  // the whole block leaves: no barrier is reached
+  const unsigned lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const unsigned tk = (unsigned)(t / ((long)nbi * nbj)), tij = (unsigned)(t - (long)tk * nbi * nbj);
+  const unsigned tj = tij / nbi, ti = tij - tj * nbi;
+  const unsigned l = threadIdx.x & 255, lj = l / tw, li = l - lj * tw;
+  const int i = (int)(tw * ti + li) + 1, j = (int)(tr * tj + lj) + 1, k = (int)(kTrajLevels * tk + wv / 4) + P.k00;
+  const bool valid = lj < tr && i <= P.ni && j <= P.nj && k <= P.nk;
+  S px = (S)0, py = (S)0, pz = (S)0;
+  S ua = (S)0, va = (S)0, wa = (S)0;
+  if (valid) {
+    const long p = p3_idx(P, i, j, k);
+    const long aw = (long)(i - 1) + (long)P.ni * ((j - 1) + (long)P.nj * (k - 1));
+    px = pxyzm[p]; py = pxyzm[p + 1]; pz = pxyzm[p + 2];
+    ua = uarr[aw]; va = varr[aw]; wa = warr[aw];
+  }
   const S* f3 = uvw_d + 3L * ((long)(1 - P.lminx) + (long)P.nit * (1 - P.lminy));
+  // box in LDS: local columns [bx0, bx1], rows [by0, by1], planes [bz0, bz1]; empty at first
+  unsigned boxes = 0;
+  int bx0 = kFar, bx1 = -kFar, by0 = kFar, by1 = -kFar, bz0 = kFar, bz1 = -kFar;
   for (int it = 0; it < niter; it++) {
     Index x;
-    double c[20], w3[3];
-    if (index_step((double)px, (double)py, (double)pz, lv, &x)) {
-      weights_ref(x, lv, c);
-      tricub3_ref<S>(f3 + 3 * x.off, c, 3L * lv.ni, 3L * lv.nij, x.zlinear, w3);
-    } else {
-      w3[0] = w3[1] = w3[2] = __builtin_nan("");
+    const bool ok = valid && index_step((double)px, (double)py, (double)pz, lv, &x);
+    const int pz1 = x.pz + (x.zlinear ? 1 : 3);
+    const bool out = ok && (x.ix - 1 < bx0 || x.ix + 2 > bx1 || x.iy - 1 < by0 || x.iy + 2 > by1 || x.pz < bz0 || pz1 > bz1);
+    // does any lane of the block need a new box?  (Word it % 3 tells; the barrier also says
+    // that every wave is done with the old one.)
+    if (__ballot(out) != 0 && lane == 0) moved[it % 3] = 1;
+    if (threadIdx.x == 0) moved[(it + 1) % 3] = 0;
+    __syncthreads();
+    bool staged = true;
+    if (__builtin_amdgcn_readfirstlane(moved[it % 3])) {
+      int ext[6] = {ok ? x.ix - 1 : kFar, ok ? -(x.ix + 2) : kFar, ok ? x.iy - 1 : kFar, ok ? -(x.iy + 2) : kFar,
+                    ok ? x.pz : kFar, ok ? -pz1 : kFar};
+      tile_min6(ext, red, boxes++);
+      const int x0 = ext[0], x1 = -ext[1], y0 = ext[2], y1 = -ext[3], z0 = ext[4], z1 = -ext[5];
+      const int mx0 = max(x0 - 1, lv.ilo), mx1 = min(x1 + 1, lv.ihi), my0 = max(y0 - 1, lv.jlo),
+                my1 = min(y1 + 1, lv.jhi), mz0 = max(z0 - 1, 0), mz1 = min(z1 + 1, lv.nk - 1);
+      const int cols = kWindPitch / 3;
+      const bool roomy = (my1 - my0 + 1) * (mz1 - mz0 + 1) <= kTrajRows && mx1 - mx0 + 1 <= cols;
+      if (roomy) { bx0 = mx0; bx1 = mx1; by0 = my0; by1 = my1; bz0 = mz0; bz1 = mz1; }
+      else { bx0 = x0; bx1 = x1; by0 = y0; by1 = y1; bz0 = z0; bz1 = z1; }
+      const int nyb = by1 - by0 + 1, nzb = bz1 - bz0 + 1;
+      const long n3 = 3L * lv.ni * (long)sizeof(S), nij3 = 3L * lv.nij * (long)sizeof(S);  // bytes of a row, of a plane
+      staged = bx1 - bx0 < cols && (long)nyb * nzb <= kTrajRows && n3 * nyb + nij3 * nzb < 0x7fff0000L;
+      if (staged) {
+        const char* b0 = (const char*)(f3 + 3 * ((bx0 - 1) + (long)(by0 - 1) * lv.ni + (long)bz0 * lv.nij));
+        const long left = (const char*)(uvw_d + 3L * P.nij * P.nk) + 16 - b0;  // (the array ends in 16 spare bytes)
+        const __amdgpu_buffer_rsrc_t rs = field_rsrc(b0, (unsigned)min(left, 0x7fff0000L));
+        const int quads = (3 * (bx1 - bx0 + 1) * (int)sizeof(S) + 15) / 16;
+        constexpr int kI = kWindPitch * (int)sizeof(S) / 1024;  // DMA instructions per row
+        for (int r = wv; r < nyb * nzb; r += kTrajWaves) {
+          const int zz = r / nyb, yy = r - zz * nyb;
+          const int off = yy * (int)n3 + zz * (int)nij3;
+#pragma unroll
+          for (int h = 0; h < kI; h++) {
+            const int q = 64 * h + (int)lane;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                rs, (__attribute__((address_space(3))) void*)(box + r * kWindPitch + h * (1024 / (int)sizeof(S))), 16,
+                q < quads ? off + 16 * q : 0x7fff0000, 0, 0, 0);
+          }
+        }
+        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+        __syncthreads();
+      } else {
+        bx0 = kFar;  // nothing in LDS
+      }
     }
-    ud = (S)w3[0]; vd = (S)w3[1]; wd = (S)w3[2];
-    xm = (double)(i + P.i0g - 1) - (dtD * (double)ud + dtA * ua) * P.inv_hx;
-    ym = (double)(j + P.j0g - 1) - (dtD * (double)vd + dtA * va) * P.inv_hy;
-    double pos = P.zm[k] - dtzD * (double)wd - dtzA * wa;
-    double zmv = fmin(fmax(pos, P.zmin), P.zmax);
-    int kk = d_level_search(P.zm, P.search_m, P.pnz_m, P.ovdzm, P.sig, P.nk, zmv);
-    int kk1 = min(P.nk + 1, max(0, kk));
-    int nb = max(min(kk1, P.nk - 1), 1);
-    pzm = (zmv - P.zm[nb]) * P.odelz_m[nb] + (double)nb;
-    px = (S)clampd(xm, P.iminposx, P.imaxposx);
-    py = (S)clampd(ym, P.iminposy, P.imaxposy);
-    pz = (S)pzm;
-  }
-  pxyzm[p] = px; pxyzm[p + 1] = py; pxyzm[p + 2] = pz;
-  uvw_dep[p] = ud; uvw_dep[p + 1] = vd; uvw_dep[p + 2] = wd;
-  if (niter > 0) {
-    wpxyz[wp_idx(P, i, j, k, 1)] = xm;
-    wpxyz[wp_idx(P, i, j, k, 2)] = ym;
-    wpxyz[wp_idx(P, i, j, k, 3)] = pzm;
+    double w3[3] = {__builtin_nan(""), __builtin_nan(""), __builtin_nan("")};
+    if (ok) {
+      double c[20];
+      weights_ref(x, lv, c);
+      if (staged) {
+        const int nyb = by1 - by0 + 1;
+        const int b = ((x.iy - 1 - by0) + nyb * (x.pz - bz0)) * kWindPitch + 3 * (x.ix - 1 - bx0);
+        const int o1 = x.zlinear ? 0 : nyb * kWindPitch, o2 = o1 + nyb * kWindPitch, o3 = o2 + o1;
+        tricub3_steps<S>([&](int h, int r, int z, S* v) {
+          int e = b + r * kWindPitch + (z == 0 ? 0 : z == 1 ? o1 : z == 2 ? o2 : o3);
+          asm("" : "+v"(e));  // one address, the six values at immediate offsets
+#pragma unroll
+          for (int q = 0; q < 6; q++) v[q] = box[e + 6 * h + q];
+        }, c, w3);
+      } else {
+        const long o1 = x.zlinear ? 0 : 3L * lv.nij, o2 = o1 + 3L * lv.nij, o3 = o2 + o1;
+        tricub3_steps<S>([&](int h, int r, int z, S* v) {
+          const S* s = f3 + 3 * x.off + 3L * r * lv.ni + (z == 0 ? 0 : z == 1 ? o1 : z == 2 ? o2 : o3) + 6 * h;
+#pragma unroll
+          for (int q = 0; q < 6; q++) v[q] = s[q];
+        }, c, w3);
+      }
+    }
+    if (valid) {
+      // (opaque in the loop: what follows from them is formed here rather than held through it)
+      int i1 = i, j1 = j;
+      asm volatile("" : "+v"(i1), "+v"(j1), "+v"(ua), "+v"(va), "+v"(wa));
+      const long p = p3_idx(P, i1, j1, k);
+      const S ud = (S)w3[0], vd = (S)w3[1], wd = (S)w3[2];
+      const double xm = (double)(i1 + P.i0g - 1) - (dtD * (double)ud + dtA * (double)ua) * P.inv_hx;
+      const double ym = (double)(j1 + P.j0g - 1) - (dtD * (double)vd + dtA * (double)va) * P.inv_hy;
+      double pos = P.zm[k] - dtzD * (double)wd - dtzA * (double)wa;
+      double zmv = fmin(fmax(pos, P.zmin), P.zmax);
+      int kk = d_level_search(P.zm, P.search_m, P.pnz_m, P.ovdzm, P.sig, P.nk, zmv);
+      int kk1 = min(P.nk + 1, max(0, kk));
+      int nb = max(min(kk1, P.nk - 1), 1);
+      const double pzm = (zmv - P.zm[nb]) * P.odelz_m[nb] + (double)nb;
+      px = (S)clampd(xm, P.iminposx, P.imaxposx);
+      py = (S)clampd(ym, P.iminposy, P.imaxposy);
+      pz = (S)pzm;
+      if (it == niter - 1) {
+        pxyzm[p] = px; pxyzm[p + 1] = py; pxyzm[p + 2] = pz;
+        uvw_dep[p] = ud; uvw_dep[p + 1] = vd; uvw_dep[p + 2] = wd;
+        wpxyz[wp_idx(P, i1, j1, k, 1)] = xm;
+        wpxyz[wp_idx(P, i1, j1, k, 2)] = ym;
+        wpxyz[wp_idx(P, i1, j1, k, 3)] = pzm;
+      }
+    }
   }
 }
 
@@ -368,6 +501,19 @@ void free_ctx(adz_ctx* c) {
   delete c;
 }
 
+// Tile of k_traject: of the widths that split the rows into equal parts of 32 to 64 points, with
+// as many rows as 256 lanes hold (at most 8, for the box), the one that leaves the fewest lanes
+// without a point.  (65 x 103 x 49, cold: 109 us per lane, 176 with tiles of 64 x 4 and a
+// whole tile for the last column, 112 with 33 x 7; 200 x 150 x 60, cold: 466 and 425.)
+void traj_tile(int ni, int nj, unsigned* tw, unsigned* tr) {
+  long best = -1;
+  for (int nt = (ni + 63) / 64; nt == (ni + 63) / 64 || (ni + nt - 1) / nt >= 32; nt++) {
+    const int w = (ni + nt - 1) / nt, r = std::min(8, 256 / w);
+    const long blocks = (long)((ni + w - 1) / w) * ((nj + r - 1) / r);
+    if (best < 0 || blocks < best) { best = blocks; *tw = w; *tr = r; }
+  }
+}
+
 template <class S>
 int run_traject(adz_ctx* c, double dt, int advec, double bA_m, double bA, const float* uu, const float* vv,
                 const float* ww, const float* ut0, const float* vt0, const float* zdt0, hipStream_t st) {
@@ -382,10 +528,12 @@ int run_traject(adz_ctx* c, double dt, int advec, double bA_m, double bA, const 
   hipLaunchKernelGGL(k_prep_uvwd<S>, dim3(nb(next)), dim3(256), 0, st, (S*)c->uvw_d, uu, vv, ww, P);
   S* arr = (S*)c->warr;
   hipLaunchKernelGGL(k_prep_arr<S>, dim3(nb(nint)), dim3(256), 0, st, arr, arr + nint, arr + 2 * nint, ut0, vt0, zdt0, P);
-  long npts = (long)P.ni * P.nj * (P.nk - P.k00 + 1);
-  hipLaunchKernelGGL(k_traject<S>, dim3(nb(npts)), dim3(256), 0, st, (S*)c->pxyzm, c->wpxyz, (S*)c->uvw_dep,
+  unsigned tw, tr;
+  traj_tile(P.ni, P.nj, &tw, &tr);
+  const long tiles = (long)((P.ni + tw - 1) / tw) * ((P.nj + tr - 1) / tr) * ((P.nk - P.k00 + kTrajLevels) / kTrajLevels);
+  hipLaunchKernelGGL(k_traject<S>, tile_grid(tiles), dim3(64 * kTrajWaves), 0, st, (S*)c->pxyzm, c->wpxyz, (S*)c->uvw_dep,
                      (const S*)c->uvw_d, arr, arr + nint, arr + 2 * nint, c->zq->dev, P, c->niter, dtA, dtD, dtzA,
-                     dtzD);
+                     dtzD, tw, tr);
   hipLaunchKernelGGL(k_copy_box<S>, dim3(nb(c->n_pm / 3)), dim3(256), 0, st, (S*)c->pm, (const S*)c->pxyzm, P, 0);
   c->niter = c->itraj;  // adz_traject.F90:120
   hipLaunchKernelGGL(k_interp_uv<S>, dim3(nb(c->n_pmu / 3)), dim3(256), 0, st, (S*)c->pmu, c->wpxyz, P, 0);
@@ -578,7 +726,7 @@ int adz_set(const adz_grid* g, int pos_dtype, int itraj, adz_ctx** out) {
   c->n_pt = 3L * (P.in - P.i0 + 1) * (P.jn - P.j0 + 1) * (nk - P.k0t + 1);
   c->n_pb = 3L * (P.inb - P.i0b + 1) * (P.jnb - P.j0b + 1) * nk;
   struct { void** p; size_t b; } al[] = {
-      {&c->uvw_d, c->n_uvw_d * sz}, {&c->warr, c->n_arr * sz}, {&c->uvw_dep, c->n_p3 * sz},
+      {&c->uvw_d, c->n_uvw_d * sz + 16}, {&c->warr, c->n_arr * sz}, {&c->uvw_dep, c->n_p3 * sz},
       {&c->pxyzm, c->n_p3 * sz},    {(void**)&c->wpxyz, (size_t)c->n_wp * 8}, {&c->pm, c->n_pm * sz},
       {&c->pmu, c->n_pmu * sz},     {&c->pmv, c->n_pmv * sz}, {&c->pt, c->n_pt * sz}, {&c->pb, c->n_pb * sz}};
   for (auto& a : al) {
