@@ -79,31 +79,35 @@ __device__ __forceinline__ long box_idx(int i0, int in, int j0, int jn, int k0, 
 }
 
 // ---------------------------------------------------------------- adz_prepareWinds
+// One level of the tile per row of the grid (no division by a level's points).
+constexpr int kMaxGridY = 65535;
+
 // adz_prepareWinds.F90:37-47 and :62-101 on the extended domain.
 template <class S>
 __global__ void k_prep_uvwd(S* __restrict__ uvw_d, const float* __restrict__ uu, const float* __restrict__ vv,
                             const float* __restrict__ ww, TrajParams P) {
-  long q = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  long n = (long)P.nij * P.nk;
-  if (q >= n) return;
-  int k = (int)(q / P.nij) + 1;
-  int j = (int)((q % P.nij) / P.nit) + P.lminy;
-  const double ir = P.inv_rayt;
-  uvw_d[3 * q + 0] = (S)(ir * (double)uu[q] * P.cy[j - P.lminy]);
-  uvw_d[3 * q + 1] = (S)(ir * (double)vv[q]);
-  double w;
-  const int nk = P.nk;
-  if (k == 1) w = P.vw5 * (double)ww[q];
-  else if (k == nk) w = P.vw6 * (double)ww[q - P.nij];
-  else {
-    const double* vw = P.vw;
-    double wx = (k >= 3) ? vw[k] : 0.0;
-    int km2 = max(1, k - 2);
-    long base = q - (long)(k - 1) * P.nij;
-    w = wx * (double)ww[base + (long)(km2 - 1) * P.nij] + vw[(nk + 1) + k] * (double)ww[q - P.nij] +
-        vw[2 * (nk + 1) + k] * (double)ww[q] + vw[3 * (nk + 1) + k] * (double)ww[q + P.nij];
+  const unsigned h = blockIdx.x * blockDim.x + threadIdx.x;
+  if (h >= (unsigned)P.nij) return;
+  const int j = (int)(h / (unsigned)P.nit) + P.lminy;
+  for (int k = (int)blockIdx.y + 1; k <= P.nk; k += (int)gridDim.y) {
+    const long q = h + (long)P.nij * (k - 1);
+    const double ir = P.inv_rayt;
+    uvw_d[3 * q + 0] = (S)(ir * (double)uu[q] * P.cy[j - P.lminy]);
+    uvw_d[3 * q + 1] = (S)(ir * (double)vv[q]);
+    double w;
+    const int nk = P.nk;
+    if (k == 1) w = P.vw5 * (double)ww[q];
+    else if (k == nk) w = P.vw6 * (double)ww[q - P.nij];
+    else {
+      const double* vw = P.vw;
+      double wx = (k >= 3) ? vw[k] : 0.0;
+      int km2 = max(1, k - 2);
+      long base = q - (long)(k - 1) * P.nij;
+      w = wx * (double)ww[base + (long)(km2 - 1) * P.nij] + vw[(nk + 1) + k] * (double)ww[q - P.nij] +
+          vw[2 * (nk + 1) + k] * (double)ww[q] + vw[3 * (nk + 1) + k] * (double)ww[q + P.nij];
+    }
+    uvw_d[3 * q + 2] = (S)w;
   }
-  uvw_d[3 * q + 2] = (S)w;
 }
 
 // adz_prepareWinds.F90:48-61 and :69-86 on the interior: arrival winds.
@@ -111,32 +115,33 @@ template <class S>
 __global__ void k_prep_arr(S* __restrict__ uarr, S* __restrict__ varr, S* __restrict__ warr,
                            const float* __restrict__ ut0, const float* __restrict__ vt0, const float* __restrict__ zdt0,
                            TrajParams P) {
-  long a = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  long nxy = (long)P.ni * P.nj;
-  if (a >= nxy * P.nk) return;
-  int k = (int)(a / nxy) + 1;
-  int j = (int)((a % nxy) / P.ni) + 1;
-  int i = (int)(a % P.ni) + 1;
-  const double alpha1 = -1.0 / 16.0, alpha2 = 9.0 / 16.0, ir = P.inv_rayt;
-  S u1 = (S)ut0[ext_idx(P, i - 2, j, k)] + (S)ut0[ext_idx(P, i + 1, j, k)];
-  S u2 = (S)ut0[ext_idx(P, i, j, k)] + (S)ut0[ext_idx(P, i - 1, j, k)];
-  uarr[a] = (S)((((double)u1 * alpha1 + (double)u2 * alpha2) * ir) * P.cy[j - P.lminy]);
-  S v1 = (S)vt0[ext_idx(P, i, j - 2, k)] + (S)vt0[ext_idx(P, i, j + 1, k)];
-  S v2 = (S)vt0[ext_idx(P, i, j, k)] + (S)vt0[ext_idx(P, i, j - 1, k)];
-  varr[a] = (S)(((double)v1 * alpha1 + (double)v2 * alpha2) * ir);
-  const int nk = P.nk;
-  double w;
-  if (k == 1) w = P.vw5 * (double)zdt0[ext_idx(P, i, j, 1)];
-  else if (k == nk) w = P.vw6 * (double)zdt0[ext_idx(P, i, j, nk - 1)];
-  else {
-    const double* vw = P.vw;
-    double wx = (k >= 3) ? vw[k] : 0.0;
-    int km2 = max(1, k - 2);
-    w = wx * (double)zdt0[ext_idx(P, i, j, km2)] + vw[(nk + 1) + k] * (double)zdt0[ext_idx(P, i, j, k - 1)] +
-        vw[2 * (nk + 1) + k] * (double)zdt0[ext_idx(P, i, j, k)] +
-        vw[3 * (nk + 1) + k] * (double)zdt0[ext_idx(P, i, j, k + 1)];
+  const unsigned h = blockIdx.x * blockDim.x + threadIdx.x, nxy = (unsigned)P.ni * (unsigned)P.nj;
+  if (h >= nxy) return;
+  const unsigned jq = h / (unsigned)P.ni;
+  const int j = (int)jq + 1, i = (int)(h - jq * (unsigned)P.ni) + 1;
+  for (int k = (int)blockIdx.y + 1; k <= P.nk; k += (int)gridDim.y) {
+    const long a = h + (long)nxy * (k - 1);
+    const double alpha1 = -1.0 / 16.0, alpha2 = 9.0 / 16.0, ir = P.inv_rayt;
+    S u1 = (S)ut0[ext_idx(P, i - 2, j, k)] + (S)ut0[ext_idx(P, i + 1, j, k)];
+    S u2 = (S)ut0[ext_idx(P, i, j, k)] + (S)ut0[ext_idx(P, i - 1, j, k)];
+    uarr[a] = (S)((((double)u1 * alpha1 + (double)u2 * alpha2) * ir) * P.cy[j - P.lminy]);
+    S v1 = (S)vt0[ext_idx(P, i, j - 2, k)] + (S)vt0[ext_idx(P, i, j + 1, k)];
+    S v2 = (S)vt0[ext_idx(P, i, j, k)] + (S)vt0[ext_idx(P, i, j - 1, k)];
+    varr[a] = (S)(((double)v1 * alpha1 + (double)v2 * alpha2) * ir);
+    const int nk = P.nk;
+    double w;
+    if (k == 1) w = P.vw5 * (double)zdt0[ext_idx(P, i, j, 1)];
+    else if (k == nk) w = P.vw6 * (double)zdt0[ext_idx(P, i, j, nk - 1)];
+    else {
+      const double* vw = P.vw;
+      double wx = (k >= 3) ? vw[k] : 0.0;
+      int km2 = max(1, k - 2);
+      w = wx * (double)zdt0[ext_idx(P, i, j, km2)] + vw[(nk + 1) + k] * (double)zdt0[ext_idx(P, i, j, k - 1)] +
+          vw[2 * (nk + 1) + k] * (double)zdt0[ext_idx(P, i, j, k)] +
+          vw[3 * (nk + 1) + k] * (double)zdt0[ext_idx(P, i, j, k + 1)];
+    }
+    warr[a] = (S)w;
   }
-  warr[a] = (S)w;
 }
 
 // ---------------------------------------------------------------- adz_traject
@@ -196,8 +201,8 @@ __device__ __forceinline__ void tricub3_steps(Read read, const double* c, double
 
 template <class S>
 __global__ __launch_bounds__(64 * kTrajWaves, sizeof(S) == 4 ? 4 : 2) void k_traject(
-    S* __restrict__ pxyzm, double* __restrict__ wpxyz, S* __restrict__ uvw_dep, const S* __restrict__ uvw_d,
-    const S* __restrict__ uarr, const S* __restrict__ varr, const S* __restrict__ warr, ZtabDev lv, TrajParams P,
+    S* __restrict__ pxyzm, double* __restrict__ wpxyz, S* __restrict__ uvw_dep, S* __restrict__ pm,
+    const S* __restrict__ uvw_d, const S* __restrict__ uarr, const S* __restrict__ varr, const S* __restrict__ warr, ZtabDev lv, TrajParams P,
     int niter, double dtA, double dtD, double dtzA, double dtzD, unsigned tw, unsigned tr) {
   __shared__ __attribute__((aligned(16))) S box[kTrajRows * kWindPitch];
   __shared__ int red[18], moved[3];
@@ -317,6 +322,10 @@ __global__ __launch_bounds__(64 * kTrajWaves, sizeof(S) == 4 ? 4 : 2) void k_tra
       if (it == niter - 1) {
         pxyzm[p] = px; pxyzm[p + 1] = py; pxyzm[p + 2] = pz;
         uvw_dep[p] = ud; uvw_dep[p + 1] = vd; uvw_dep[p + 2] = wd;
+        if (i1 >= P.i0 && i1 <= P.in && j1 >= P.j0 && j1 <= P.jn && k >= P.k0) {  // Adz_pm, adz_traject.F90:112-116
+          const long m = box_idx(P.i0, P.in, P.j0, P.jn, P.k0, i1, j1, k);
+          pm[m] = px; pm[m + 1] = py; pm[m + 2] = pz;
+        }
         wpxyz[wp_idx(P, i1, j1, k, 1)] = xm;
         wpxyz[wp_idx(P, i1, j1, k, 2)] = ym;
         wpxyz[wp_idx(P, i1, j1, k, 3)] = pzm;
@@ -344,101 +353,92 @@ __global__ void k_inittraj(S* __restrict__ pxyzm, double* __restrict__ wpxyz, Tr
 }
 
 // ---------------------------------------------------------------- adz_interp_traj
-// u- and v-grid positions, adz_interp_traj.F90:45-78 (which = 0: u, 1: v)
+// Positions of the u and v grids (Adz_pmu, Adz_pmv: adz_interp_traj.F90:45-78) and of the
+// thermodynamic levels (Adz_pb: :80-174, and its part Adz_pt: :176-181) from the FP64 history
+// W, in one pass over it.  A lane takes kc consecutive levels of one column, the four levels of
+// the vertical stencil passing through its registers; a block's 64 columns by 4 rows share the
+// horizontal stencils in the first-level cache.
+//
+// What bounds it: memory, 88 bytes of history, winds and positions per point at 2.8 TB/s, in
+// nine streams.  1024 x 512 x 84: 1.22 ms in one kernel (1.26 with an eighth of the tiles per
+// XCD; 4 or 16 levels per lane 1.24 and 1.35); as five (pmu, pmv, pb and the copies into pt
+// and into pm, now stored by k_traject), each reading the history again, 1.91 ms.
 template <class S>
-__global__ void k_interp_uv(S* __restrict__ out, const double* __restrict__ W, TrajParams P, int which) {
-  long a = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  int i0 = which == 0 ? P.i0u : P.i0, in = which == 0 ? P.inu : P.in;
-  int j0 = which == 0 ? P.j0 : P.j0v, jn = which == 0 ? P.jn : P.jnv;
-  long nx = in - i0 + 1, ny = jn - j0 + 1;
-  if (nx <= 0 || ny <= 0 || a >= nx * ny * (P.nk - P.k0 + 1)) return;
-  int k = (int)(a / (nx * ny)) + P.k0;
-  int j = (int)((a % (nx * ny)) / nx) + j0;
-  int i = (int)(a % nx) + i0;
-  const double aa = -0.0625, bb = 0.5625;
-  int di = which == 0 ? 1 : 0, dj = which == 0 ? 0 : 1;
-  double r[3];
-  for (int c = 1; c <= 3; c++) {
-    double wm1 = W[wp_idx(P, i - di, j - dj, k, c)], w0 = W[wp_idx(P, i, j, k, c)];
-    double w1 = W[wp_idx(P, i + di, j + dj, k, c)], w2 = W[wp_idx(P, i + 2 * di, j + 2 * dj, k, c)];
-    r[c - 1] = aa * (wm1 + w2) + bb * (w0 + w1);
-  }
-  if (which == 0) r[0] = r[0] - 0.5; else r[1] = r[1] - 0.5;
-  long q = box_idx(i0, in, j0, jn, P.k0, i, j, k);
-  out[q] = (S)clampd(r[0], P.iminposx, P.imaxposx);
-  out[q + 1] = (S)clampd(r[1], P.iminposy, P.imaxposy);
-  out[q + 2] = (S)clampd(r[2], 0.0, (double)(P.nk + 1));
-}
-
-// thermodynamic-level positions Adz_pb, adz_interp_traj.F90:80-174
-template <class S>
-__global__ void k_interp_b(S* __restrict__ pb, const double* __restrict__ W, const S* __restrict__ uvw_dep,
-                           const float* __restrict__ zdt0, TrajParams P, double dtzD, double dtzA) {
-  long a = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  long nx = P.inb - P.i0b + 1, ny = P.jnb - P.j0b + 1;
-  if (nx <= 0 || ny <= 0 || a >= nx * ny * P.nk) return;
-  int k = (int)(a / (nx * ny)) + 1;
-  int j = (int)((a % (nx * ny)) / nx) + P.j0b;
-  int i = (int)(a % nx) + P.i0b;
-  const int nk = P.nk;
-  const double half = 0.5;
-  int kstart = max(P.k00i, 2);
-  long q = box_idx(P.i0b, P.inb, P.j0b, P.jnb, 1, i, j, k);
-  auto UD3 = [&](int kk) { return (double)uvw_dep[p3_idx(P, i, j, kk) + 2]; };
-  auto Z0 = [&](int kk) { return (double)zdt0[ext_idx(P, i, j, kk)]; };
+__global__ __launch_bounds__(256) void k_sets(S* __restrict__ pmu, S* __restrict__ pmv, S* __restrict__ pb,
+                                              S* __restrict__ pt, const double* __restrict__ W,
+                                              const S* __restrict__ uvw_dep, const float* __restrict__ zdt0,
+                                              TrajParams P, double dtzD, double dtzA, int kc) {
+  const unsigned nbi = (P.ni + 63) / 64, nbj = (P.nj + 3) / 4, nbk = (P.nk + kc - 1) / kc;
+  const long ntiles = (long)nbi * nbj * nbk, t = tile_of_block(ntiles, 0);
+  if (t >= ntiles) return;
+  const unsigned tk = (unsigned)(t / ((long)nbi * nbj)), tij = (unsigned)(t - (long)tk * nbi * nbj), tj = tij / nbi;
+  const int i = (int)(64 * (tij - tj * nbi) + (threadIdx.x & 63)) + 1, j = (int)(4 * tj + (threadIdx.x >> 6)) + 1;
+  if (i > P.ni || j > P.nj) return;
+  const int nk = P.nk, k1 = (int)tk * kc + 1, k2 = min(nk, k1 + kc - 1), kstart = max(P.k00i, 2);
+  const bool onu = i >= P.i0u && i <= P.inu && j >= P.j0 && j <= P.jn;
+  const bool onv = i >= P.i0 && i <= P.in && j >= P.j0v && j <= P.jnv;
+  const bool onb = i >= P.i0b && i <= P.inb && j >= P.j0b && j <= P.jnb;
+  const bool ont = i >= P.i0 && i <= P.in && j >= P.j0 && j <= P.jn;
+  const double aa = -0.0625, bb = 0.5625, half = 0.5;
   const double* vw = P.vw;
-  if (k >= kstart && k <= nk - 2) {
-    double v1 = vw[4 * (nk + 1) + k], v2 = vw[5 * (nk + 1) + k], v3 = vw[6 * (nk + 1) + k], v4 = vw[7 * (nk + 1) + k];
-    double xt = v1 * W[wp_idx(P, i, j, k - 1, 1)] + v2 * W[wp_idx(P, i, j, k, 1)] + v3 * W[wp_idx(P, i, j, k + 1, 1)] +
-                v4 * W[wp_idx(P, i, j, k + 2, 1)];
-    double yt = v1 * W[wp_idx(P, i, j, k - 1, 2)] + v2 * W[wp_idx(P, i, j, k, 2)] + v3 * W[wp_idx(P, i, j, k + 1, 2)] +
-                v4 * W[wp_idx(P, i, j, k + 2, 2)];
-    double wdt = v1 * UD3(k - 1) + v2 * UD3(k) + v3 * UD3(k + 1) + v4 * UD3(k + 2);
-    double zt = P.zt[k] - dtzD * wdt - dtzA * Z0(k);
-    pb[q] = (S)clampd(xt, P.iminposx, P.imaxposx);
-    pb[q + 1] = (S)clampd(yt, P.iminposy, P.imaxposy);
-    pb[q + 2] = (S)d_zindx(P, zt);
-  } else if (k == nk - 1) {
-    double xt = (W[wp_idx(P, i, j, k, 1)] + W[wp_idx(P, i, j, k + 1, 1)]) * half;
-    double yt = (W[wp_idx(P, i, j, k, 2)] + W[wp_idx(P, i, j, k + 1, 2)]) * half;
-    double wdt = (UD3(k) + UD3(k + 1)) * half;
-    double zt = P.zt[k] - dtzD * wdt - dtzA * Z0(k);
-    pb[q] = (S)clampd(xt, P.iminposx, P.imaxposx);
-    pb[q + 1] = (S)clampd(yt, P.iminposy, P.imaxposy);
-    pb[q + 2] = (S)d_zindx(P, zt);
-  } else if (k == nk) {
-    double xt = P.wp_nk * W[wp_idx(P, i, j, k, 1)] + P.wm_nk * W[wp_idx(P, i, j, k - 1, 1)];
-    double yt = P.wp_nk * W[wp_idx(P, i, j, k, 2)] + P.wm_nk * W[wp_idx(P, i, j, k - 1, 2)];
-    pb[q] = (S)clampd(xt, P.iminposx, P.imaxposx);
-    pb[q + 1] = (S)clampd(yt, P.iminposy, P.imaxposy);
-    double wdt = (UD3(k - 1) + UD3(k)) * half;
-    double zt = P.zt[k] - P.ww_star * (dtzD * wdt + dtzA * Z0(k - 1));
-    pb[q + 2] = (S)d_zindx(P, zt);
-  } else if (k == 1 && P.k00i == 1) {
-    double xt = (W[wp_idx(P, i, j, 1, 1)] + W[wp_idx(P, i, j, 2, 1)]) * half;
-    double yt = (W[wp_idx(P, i, j, 1, 2)] + W[wp_idx(P, i, j, 2, 2)]) * half;
-    double wdt = (UD3(1) + UD3(2)) * half;
-    double zt = P.zt[1] - dtzD * wdt - dtzA * Z0(1);
-    pb[q] = (S)clampd(xt, P.iminposx, P.imaxposx);
-    pb[q + 1] = (S)clampd(yt, P.iminposy, P.imaxposy);
-    pb[q + 2] = (S)d_zindx(P, zt);
+  // x, y and vertical wind of levels k-1, k, k+1 and k+2 (levels outside [k0m, nk] are not used)
+  double x[4], y[4], d[4];
+  auto level = [&](int q, int k) {
+    k = min(max(k, P.k0m), nk);
+    x[q] = W[wp_idx(P, i, j, k, 1)];
+    y[q] = W[wp_idx(P, i, j, k, 2)];
+    d[q] = (double)uvw_dep[p3_idx(P, i, j, k) + 2];
+  };
+  level(1, k1 - 1); level(2, k1); level(3, k1 + 1);
+  for (int k = k1; k <= k2; k++) {
+#pragma unroll
+    for (int q = 0; q < 3; q++) { x[q] = x[q + 1]; y[q] = y[q + 1]; d[q] = d[q + 1]; }
+    level(3, k + 2);
+    const double z0 = W[wp_idx(P, i, j, k, 3)];
+    auto between = [&](double w0, int c, int di, int dj) {  // half a point back, along i or j
+      const double wm1 = W[wp_idx(P, i - di, j - dj, k, c)], w1 = W[wp_idx(P, i + di, j + dj, k, c)];
+      const double w2 = W[wp_idx(P, i + 2 * di, j + 2 * dj, k, c)];
+      return aa * (wm1 + w2) + bb * (w0 + w1);
+    };
+    auto put = [&](S* out, long q, double r0, double r1, double r2) {
+      out[q] = (S)clampd(r0, P.iminposx, P.imaxposx);
+      out[q + 1] = (S)clampd(r1, P.iminposy, P.imaxposy);
+      out[q + 2] = (S)clampd(r2, 0.0, (double)(nk + 1));
+    };
+    if (onu && k >= P.k0)
+      put(pmu, box_idx(P.i0u, P.inu, P.j0, P.jn, P.k0, i, j, k), between(x[1], 1, 1, 0) - 0.5, between(y[1], 2, 1, 0),
+          between(z0, 3, 1, 0));
+    if (onv && k >= P.k0)
+      put(pmv, box_idx(P.i0, P.in, P.j0v, P.jnv, P.k0, i, j, k), between(x[1], 1, 0, 1), between(y[1], 2, 0, 1) - 0.5,
+          between(z0, 3, 0, 1));
+    if (!onb || (k == 1 ? P.k00i != 1 : k < kstart)) continue;
+    double xt, yt, zt;
+    if (k >= 2 && k <= nk - 2) {
+      double v1 = vw[4 * (nk + 1) + k], v2 = vw[5 * (nk + 1) + k], v3 = vw[6 * (nk + 1) + k], v4 = vw[7 * (nk + 1) + k];
+      xt = v1 * x[0] + v2 * x[1] + v3 * x[2] + v4 * x[3];
+      yt = v1 * y[0] + v2 * y[1] + v3 * y[2] + v4 * y[3];
+      double wdt = v1 * d[0] + v2 * d[1] + v3 * d[2] + v4 * d[3];
+      zt = P.zt[k] - dtzD * wdt - dtzA * (double)zdt0[ext_idx(P, i, j, k)];
+    } else if (k < nk) {  // 1 and nk - 1
+      xt = (x[1] + x[2]) * half;
+      yt = (y[1] + y[2]) * half;
+      double wdt = (d[1] + d[2]) * half;
+      zt = P.zt[k] - dtzD * wdt - dtzA * (double)zdt0[ext_idx(P, i, j, k)];
+    } else {
+      xt = P.wp_nk * x[1] + P.wm_nk * x[0];
+      yt = P.wp_nk * y[1] + P.wm_nk * y[0];
+      double wdt = (d[0] + d[1]) * half;
+      zt = P.zt[k] - P.ww_star * (dtzD * wdt + dtzA * (double)zdt0[ext_idx(P, i, j, k - 1)]);
+    }
+    const S sx = (S)clampd(xt, P.iminposx, P.imaxposx), sy = (S)clampd(yt, P.iminposy, P.imaxposy);
+    const S sz = (S)d_zindx(P, zt);
+    const long q = box_idx(P.i0b, P.inb, P.j0b, P.jnb, 1, i, j, k);
+    pb[q] = sx; pb[q + 1] = sy; pb[q + 2] = sz;
+    if (ont && k >= P.k0t) {
+      const long m = box_idx(P.i0, P.in, P.j0, P.jn, P.k0t, i, j, k);
+      pt[m] = sx; pt[m + 1] = sy; pt[m + 2] = sz;
+    }
   }
-}
-
-// Adz_pm = Adz_pxyzm and Adz_pt = Adz_pb on [i0:in]x[j0:jn] (adz_traject.F90:112-116,
-// adz_interp_traj.F90:176-181); which = 0: pm, 1: pt
-template <class S>
-__global__ void k_copy_box(S* __restrict__ out, const S* __restrict__ src, TrajParams P, int which) {
-  long a = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  long nx = P.in - P.i0 + 1, ny = P.jn - P.j0 + 1;
-  int kb = which == 0 ? P.k0 : P.k0t;
-  if (nx <= 0 || ny <= 0 || a >= nx * ny * (P.nk - kb + 1)) return;
-  int k = (int)(a / (nx * ny)) + kb;
-  int j = (int)((a % (nx * ny)) / nx) + P.j0;
-  int i = (int)(a % nx) + P.i0;
-  long q = box_idx(P.i0, P.in, P.j0, P.jn, kb, i, j, k);
-  long r = which == 0 ? p3_idx(P, i, j, k) : box_idx(P.i0b, P.inb, P.j0b, P.jnb, 1, i, j, k);
-  out[q] = src[r]; out[q + 1] = src[r + 1]; out[q + 2] = src[r + 2];
 }
 
 }  // namespace adz
@@ -524,23 +524,22 @@ int run_traject(adz_ctx* c, double dt, int advec, double bA_m, double bA, const 
   if (advec == 3) { dtA = (1.0 - bA_m) * dt; dtzA = (1.0 - bA) * dt; }
   double dtD = dt - dtA, dtzD = dt - dtzA;
   if (advec == 0) dtA = dtD = dtzA = dtzD = 0.0;
-  long next = (long)P.nij * P.nk, nint = (long)P.ni * P.nj * P.nk;
-  hipLaunchKernelGGL(k_prep_uvwd<S>, dim3(nb(next)), dim3(256), 0, st, (S*)c->uvw_d, uu, vv, ww, P);
+  long nint = (long)P.ni * P.nj * P.nk;
+  hipLaunchKernelGGL(k_prep_uvwd<S>, dim3(nb(P.nij), std::min(P.nk, kMaxGridY)), dim3(256), 0, st, (S*)c->uvw_d, uu, vv, ww, P);
   S* arr = (S*)c->warr;
-  hipLaunchKernelGGL(k_prep_arr<S>, dim3(nb(nint)), dim3(256), 0, st, arr, arr + nint, arr + 2 * nint, ut0, vt0, zdt0, P);
+  hipLaunchKernelGGL(k_prep_arr<S>, dim3(nb((long)P.ni * P.nj), std::min(P.nk, kMaxGridY)), dim3(256), 0, st, arr, arr + nint, arr + 2 * nint, ut0, vt0, zdt0, P);
   unsigned tw, tr;
   traj_tile(P.ni, P.nj, &tw, &tr);
   const long tiles = (long)((P.ni + tw - 1) / tw) * ((P.nj + tr - 1) / tr) * ((P.nk - P.k00 + kTrajLevels) / kTrajLevels);
   hipLaunchKernelGGL(k_traject<S>, tile_grid(tiles), dim3(64 * kTrajWaves), 0, st, (S*)c->pxyzm, c->wpxyz, (S*)c->uvw_dep,
-                     (const S*)c->uvw_d, arr, arr + nint, arr + 2 * nint, c->zq->dev, P, c->niter, dtA, dtD, dtzA,
+                     (S*)c->pm, (const S*)c->uvw_d, arr, arr + nint, arr + 2 * nint, c->zq->dev, P, c->niter, dtA, dtD, dtzA,
                      dtzD, tw, tr);
-  hipLaunchKernelGGL(k_copy_box<S>, dim3(nb(c->n_pm / 3)), dim3(256), 0, st, (S*)c->pm, (const S*)c->pxyzm, P, 0);
   c->niter = c->itraj;  // adz_traject.F90:120
-  hipLaunchKernelGGL(k_interp_uv<S>, dim3(nb(c->n_pmu / 3)), dim3(256), 0, st, (S*)c->pmu, c->wpxyz, P, 0);
-  hipLaunchKernelGGL(k_interp_uv<S>, dim3(nb(c->n_pmv / 3)), dim3(256), 0, st, (S*)c->pmv, c->wpxyz, P, 1);
-  hipLaunchKernelGGL(k_interp_b<S>, dim3(nb(c->n_pb / 3)), dim3(256), 0, st, (S*)c->pb, c->wpxyz, (const S*)c->uvw_dep,
-                     zdt0, P, dtzD, dtzA);
-  hipLaunchKernelGGL(k_copy_box<S>, dim3(nb(c->n_pt / 3)), dim3(256), 0, st, (S*)c->pt, (const S*)c->pb, P, 1);
+  // levels per lane: as many as leave eight waves for every SIMD, at most 8
+  const long cols = (long)((P.ni + 63) / 64) * ((P.nj + 3) / 4);
+  const int kc = (int)std::min(8L, std::max(1L, cols * 4 * P.nk / (8 * 1024)));
+  hipLaunchKernelGGL(k_sets<S>, tile_grid(cols * ((P.nk + kc - 1) / kc)), dim3(256), 0, st, (S*)c->pmu, (S*)c->pmv,
+                     (S*)c->pb, (S*)c->pt, c->wpxyz, (const S*)c->uvw_dep, zdt0, P, dtzD, dtzA, kc);
   ADZ_HIP_CHECK(hipGetLastError());
   return ADZ_OK;
 }
