@@ -45,7 +45,14 @@
 // trips to memory (the poll, f, the stores).  With one launch per hyperplane of cells the call
 // took 21.1 ms on any front; with one wave per cell in this scheme 7.4 to 16 ms; with windows
 // of 16, 6.2 (fronts along j) to 21 ms (along i); of 8, 5.8 to 13.9; of 2, 6.5 to 9.6; of 4,
-// 4.9 to 7.9 ms, and 5.9 to 9.6 with the two fences that order f against the bits.
+// 4.9 to 7.9 ms.
+//
+// f is read and written by agent-scope atomics only, which pass the caches that the XCDs do
+// not share, so a window needs no fence that writes back or invalidates a whole L2: it waits
+// for its own stores before it clears its bits.  With such fences, and with more waves, the
+// waves are in each other's way: 20 tracers of 512 x 384 x 84 with fronts 40 ms as a launch per
+// hyperplane, 74 with fences and 2048 waves, 42 with 512 waves, 23 without the fences; 6 smooth
+// tracers of 1024 x 512 x 84 37, 41, 30 and 22.5 ms.
 // Arithmetic is the reference's `real` arithmetic as written (built without contraction).
 #include <algorithm>
 #include <cstring>
@@ -59,7 +66,7 @@ constexpr int kIlBlock = 256;
 constexpr int kIlScan = 1024;
 constexpr int kIlWin = 4;          // cells of a row per piece of work
 constexpr uint64_t kIlMask = (1ull << kIlWin) - 1;
-constexpr int kIlWaves = 2048;     // most waves of the visiting launch
+constexpr int kIlWaves = 512;      // most waves of the visiting launch
 constexpr int kIlSpin = 1 << 22;   // polls of one wait (about 1 us each) before it gives up
 
 struct IlmcTr {
@@ -465,9 +472,12 @@ __global__ __launch_bounds__(64) void k_il_visit(IlmcArgs A) {
     const unsigned marked = (unsigned)((il_load(x.pend) >> (x.di & 63)) & kIlMask);
     il_fetch<S, AB>(A, T, x, K, L);
     if (!il_wait<S, AB>(A, x)) return;
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // f is loaded after the polls came back clear
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup");  // f is loaded after the polls came back clear
     const int moved = il_visit<S, AB>(A, T, x, marked, K, L);
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");  // the window's values are out before its bits go
+    // the window's values are out before its bits go: the stores of f, agent-scope atomics that
+    // go through to where every XCD sees them, have been acknowledged
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
     if (lane == 0) {
       __hip_atomic_fetch_and(x.pend, ~((uint64_t)marked << (x.di & 63)), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
       if (A.counts && moved) atomicAdd((unsigned long long*)&A.counts[3 * x.n], (unsigned long long)moved);
