@@ -351,8 +351,7 @@ def main():
             with torch.cuda.graph(gil, stream=sg):
                 il(airm0, counts)
         torch.cuda.current_stream().wait_stream(sg)
-        ilmc = {"tracers": len(ids_l), "cells_per_tracer": Nt_il, "sweep_max": 2,
-                "hyperplane_launches": (tbox[1] - tbox[0]) + 5 * (tbox[3] - tbox[2]) + 25 * (cfg.nk - tbox[4]) + 1}
+        ilmc = {"tracers": len(ids_l), "cells_per_tracer": Nt_il, "sweep_max": 2}
         for form in ("ref_math", "f32_math"):
             if form == "ref_math":
                 A.adz_tricub_hlt(stk, pt, ctx.ztab(True), *tbox[:5], tbox[5], mod_layout, ext=False,
@@ -381,8 +380,7 @@ def main():
             ilmc[form] = {"ms": round(min(t_ilg), 3), "ms_eager": round(min(t_il), 3), "cells_out_of_bounds": viol,
                           "sweeps_moving_mass": cnt[0], "min_resets": cnt[1], "max_resets": cnt[2]}
             log(f"ILMC beside the step ({form}): {min(t_ilg):.2f} ms in a graph ({min(t_il):.2f} eager) for "
-                f"{len(ids_l)} tracers, {viol} cells out of bounds, {cnt[0]} sweeps moved mass, "
-                f"{ilmc['hyperplane_launches']} hyperplane launches")
+                f"{len(ids_l)} tracers, {viol} cells out of bounds, {cnt[0]} sweeps moved mass")
         del gil
         il.free()
         torch.cuda.empty_cache()
@@ -896,7 +894,7 @@ def kernel_source_sha():
     import hashlib
 
     h = hashlib.sha256()
-    for fn in ("adz_batched.hip", "adz_common.h", "adz_eval.h"):
+    for fn in ("adz_batched.hip", "adz_common.h", "adz_eval.h", "adz_tile.h"):
         with open(os.path.join(ROOT, "gem_amd", "csrc", fn), "rb") as f:
             h.update(f.read())
     return h.hexdigest()[:16]
