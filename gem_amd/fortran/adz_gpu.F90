@@ -908,7 +908,7 @@ contains
    end subroutine ILMC_LAM
 
    ! ILMC on the tracers ns(:) of the current group at once (they do not interact): one
-   ! cached plan, one launch per hyperplane for all of them
+   ! cached plan, one launch sequence for all of them
    subroutine ilmc_tracers(ns, F_i0, F_in, F_j0, F_jn, F_name_S)
       integer, intent(in) :: ns(:), F_i0, F_in, F_j0, F_jn
       character(len=*), intent(in) :: F_name_S
