@@ -137,3 +137,30 @@ def test_staged_bf16_equals_per_lane(cuda, ni, nj, nk, halo, nf, ext, deform, sp
             # minNum / maxNum do not tell +0 from -0
             same = (a.view(np.uint32) == b.view(np.uint32)) | (np.isnan(a) & np.isnan(b)) | ((a == 0) & (b == 0))
             assert same.all(), (stage, q, int((~same).sum()))
+
+
+def test_more_blocks_than_a_row_of_the_grid(cuda):
+    """One column of 4099 x 4101 targets: 2.1 M tiles, whose blocks take a second row of the
+    grid; the call and the plan against per-lane loads."""
+    import torch
+
+    from gem_amd import _lib as L
+    from gem_amd import adz as A
+    from gem_amd import tricublin as TC
+
+    ni, nj, nk = 1, 4099, 4101
+    nx, ny = ni + 2 * MH, nj + 2 * MH
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    geom = TC.Ztab(np.arange(nk) + 1.0, nx, ny).set_bounds(1 - MH, ni + MH, 1 - MH, nj + MH)
+    pos = torch.rand(nk, nj, ni, 3, generator=gen, device="cuda") * 0.9
+    pos[..., 0] += 1.0
+    pos[..., 1] += torch.arange(1, nj + 1, device="cuda").view(1, nj, 1)
+    pos[..., 2] += torch.arange(1, nk + 1, device="cuda").view(nk, 1, 1)
+    src = [torch.rand(nx * ny * nk, generator=gen, device="cuda") for _ in range(2)]
+    s = (geom, (1, ni, 1, nj, 1, nk), pos.reshape(-1), src, MH + nx * MH)
+    want = _run(torch, A, L, s, torch.float32, L.ADZ_MATH_F32, 0, False, ni, nj, nk, 2)
+    for stage in ("call", None, 7):
+        got = _run(torch, A, L, s, torch.float32, L.ADZ_MATH_F32, 0, False, ni, nj, nk, stage)
+        for q, (a, b) in enumerate(zip(got, want)):
+            same = (a.view(np.uint32) == b.view(np.uint32)) | ((a == 0) & (b == 0))
+            assert same.all(), (stage, q, int((~same).sum()))
