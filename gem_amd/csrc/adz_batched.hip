@@ -276,17 +276,16 @@ __device__ __forceinline__ void per_lane(const DevItem& it, const Fields& F, int
   }
 }
 
-// The same for the few tiles whose box is not staged, one stencil row at a time: each value
-// goes through the operations of the evaluators above in their order, but only one row is
-// held, so that the staged kernels, which contain this path, keep their registers for the
-// staged one.
-template <class TF, int MATH, int POST, class Fields>
-__device__ __forceinline__ void per_lane_rows(const DevItem& it, const Fields& F, int f0, int f1, const Index& x,
-                                              bool ok, bool valid, const double* cw, long o) {
+// The same for the tiles whose box is not staged, one stencil row at a time: each value goes
+// through the operations of the evaluators above in their order, but only one row is held (two
+// of FP32 sources), so that the staged kernels, which contain this path, keep their registers
+// for the staged one.  row(r, q) reads row r of field f, q[plane][column].
+template <class TF, int MATH, int POST, class Fields, class Row>
+__device__ __forceinline__ void eval_by_rows(const Fields& F, int f, const double* cw, long o, Row row) {
   typedef typename std::conditional<MATH == ADZ_MATH_REF, double, float>::type TC;
   typedef typename std::conditional<MATH == ADZ_MATH_REF && sizeof(TF) == 8, double, float>::type TM;
+  constexpr bool kAhead = sizeof(TF) == 4;  // the next row is on its way
   const TC* c = (const TC*)cw;
-  const long gni = it.lv.ni, o1 = x.zlinear ? 0 : (long)it.lv.nij, o2 = o1 + it.lv.nij, o3 = o2 + o1;
   auto wide = [](TF v) -> TC {
     if constexpr (MATH == ADZ_MATH_REF) return to_f64<TF>(v);
     else return to_f32<TF>(v);
@@ -295,74 +294,118 @@ __device__ __forceinline__ void per_lane_rows(const DevItem& it, const Fields& F
     if constexpr (MATH == ADZ_MATH_REF) return fma(p, q, r);
     else return fmaf(p, q, r);
   };
-#pragma unroll 1
-  for (int f = f0; f < f1; f++) {
-    if (!ok) {
-      if (valid) store_nan<TF, MATH, POST>(F, f, o);
-      continue;
-    }
-    const typename GPtr<TF>::ctype s0 = (typename GPtr<TF>::ctype)F.s(f) + x.off;
-    TC ya[4] = {0, 0, 0, 0}, vl[4] = {0, 0, 0, 0};
-    TM vmi[4] = {0, 0, 0, 0}, vma[4] = {0, 0, 0, 0}, lo = 0, hi = 0;
-#pragma unroll 1
-    for (int r = 0; r < 4; r++) {
-      const typename GPtr<TF>::ctype s = s0 + r * gni;
-      const TC cy = r == 0 ? c[4] : (r == 1 ? c[5] : (r == 2 ? c[6] : c[7]));
-      TF p1[4], p2[4];
+  TF q[kAhead ? 2 : 1][4][4];
+  if (kAhead) row(0, q[0]);
+  TC ya[4] = {0, 0, 0, 0}, vl[4] = {0, 0, 0, 0};
+  TM vmi[4] = {0, 0, 0, 0}, vma[4] = {0, 0, 0, 0}, lo = 0, hi = 0;
+#pragma unroll kAhead ? 4 : 1
+  for (int r = 0; r < 4; r++) {
+    if (!kAhead) row(r, q[0]);
+    else if (r < 3) row(r + 1, q[(r + 1) & 1]);
+    const TF(&v)[4][4] = q[kAhead ? r & 1 : 0];
+    const TC cy = r == 0 ? c[4] : (r == 1 ? c[5] : (r == 2 ? c[6] : c[7]));
 #pragma unroll
-      for (int i = 0; i < 4; i++) {
-        p1[i] = s[o1 + i];
-        p2[i] = s[o2 + i];
-        TC za = wide(s[i]) * c[8];
-        za = fm(wide(p1[i]), c[9], za);
-        za = fm(wide(p2[i]), c[10], za);
-        za = fm(wide(s[o3 + i]), c[11], za);
-        ya[i] = r == 0 ? za * cy : fm(za, cy, ya[i]);
-      }
-      if (POST) {
-        if (r == 1 || r == 2)
-#pragma unroll
-          for (int i = 0; i < 4; i++) {
-            TC vz = wide(p1[i]) * c[18];
-            vz = fm(wide(p2[i]), c[19], vz);
-            vl[i] = r == 1 ? vz * c[16] : fm(vz, c[17], vl[i]);
-          }
-        if constexpr (MATH == ADZ_MATH_REF) {
-#pragma unroll
-          for (int i = 1; i < 3; i++) {
-            const TM a = (TM)to_f64<TF>(p1[i]), b = (TM)to_f64<TF>(p2[i]);
-            if (r == 0) { vmi[i] = a; vma[i] = a; }
-            else { vmi[i] = (vmi[i] < a) ? vmi[i] : a; vma[i] = (vma[i] > a) ? vma[i] : a; }
-            vmi[i] = (vmi[i] < b) ? vmi[i] : b;
-            vma[i] = (vma[i] > b) ? vma[i] : b;
-          }
-        } else {
-          const float a1 = to_f32<TF>(p1[1]), a2 = to_f32<TF>(p1[2]), b1 = to_f32<TF>(p2[1]), b2 = to_f32<TF>(p2[2]);
-          if (r == 0) lo = hi = a1;
-          lo = fminf(fminf(lo, a1), fminf(a2, fminf(b1, b2)));
-          hi = fmaxf(fmaxf(hi, a1), fmaxf(a2, fmaxf(b1, b2)));
-        }
-      }
-    }
-    TC v, l = 0, mi = 0, ma = 0;
-    if constexpr (MATH == ADZ_MATH_REF) {
-      const TC y0 = ya[0] * c[0], y1 = ya[1] * c[1], y2 = ya[2] * c[2], y3 = ya[3] * c[3];
-      v = (y0 + y2) + (y1 + y3);
-    } else {
-      v = fm(ya[3], c[3], fm(ya[2], c[2], fm(ya[1], c[1], ya[0] * c[0])));
+    for (int i = 0; i < 4; i++) {
+      TC za = wide(v[0][i]) * c[8];
+      za = fm(wide(v[1][i]), c[9], za);
+      za = fm(wide(v[2][i]), c[10], za);
+      za = fm(wide(v[3][i]), c[11], za);
+      ya[i] = r == 0 ? za * cy : fm(za, cy, ya[i]);
     }
     if (POST) {
-      const TC l0 = vl[0] * c[12], l1 = vl[1] * c[13], l2 = vl[2] * c[14], l3 = vl[3] * c[15];
-      l = (l0 + l2) + (l1 + l3);
+      if (r == 1 || r == 2)
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+          TC vz = wide(v[1][i]) * c[18];
+          vz = fm(wide(v[2][i]), c[19], vz);
+          vl[i] = r == 1 ? vz * c[16] : fm(vz, c[17], vl[i]);
+        }
       if constexpr (MATH == ADZ_MATH_REF) {
-        mi = (TC)((vmi[1] < vmi[2]) ? vmi[1] : vmi[2]);
-        ma = (TC)((vma[1] > vma[2]) ? vma[1] : vma[2]);
+#pragma unroll
+        for (int i = 1; i < 3; i++) {
+          const TM a = (TM)to_f64<TF>(v[1][i]), b = (TM)to_f64<TF>(v[2][i]);
+          if (r == 0) { vmi[i] = a; vma[i] = a; }
+          else { vmi[i] = (vmi[i] < a) ? vmi[i] : a; vma[i] = (vma[i] > a) ? vma[i] : a; }
+          vmi[i] = (vmi[i] < b) ? vmi[i] : b;
+          vma[i] = (vma[i] > b) ? vma[i] : b;
+        }
       } else {
-        mi = lo;
-        ma = hi;
+        const float a1 = to_f32<TF>(v[1][1]), a2 = to_f32<TF>(v[1][2]), b1 = to_f32<TF>(v[2][1]), b2 = to_f32<TF>(v[2][2]);
+        if (r == 0) lo = hi = a1;
+        lo = fminf(fminf(lo, a1), fminf(a2, fminf(b1, b2)));
+        hi = fmaxf(fmaxf(hi, a1), fmaxf(a2, fmaxf(b1, b2)));
       }
     }
-    store_out<TF, MATH, POST>(F, f, o, v, l, mi, ma);
+    if constexpr (kAhead) {  // the row is done with here, and no further one is read before
+      asm volatile("" : "+v"(ya[0]), "+v"(ya[1]), "+v"(ya[2]), "+v"(ya[3])::"memory");
+      if (POST) asm volatile("" : "+v"(vl[0]), "+v"(vl[1]), "+v"(vl[2]), "+v"(vl[3]));
+    }
+  }
+  TC v, l = 0, mi = 0, ma = 0;
+  if constexpr (MATH == ADZ_MATH_REF) {
+    const TC y0 = ya[0] * c[0], y1 = ya[1] * c[1], y2 = ya[2] * c[2], y3 = ya[3] * c[3];
+    v = (y0 + y2) + (y1 + y3);
+  } else {
+    v = fm(ya[3], c[3], fm(ya[2], c[2], fm(ya[1], c[1], ya[0] * c[0])));
+  }
+  if (POST) {
+    const TC l0 = vl[0] * c[12], l1 = vl[1] * c[13], l2 = vl[2] * c[14], l3 = vl[3] * c[15];
+    l = (l0 + l2) + (l1 + l3);
+    if constexpr (MATH == ADZ_MATH_REF) {
+      mi = (TC)((vmi[1] < vmi[2]) ? vmi[1] : vmi[2]);
+      ma = (TC)((vma[1] > vma[2]) ? vma[1] : vma[2]);
+    } else {
+      mi = lo;
+      ma = hi;
+    }
+  }
+  store_out<TF, MATH, POST>(F, f, o, v, l, mi, ma);
+}
+
+// Every field of a tile whose box is not staged, read per lane: from global memory, or for FP32
+// sources within 32-bit offsets by buffer loads (a row's stride is uniform and goes in the
+// instruction's scalar offset).  The whole block comes here, and its waves go from field to
+// field together: what bounds this path is the first-level cache, which holds the lines of one
+// field that the waves share but not those of several.  512 x 384 x 84, sheared positions (no
+// box fits), us per call: 4 FP32 fields 1590 with the waves on their own, 1000 now (1080 in the
+// build whose staged kernels held one field's 16 rows in registers); 10 with lin/min/max 5180
+// and 3510 (3540); 6 in the reference's arithmetic 2200 and 1560 (1950).
+template <class TF, int MATH, int POST, class Fields>
+__device__ __forceinline__ void per_lane_rows(const DevItem& it, const Fields& F, int f0, int f1, const Index& x,
+                                              bool ok, bool valid, const double* cw, long o) {
+  const long gni = it.lv.ni, o1 = x.zlinear ? 0 : (long)it.lv.nij, o2 = o1 + it.lv.nij, o3 = o2 + o1;
+  auto one = [&](int f) {
+    if constexpr (std::is_same<TF, float>::value) {
+      if (it.span) {
+        const int e = (int)(x.off - it.minoff) * 4, b1 = (int)o1 * 4, b2 = (int)o2 * 4, b3 = (int)o3 * 4;
+        const int rstride = (int)(gni * 4);
+        const __amdgpu_buffer_rsrc_t rs = field_rsrc((const float*)F.s(f) + it.minoff, it.span);
+        eval_by_rows<TF, MATH, POST>(F, f, cw, o, [&](int r, TF(&q)[4][4]) {
+#pragma unroll
+          for (int z = 0; z < 4; z++) {
+            const int b = e + (z == 0 ? 0 : z == 1 ? b1 : z == 2 ? b2 : b3);
+            const f32x4 v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, b, r * rstride, 0));
+#pragma unroll
+            for (int i = 0; i < 4; i++) q[z][i] = v[i];
+          }
+        });
+        return;
+      }
+    }
+    const typename GPtr<TF>::ctype s0 = (typename GPtr<TF>::ctype)F.s(f) + x.off;
+    eval_by_rows<TF, MATH, POST>(F, f, cw, o, [&](int r, TF(&q)[4][4]) {
+      const typename GPtr<TF>::ctype s = s0 + r * gni;
+#pragma unroll
+      for (int z = 0; z < 4; z++)
+#pragma unroll
+        for (int i = 0; i < 4; i++) q[z][i] = s[(z == 0 ? 0 : z == 1 ? o1 : z == 2 ? o2 : o3) + i];
+    });
+  };
+#pragma unroll 1
+  for (int f = f0; f < f1; f++) {
+    if (ok) one(f);
+    else if (valid) store_nan<TF, MATH, POST>(F, f, o);
+    __syncthreads();
   }
 }
 
@@ -1163,10 +1206,21 @@ __device__ __forceinline__ void dma_tile(const DevItem& it, const Fields& F, lon
   const long last = (long)(x0 - 1) + (long)kE * cpr - 1 + (long)(y0 + nyb - 2) * gni + (long)(z0 + nzb - 1) * gnij -
                     it.minoff;
   const unsigned span = it.span / 4 * SZ;  // (it.span is in bytes of FP32)
-  if (nrows > kRows || cpr > kQ || !stageable(it, SZ) || first < 0 || (last + 1) * 4 > (long)it.span) {
+  // (FP64 fields: marked unlikely, so that it is this path that gives up registers and not the
+  // staged one, whose reloads would wait for the boxes under way: 4 fields of 512 x 384 x 84 with
+  // lin/min/max 1.07 ms, 1.19 without.  The 4-byte kernels reload nothing there, and lose 4 % by
+  // the mark.)
+#define ADZ_UNSTAGED nrows > kRows || cpr > kQ || !stageable(it, SZ) || first < 0 || (last + 1) * 4 > (long)it.span
+  if constexpr (SZ == 8) {
+    if (__builtin_expect(ADZ_UNSTAGED, 0)) {
+      per_lane_rows<TF, MATH, POST>(it, F, f0, f1, x, ok, valid, cw, od + it.omin);
+      return;
+    }
+  } else if (ADZ_UNSTAGED) {
     per_lane_rows<TF, MATH, POST>(it, F, f0, f1, x, ok, valid, cw, od + it.omin);
     return;
   }
+#undef ADZ_UNSTAGED
   // this lane's DMA slots: instruction q of wave wv fills the 64 quads g*64 .. g*64+63 of
   // the buffer (g = wv + W q), quad Q = row Q / kQ, column quad Q % kQ; byte offsets from
   // minoff of the lane's quad, or one out of range where the box has none
@@ -1435,9 +1489,13 @@ __global__ __launch_bounds__(kTile) void k_hlt(DevItem it, InlineFields F) {
 // Measured against 64 x 8 x 1 tiles with 62 rows per box, where a third of the tiles of a
 // 200 x 150 grid and four fifths of a 512 x 384 one fitted: 3 fields of 200 x 150 x 60 in the
 // reference's arithmetic 63.7 -> 54.8 us; in FP32, 4 fields of 512 x 384 x 84 681 -> 550 us,
-// 8 of 2048 x 1024 x 84 13.4 -> 8.2 ms.  Super-columns of 3 tile rows in place of rows, then
-// levels: 8.2 and 55 against 8.3 and 52 us (3 fields of 200 x 150 x 60, FP32).
-constexpr int kHltOrder = 0;
+// 8 of 2048 x 1024 x 84 13.4 -> 8.2 ms.
+// Tile order: super-columns of three tile rows, which read a source plane again while it is in
+// an XCD's L2; rows, then levels, where lin/min/max are stored, whose streams prefer it.  us,
+// super-columns (rows): 512 x 384 x 84, smooth positions, 4 FP64 fields 705 (735), 4 FP32 419
+// (426), 2 FP32 with lin/min/max 355 (342); sheared by up to 0.8 cells per cell, 4 FP64 2276
+// (2899), 4 FP32 1299 (1686); 3 fields of 200 x 150 x 60, reference arithmetic, 52.4 (50.3).
+constexpr int hlt_order(int post) { return post & ADZ_POST_STORE ? 0 : 3; }
 constexpr int kHltTH = kTJ, kHltTL = 2;
 
 template <class TF, class TP, int MATH, int POST>
@@ -1446,7 +1504,7 @@ __global__ __launch_bounds__(64 * kHltTH * kHltTL,
   ADZ_BOXES(TF, kHltTH * kHltTL, dma_waves(sizeof(TF), kHltTH * kHltTL, MATH, POST))
   const long t = tile_of_block(ntiles, 1);
   if (t >= ntiles) return;  // the whole block leaves: no barrier is reached
-  dma_tile<TF, MATH, POST, TP, kHltTH, kHltTL>(it, F, t, 0, it.nf, boxA, boxB, red, 0, kHltOrder);
+  dma_tile<TF, MATH, POST, TP, kHltTH, kHltTL>(it, F, t, 0, it.nf, boxA, boxB, red, 0, hlt_order(POST));
 }
 
 }  // namespace adz
@@ -1702,7 +1760,7 @@ int adz_tricub_hlt(const adz_field* fld, int nptr, const void* xyz, int pdtype, 
     DevItem it;
     if (!fill_item(&it, geom, xyz, i0, in, j0, jn, k0, nk, dminx, dmaxx, dminy, dmaxy, ext, nf))
       return fail(ADZ_EINVAL, "adz_tricub_hlt: bad box or descriptor");
-    if (item_ptiles(it.nx, it.ny, it.nz, kHltOrder) >= (1L << 31) - 8)
+    if (item_ptiles(it.nx, it.ny, it.nz, 0) >= (1L << 31) - 8)
       return fail(ADZ_EINVAL, "adz_tricub_hlt: a box of 2^31 tiles or more");
     InlineFields F;
     std::memset(&F, 0, sizeof(F));
@@ -1714,7 +1772,7 @@ int adz_tricub_hlt(const adz_field* fld, int nptr, const void* xyz, int pdtype, 
                         !few_fields(fdtype, math, post, (long)it.nx * it.ny * it.nz, nf);
     void* kern = pick<false>(fdtype, pdtype, math, post, staged ? 7 : 2);
     if (staged) {  // k_hlt5: LDS-staged boxes, an eighth of the tile list per XCD
-      long ntiles = item_ptiles(it.nx, it.ny, it.nz, kHltOrder, kTI, kHltTH, kHltTL);
+      long ntiles = item_ptiles(it.nx, it.ny, it.nz, hlt_order(post), kTI, kHltTH, kHltTL);
       void* args[] = {&it, &F, &ntiles};
       ADZ_HIP_CHECK(hipLaunchKernel(kern, tile_grid(ntiles), dim3(64 * kHltTH * kHltTL), args, 0, (hipStream_t)stream));
     } else {
