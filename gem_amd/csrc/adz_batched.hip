@@ -1689,14 +1689,17 @@ bool few_fields(int fdtype, int math, int post, long targets, int fields) {
 // Tiles walk rows, then levels, where lin/min/max are stored (levels first, 3.95 and 15.5 ms
 // in lines two and three), else the levels of a column first (rows first 3.95 ms in line
 // one); FP64 fields super-columns of two tile rows (line five; rows first 0.77).
-// Items beyond 32-bit offsets, and too few fields (few_fields): per-lane loads (stage 2).
+// Too few fields (few_fields), and plans of which every item is beyond 32-bit offsets: per-lane
+// loads (stage 2).  Such an item among others reads per lane in the staged kernel: six subdomains
+// of 64 x 48 to 512 x 384 and one more with a source of 2600 x 2600 x 84, 6 FP32 fields, 1.53 ms
+// (2.42 with stage 2 for all).
 adz_tune default_tune(int fdtype, int math, int post, bool staged, long targets, int fields) {
   if (!staged) return adz_tune{10, 0, 4, 1, 2, 3};
   if (few_fields(fdtype, math, post, targets, fields)) return adz_tune{10, 0, 32, 1, 2, targets < (1L << 24) ? 1 : 0};
   return adz_tune{10, 0, 8, 1, 7, fdtype == ADZ_F64 ? 2 : post & ADZ_POST_STORE ? 0 : 1};
 }
 adz_tune default_tune(const adz_item* items, int nitems, int fdtype, int math, int post) {
-  bool staged = true;
+  bool staged = false;
   long targets = 0;
   int fields = 0;
   for (int q = 0; q < nitems && items; q++) {
@@ -1704,7 +1707,7 @@ adz_tune default_tune(const adz_item* items, int nitems, int fdtype, int math, i
     DevItem d;
     if (fill_item(&d, a.geom, a.xyz, a.i0, a.in, a.j0, a.jn, a.k0, a.nk, a.dminx, a.dmaxx, a.dminy, a.dmaxy, a.ext,
                   a.nptr)) {
-      staged = staged && stageable(d, field_bytes(fdtype));
+      staged = staged || stageable(d, field_bytes(fdtype));
       targets += (long)d.nx * d.ny * d.nz;
       fields = std::max(fields, a.nptr);
     }

@@ -227,8 +227,8 @@ typedef struct adz_item {
 } adz_item;
 
 /* Tile parameters of the persistent kernel; zero fields_per_pass / blocks_per_cu take the
-   built-in default: ten fields per pass, stage 7 (stage 2 for arrays beyond 32-bit byte
-   offsets, and for one field where that is too few to stage).  Stage 0 takes the built-in
+   built-in default: ten fields per pass, stage 7 (stage 2 where all items are beyond 32-bit
+   byte offsets, and for one field where that is too few to stage).  Stage 0 takes the built-in
    staging together with its level_inner; adz_plan_autotune searches them on the actual
    plan. */
 typedef struct adz_tune {
