@@ -276,15 +276,12 @@ __device__ __forceinline__ void per_lane(const DevItem& it, const Fields& F, int
   }
 }
 
-// The same for the tiles whose box is not staged, one stencil row at a time: each value goes
-// through the operations of the evaluators above in their order, but only one row is held (two
-// of FP32 sources), so that the staged kernels, which contain this path, keep their registers
-// for the staged one.  row(r, q) reads row r of field f, q[plane][column].
-template <class TF, int MATH, int POST, class Fields, class Row>
-__device__ __forceinline__ void eval_by_rows(const Fields& F, int f, const double* cw, long o, Row row) {
-  typedef typename std::conditional<MATH == ADZ_MATH_REF, double, float>::type TC;
+// The same one stencil row at a time: each value goes through the operations of the evaluators
+// above in their order, but only one row is held (two with AHEAD, the next one on its way).
+// row(r, q) reads row r, q[plane][column].
+template <class TF, int MATH, int POST, bool AHEAD, class Row, class TC>
+__device__ __forceinline__ void eval_by_rows(Row row, const double* cw, TC* v_, TC* l_, TC* mi_, TC* ma_) {
   typedef typename std::conditional<MATH == ADZ_MATH_REF && sizeof(TF) == 8, double, float>::type TM;
-  constexpr bool kAhead = sizeof(TF) == 4;  // the next row is on its way
   const TC* c = (const TC*)cw;
   auto wide = [](TF v) -> TC {
     if constexpr (MATH == ADZ_MATH_REF) return to_f64<TF>(v);
@@ -294,15 +291,15 @@ __device__ __forceinline__ void eval_by_rows(const Fields& F, int f, const doubl
     if constexpr (MATH == ADZ_MATH_REF) return fma(p, q, r);
     else return fmaf(p, q, r);
   };
-  TF q[kAhead ? 2 : 1][4][4];
-  if (kAhead) row(0, q[0]);
+  TF q[AHEAD ? 2 : 1][4][4];
+  if (AHEAD) row(0, q[0]);
   TC ya[4] = {0, 0, 0, 0}, vl[4] = {0, 0, 0, 0};
   TM vmi[4] = {0, 0, 0, 0}, vma[4] = {0, 0, 0, 0}, lo = 0, hi = 0;
-#pragma unroll kAhead ? 4 : 1
+#pragma unroll AHEAD ? 4 : 1
   for (int r = 0; r < 4; r++) {
-    if (!kAhead) row(r, q[0]);
+    if (!AHEAD) row(r, q[0]);
     else if (r < 3) row(r + 1, q[(r + 1) & 1]);
-    const TF(&v)[4][4] = q[kAhead ? r & 1 : 0];
+    const TF(&v)[4][4] = q[AHEAD ? r & 1 : 0];
     const TC cy = r == 0 ? c[4] : (r == 1 ? c[5] : (r == 2 ? c[6] : c[7]));
 #pragma unroll
     for (int i = 0; i < 4; i++) {
@@ -336,30 +333,28 @@ __device__ __forceinline__ void eval_by_rows(const Fields& F, int f, const doubl
         hi = fmaxf(fmaxf(hi, a1), fmaxf(a2, fmaxf(b1, b2)));
       }
     }
-    if constexpr (kAhead) {  // the row is done with here, and no further one is read before
+    if constexpr (AHEAD) {  // the row is done with here, and no further one is read before
       asm volatile("" : "+v"(ya[0]), "+v"(ya[1]), "+v"(ya[2]), "+v"(ya[3])::"memory");
-      if (POST) asm volatile("" : "+v"(vl[0]), "+v"(vl[1]), "+v"(vl[2]), "+v"(vl[3]));
+      if (POST & ADZ_POST_STORE) asm volatile("" : "+v"(vl[0]), "+v"(vl[1]), "+v"(vl[2]), "+v"(vl[3]));
     }
   }
-  TC v, l = 0, mi = 0, ma = 0;
   if constexpr (MATH == ADZ_MATH_REF) {
     const TC y0 = ya[0] * c[0], y1 = ya[1] * c[1], y2 = ya[2] * c[2], y3 = ya[3] * c[3];
-    v = (y0 + y2) + (y1 + y3);
+    *v_ = (y0 + y2) + (y1 + y3);
   } else {
-    v = fm(ya[3], c[3], fm(ya[2], c[2], fm(ya[1], c[1], ya[0] * c[0])));
+    *v_ = fm(ya[3], c[3], fm(ya[2], c[2], fm(ya[1], c[1], ya[0] * c[0])));
   }
   if (POST) {
     const TC l0 = vl[0] * c[12], l1 = vl[1] * c[13], l2 = vl[2] * c[14], l3 = vl[3] * c[15];
-    l = (l0 + l2) + (l1 + l3);
+    *l_ = (l0 + l2) + (l1 + l3);
     if constexpr (MATH == ADZ_MATH_REF) {
-      mi = (TC)((vmi[1] < vmi[2]) ? vmi[1] : vmi[2]);
-      ma = (TC)((vma[1] > vma[2]) ? vma[1] : vma[2]);
+      *mi_ = (TC)((vmi[1] < vmi[2]) ? vmi[1] : vmi[2]);
+      *ma_ = (TC)((vma[1] > vma[2]) ? vma[1] : vma[2]);
     } else {
-      mi = lo;
-      ma = hi;
+      *mi_ = lo;
+      *ma_ = hi;
     }
   }
-  store_out<TF, MATH, POST>(F, f, o, v, l, mi, ma);
 }
 
 // Every field of a tile whose box is not staged, read per lane: from global memory, or for FP32
@@ -373,27 +368,34 @@ __device__ __forceinline__ void eval_by_rows(const Fields& F, int f, const doubl
 template <class TF, int MATH, int POST, class Fields>
 __device__ __forceinline__ void per_lane_rows(const DevItem& it, const Fields& F, int f0, int f1, const Index& x,
                                               bool ok, bool valid, const double* cw, long o) {
+  typedef typename std::conditional<MATH == ADZ_MATH_REF, double, float>::type TC;
+  constexpr bool kAhead = sizeof(TF) == 4;  // (two rows of FP64 values, or of 2-byte loads, do not fit)
   const long gni = it.lv.ni, o1 = x.zlinear ? 0 : (long)it.lv.nij, o2 = o1 + it.lv.nij, o3 = o2 + o1;
   auto one = [&](int f) {
+    TC v, l = 0, mi = 0, ma = 0;
+    auto eval = [&](auto row) {
+      eval_by_rows<TF, MATH, POST, kAhead>(row, cw, &v, &l, &mi, &ma);
+      store_out<TF, MATH, POST>(F, f, o, v, l, mi, ma);
+    };
     if constexpr (std::is_same<TF, float>::value) {
       if (it.span) {
         const int e = (int)(x.off - it.minoff) * 4, b1 = (int)o1 * 4, b2 = (int)o2 * 4, b3 = (int)o3 * 4;
         const int rstride = (int)(gni * 4);
         const __amdgpu_buffer_rsrc_t rs = field_rsrc((const float*)F.s(f) + it.minoff, it.span);
-        eval_by_rows<TF, MATH, POST>(F, f, cw, o, [&](int r, TF(&q)[4][4]) {
+        eval([&](int r, TF(&q)[4][4]) {
 #pragma unroll
           for (int z = 0; z < 4; z++) {
             const int b = e + (z == 0 ? 0 : z == 1 ? b1 : z == 2 ? b2 : b3);
-            const f32x4 v = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, b, r * rstride, 0));
+            const f32x4 w = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs, b, r * rstride, 0));
 #pragma unroll
-            for (int i = 0; i < 4; i++) q[z][i] = v[i];
+            for (int i = 0; i < 4; i++) q[z][i] = w[i];
           }
         });
         return;
       }
     }
     const typename GPtr<TF>::ctype s0 = (typename GPtr<TF>::ctype)F.s(f) + x.off;
-    eval_by_rows<TF, MATH, POST>(F, f, cw, o, [&](int r, TF(&q)[4][4]) {
+    eval([&](int r, TF(&q)[4][4]) {
       const typename GPtr<TF>::ctype s = s0 + r * gni;
 #pragma unroll
       for (int z = 0; z < 4; z++)
@@ -1295,21 +1297,32 @@ __device__ __forceinline__ void dma_tile(const DevItem& it, const Fields& F, lon
     if constexpr (SZ == 2) {
       // a stencil row from the three words that hold it; with rows of odd length every other
       // one begins at the other half of a word
-      u32x2 q[4][4];
       const int other = ni32 & 1;
+      auto words = [&](int r, int z) {
+        const int h = odd[z] ^ half, e = lb[z] + (r & 1 ? h ^ other : h);
+        const unsigned* b = (const unsigned*)buf + (e >> 1) + r * (kPitch / 2);
+        const unsigned sh = (unsigned)e << 4;  // 16 where odd (a shift of 32 bits or more is taken modulo 32)
+        return u32x2{__builtin_amdgcn_alignbit(b[1], b[0], sh), __builtin_amdgcn_alignbit(b[2], b[1], sh)};
+      };
+      if constexpr (POST == ADZ_POST_CLIP) {
+        // row by row: read as below the values would not fit 80 registers, and the reloads in
+        // every step cost more than the boxes gain
+        eval_by_rows<TF, MATH, POST, true>([&](int r, TF(&q)[4][4]) {
 #pragma unroll
-      for (int z = 0; z < 4; z++) {
-        const int h = odd[z] ^ half, e0 = lb[z] + h, e1 = lb[z] + (h ^ other);
-        const unsigned* b0 = (const unsigned*)buf + (e0 >> 1);
-        const unsigned* b1 = (const unsigned*)buf + (e1 >> 1);
+          for (int z = 0; z < 4; z++) {
+            const u32x2 w = words(r, z);
 #pragma unroll
-        for (int r = 0; r < 4; r++) {
-          const unsigned* b = (r & 1 ? b1 : b0) + r * (kPitch / 2);
-          const unsigned sh = (unsigned)(r & 1 ? e1 : e0) << 4;  // 16 where odd (a shift of 32 bits or more is taken modulo 32)
-          q[r][z] = u32x2{__builtin_amdgcn_alignbit(b[1], b[0], sh), __builtin_amdgcn_alignbit(b[2], b[1], sh)};
-        }
+            for (int i = 0; i < 4; i++) q[z][i] = __builtin_bit_cast(bf16, (uint16_t)(w[i >> 1] >> (16 * (i & 1))));
+          }
+        }, cw, &v, &l, &mi, &ma);
+      } else {
+        u32x2 q[4][4];
+#pragma unroll
+        for (int z = 0; z < 4; z++)
+#pragma unroll
+          for (int r = 0; r < 4; r++) q[r][z] = words(r, z);
+        eval_vals<TF, MATH, POST>(HalfStencil{q}, cw, &v, &l, &mi, &ma);
       }
-      eval_vals<TF, MATH, POST>(HalfStencil{q}, cw, &v, &l, &mi, &ma);
     } else {
       const TF* b0 = buf + lb[0];
       const TF* b1 = buf + lb[1];
