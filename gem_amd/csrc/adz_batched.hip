@@ -1678,16 +1678,26 @@ void* pick(int fdt, int pdt, int math, int post, int stage = 2) {
 
 int field_bytes(int fdtype) { return fdtype == ADZ_F64 ? 8 : fdtype == ADZ_F32 ? 4 : 2; }
 
-// Too few fields to pay for a tile's extents and its first box?  One FP32 or unclipped FP64
-// field below 2^24 targets, or one clipped FP32 field in the reference's arithmetic.  Per-lane
-// loads (staged boxes), us, 304 x 227 x 84 and 800 x 500 x 84: FP32 arithmetic, one field 65
-// (78) and 427 (458), clipped 84 (88) and 595 (530), two 105 (98) and 750 (601); reference
-// arithmetic, one field 83 (96) and 575 (553), clipped 107 (134) and 737 (855), two clipped 183
-// (183) and 1257 (1135); FP64, one field 115 (120) and 803 (748), clipped 181 (150) and 1278
-// (946); BF16, one field 90 (93) and 585 (570).
-bool few_fields(int fdtype, int math, int post, long targets, int fields) {
-  if (fields > 1 || fdtype == ADZ_BF16 || (fdtype == ADZ_F64 && post)) return false;
-  return targets < (1L << 24) || (math != ADZ_MATH_F32 && post);
+// One field, which does not pay for a tile's extents and its first box?  By what was measured, us,
+// per-lane loads (staged boxes) of one field of 304 x 227 x 84, 512 x 384 x 84 and 1024 x 512 x 84;
+// two fields of 304 x 227 x 84 and more gain by staging in every form.  The call / a plan:
+//   FP32 arithmetic              61 (73), 198 (213), 535 (574)     / 64 (78), 201 (233), 560 (631)
+//     clipped                    61 (74), 204 (214), 546 (579)     / 68 (78), 213 (228), 596 (617)
+//     lin/min/max                77 (76), 281 (237), 749 (636)     / 83 (86), 283 (269), 812 (713)
+//   reference arithmetic         81 (89), 261 (250), 709 (682)     / 83 (92), 254 (266), 710 (723)
+//     clipped                    116 (126), 352 (364), 949 (987)   / 85 (128), 250 (379), 687 (1018)
+//     lin/min/max                115 (126), 383 (395), 1027 (1068) / 108 (135), 340 (417), 940 (1129)
+//   FP64                         112 (120), 377 (351), 995 (946)   / 116 (122), 359 (358), 1029 (949)
+//     clipped                    143 (141), 439 (417), 1156 (1122) / 122 (142), 362 (431), 1016 (1160)
+//     lin/min/max                168 (145), 554 (447), 1449 (1186) / 181 (151), 600 (458), 1630 (1225)
+//   BF16                         88 (87), 249 (233), 737 (667)     / 90 (92), 252 (257), 774 (725)
+//     lin/min/max                101 (93), 337 (270), 880 (737)    / 108 (103), 342 (300), 938 (809)
+bool few_fields(int fdtype, int math, int post, long targets, int fields, bool plan) {
+  if (fields > 1 || fdtype == ADZ_BF16) return false;
+  const bool few = targets < (1L << 23);
+  if (fdtype == ADZ_F64) return post & ADZ_POST_STORE ? false : post ? plan : few;
+  if (math == ADZ_MATH_F32) return post & ADZ_POST_STORE ? few : true;
+  return post || few || (plan && targets < (1L << 26));  // (a plan of 1600 x 1200 x 84: 2.75 ms, staged 2.70)
 }
 
 // Built-in tile parameters: ten fields per pass, LDS-staged boxes of tiles of 64 x 4 targets x
@@ -1708,7 +1718,7 @@ bool few_fields(int fdtype, int math, int post, long targets, int fields) {
 // (2.42 with stage 2 for all).
 adz_tune default_tune(int fdtype, int math, int post, bool staged, long targets, int fields) {
   if (!staged) return adz_tune{10, 0, 4, 1, 2, 3};
-  if (few_fields(fdtype, math, post, targets, fields)) return adz_tune{10, 0, 32, 1, 2, targets < (1L << 24) ? 1 : 0};
+  if (few_fields(fdtype, math, post, targets, fields, true)) return adz_tune{10, 0, 32, 1, 2, targets < (1L << 24) ? 1 : 0};
   return adz_tune{10, 0, 8, 1, 7, fdtype == ADZ_F64 ? 2 : post & ADZ_POST_STORE ? 0 : 1};
 }
 adz_tune default_tune(const adz_item* items, int nitems, int fdtype, int math, int post) {
@@ -1785,7 +1795,7 @@ int adz_tricub_hlt(const adz_field* fld, int nptr, const void* xyz, int pdtype, 
       F.src[f] = a.src; F.dst[f] = a.dst; F.lin[f] = a.lin; F.mn[f] = a.mn; F.mx[f] = a.mx;
     }
     const bool staged = stageable(it, field_bytes(fdtype)) &&
-                        !few_fields(fdtype, math, post, (long)it.nx * it.ny * it.nz, nf);
+                        !few_fields(fdtype, math, post, (long)it.nx * it.ny * it.nz, nf, false);
     void* kern = pick<false>(fdtype, pdtype, math, post, staged ? 7 : 2);
     if (staged) {  // k_hlt5: LDS-staged boxes, an eighth of the tile list per XCD
       long ntiles = item_ptiles(it.nx, it.ny, it.nz, hlt_order(post), kTI, kHltTH, kHltTL);
