@@ -148,14 +148,16 @@ __global__ void k_prep_arr(S* __restrict__ uarr, S* __restrict__ varr, S* __rest
 // adz_traject.F90:66-104: niter fixed-point updates of one arrival point (i,j,k) per lane.
 //
 // A block takes a tile of tw x tr points, at most 256, on kTrajLevels levels (four waves per
-// level; 64 x 4 on wide grids, see traj_tile) and copies the box of the derived winds (three interleaved components) that its points read
-// into LDS; every iteration reduces the box it needs over the block and stages a new one only
-// where that leaves the one in LDS, which has a margin of one element on every side where that
-// fits.  The stencil of a point is 192 values, of which the lanes of a tile read few that
+// level; 64 x 4 on wide grids, see traj_tile) and copies the box of the derived winds (three
+// interleaved components) that its points read into LDS; every iteration reduces the box it needs
+// over the block and stages a new one only where that leaves the one in LDS, which has a margin of
+// one element on every side where that fits.  The stencil of a point is 192 values, of which the lanes of a tile read few that
 // differ; as per-lane loads they were 48 16-byte loads per lane and iteration.
 // Rows of the box begin kWindPitch elements apart (a row is one 1 KB DMA instruction of a
 // wave, two in FP64): lanes are three words apart, free of bank conflicts, and rows a multiple
 // of the banks.  A tile whose box does not fit reads per lane, in the same arithmetic and order.
+// FLAT (tw = 0): blocks of 256 points in the order of the arrays, which fill their lanes in rows
+// of any length, and every lane reads for itself.
 //
 // What bounds it: FP64 arithmetic.  1024 x 512 x 84 points, three iterations: 4.5 ms as
 // per-lane loads with 70 % of the cycles issuing vector instructions (880 per iteration, 192
@@ -199,26 +201,35 @@ __device__ __forceinline__ void tricub3_steps(Read read, const double* c, double
   }
 }
 
-template <class S>
-__global__ __launch_bounds__(64 * kTrajWaves, sizeof(S) == 4 ? 4 : 2) void k_traject(
+template <class S, bool FLAT>
+__global__ __launch_bounds__(FLAT ? 256 : 64 * kTrajWaves, FLAT ? 1 : sizeof(S) == 4 ? 4 : 2) void k_traject(
     S* __restrict__ pxyzm, double* __restrict__ wpxyz, S* __restrict__ uvw_dep, S* __restrict__ pm,
     const S* __restrict__ uvw_d, const S* __restrict__ uarr, const S* __restrict__ varr, const S* __restrict__ warr, ZtabDev lv, TrajParams P,
     int niter, double dtA, double dtD, double dtzA, double dtzD, unsigned tw, unsigned tr) {
-  __shared__ __attribute__((aligned(16))) S box[kTrajRows * kWindPitch];
+  __shared__ __attribute__((aligned(16))) S box[FLAT ? 4 : kTrajRows * kWindPitch];
   __shared__ int red[18], moved[3];
-  if (threadIdx.x < 18) red[threadIdx.x] = kFar;
-  if (threadIdx.x < 3) moved[threadIdx.x] = 0;
-  __syncthreads();
-  const unsigned nbi = (P.ni + tw - 1) / tw, nbj = (P.nj + tr - 1) / tr;
-  const unsigned nbk = (P.nk - P.k00 + kTrajLevels) / kTrajLevels;
-  const long ntiles = (long)nbi * nbj * nbk, t = tile_of_block(ntiles, 1);
-  if (t >= ntiles) return;  // the whole block leaves: no barrier is reached
   const unsigned lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const unsigned tk = (unsigned)(t / ((long)nbi * nbj)), tij = (unsigned)(t - (long)tk * nbi * nbj);
-  const unsigned tj = tij / nbi, ti = tij - tj * nbi;
-  const unsigned l = threadIdx.x & 255, lj = l / tw, li = l - lj * tw;
-  const int i = (int)(tw * ti + li) + 1, j = (int)(tr * tj + lj) + 1, k = (int)(kTrajLevels * tk + wv / 4) + P.k00;
-  const bool valid = lj < tr && i <= P.ni && j <= P.nj && k <= P.nk;
+  int i, j, k;
+  bool valid;
+  if constexpr (FLAT) {
+    const unsigned a = blockIdx.x * 256 + threadIdx.x, nxy = (unsigned)P.ni * (unsigned)P.nj;
+    const unsigned kq = a / nxy, rem = a - kq * nxy, jq = rem / (unsigned)P.ni;
+    i = (int)(rem - jq * (unsigned)P.ni) + 1; j = (int)jq + 1; k = (int)kq + P.k00;
+    valid = k <= P.nk;
+  } else {
+    if (threadIdx.x < 18) red[threadIdx.x] = kFar;
+    if (threadIdx.x < 3) moved[threadIdx.x] = 0;
+    __syncthreads();
+    const unsigned nbi = (P.ni + tw - 1) / tw, nbj = (P.nj + tr - 1) / tr;
+    const unsigned nbk = (P.nk - P.k00 + kTrajLevels) / kTrajLevels;
+    const long ntiles = (long)nbi * nbj * nbk, t = tile_of_block(ntiles, 1);
+    if (t >= ntiles) return;  // the whole block leaves: no barrier is reached
+    const unsigned tk = (unsigned)(t / ((long)nbi * nbj)), tij = (unsigned)(t - (long)tk * nbi * nbj);
+    const unsigned tj = tij / nbi, ti = tij - tj * nbi;
+    const unsigned l = threadIdx.x & 255, lj = l / tw, li = l - lj * tw;
+    i = (int)(tw * ti + li) + 1; j = (int)(tr * tj + lj) + 1; k = (int)(kTrajLevels * tk + wv / 4) + P.k00;
+    valid = lj < tr && i <= P.ni && j <= P.nj && k <= P.nk;
+  }
   S px = (S)0, py = (S)0, pz = (S)0;
   S ua = (S)0, va = (S)0, wa = (S)0;
   if (valid) {
@@ -235,55 +246,59 @@ __global__ __launch_bounds__(64 * kTrajWaves, sizeof(S) == 4 ? 4 : 2) void k_tra
     Index x;
     const bool ok = valid && index_step((double)px, (double)py, (double)pz, lv, &x);
     const int pz1 = x.pz + (x.zlinear ? 1 : 3);
-    const bool out = ok && (x.ix - 1 < bx0 || x.ix + 2 > bx1 || x.iy - 1 < by0 || x.iy + 2 > by1 || x.pz < bz0 || pz1 > bz1);
-    // does any lane of the block need a new box?  (Word it % 3 tells; the barrier also says
-    // that every wave is done with the old one.)
-    if (__ballot(out) != 0 && lane == 0) moved[it % 3] = 1;
-    if (threadIdx.x == 0) moved[(it + 1) % 3] = 0;
-    __syncthreads();
-    bool staged = true;
-    if (__builtin_amdgcn_readfirstlane(moved[it % 3])) {
-      int ext[6] = {ok ? x.ix - 1 : kFar, ok ? -(x.ix + 2) : kFar, ok ? x.iy - 1 : kFar, ok ? -(x.iy + 2) : kFar,
-                    ok ? x.pz : kFar, ok ? -pz1 : kFar};
-      tile_min6(ext, red, boxes++);
-      const int x0 = ext[0], x1 = -ext[1], y0 = ext[2], y1 = -ext[3], z0 = ext[4], z1 = -ext[5];
-      const int mx0 = max(x0 - 1, lv.ilo), mx1 = min(x1 + 1, lv.ihi), my0 = max(y0 - 1, lv.jlo),
-                my1 = min(y1 + 1, lv.jhi), mz0 = max(z0 - 1, 0), mz1 = min(z1 + 1, lv.nk - 1);
-      const int cols = kWindPitch / 3;
-      const bool roomy = (my1 - my0 + 1) * (mz1 - mz0 + 1) <= kTrajRows && mx1 - mx0 + 1 <= cols;
-      if (roomy) { bx0 = mx0; bx1 = mx1; by0 = my0; by1 = my1; bz0 = mz0; bz1 = mz1; }
-      else { bx0 = x0; bx1 = x1; by0 = y0; by1 = y1; bz0 = z0; bz1 = z1; }
-      const int nyb = by1 - by0 + 1, nzb = bz1 - bz0 + 1;
-      const long n3 = 3L * lv.ni * (long)sizeof(S), nij3 = 3L * lv.nij * (long)sizeof(S);  // bytes of a row, of a plane
-      staged = bx1 - bx0 < cols && (long)nyb * nzb <= kTrajRows && n3 * nyb + nij3 * nzb < 0x7fff0000L;
-      if (staged) {
-        const char* b0 = (const char*)(f3 + 3 * ((bx0 - 1) + (long)(by0 - 1) * lv.ni + (long)bz0 * lv.nij));
-        const long left = (const char*)(uvw_d + 3L * P.nij * P.nk) + 16 - b0;  // (the array ends in 16 spare bytes)
-        const __amdgpu_buffer_rsrc_t rs = field_rsrc(b0, (unsigned)min(left, 0x7fff0000L));
-        const int quads = (3 * (bx1 - bx0 + 1) * (int)sizeof(S) + 15) / 16;
-        constexpr int kI = kWindPitch * (int)sizeof(S) / 1024;  // DMA instructions per row
-        for (int r = wv; r < nyb * nzb; r += kTrajWaves) {
-          const int zz = r / nyb, yy = r - zz * nyb;
-          const int off = yy * (int)n3 + zz * (int)nij3;
-#pragma unroll
-          for (int h = 0; h < kI; h++) {
-            const int q = 64 * h + (int)lane;
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                rs, (__attribute__((address_space(3))) void*)(box + r * kWindPitch + h * (1024 / (int)sizeof(S))), 16,
-                q < quads ? off + 16 * q : 0x7fff0000, 0, 0, 0);
+    bool staged = !FLAT;
+    if constexpr (!FLAT) {
+      const bool out = ok && (x.ix - 1 < bx0 || x.ix + 2 > bx1 || x.iy - 1 < by0 || x.iy + 2 > by1 || x.pz < bz0 || pz1 > bz1);
+      // does any lane of the block need a new box?  (Word it % 3 tells; the barrier also says
+      // that every wave is done with the old one.)
+      if (__ballot(out) != 0 && lane == 0) moved[it % 3] = 1;
+      if (threadIdx.x == 0) moved[(it + 1) % 3] = 0;
+      __syncthreads();
+      if (__builtin_amdgcn_readfirstlane(moved[it % 3])) {
+        int ext[6] = {ok ? x.ix - 1 : kFar, ok ? -(x.ix + 2) : kFar, ok ? x.iy - 1 : kFar, ok ? -(x.iy + 2) : kFar,
+                      ok ? x.pz : kFar, ok ? -pz1 : kFar};
+        tile_min6(ext, red, boxes++);
+        const int x0 = ext[0], x1 = -ext[1], y0 = ext[2], y1 = -ext[3], z0 = ext[4], z1 = -ext[5];
+        const int mx0 = max(x0 - 1, lv.ilo), mx1 = min(x1 + 1, lv.ihi), my0 = max(y0 - 1, lv.jlo),
+                  my1 = min(y1 + 1, lv.jhi), mz0 = max(z0 - 1, 0), mz1 = min(z1 + 1, lv.nk - 1);
+        const int cols = kWindPitch / 3;
+        const bool roomy = (my1 - my0 + 1) * (mz1 - mz0 + 1) <= kTrajRows && mx1 - mx0 + 1 <= cols;
+        if (roomy) { bx0 = mx0; bx1 = mx1; by0 = my0; by1 = my1; bz0 = mz0; bz1 = mz1; }
+        else { bx0 = x0; bx1 = x1; by0 = y0; by1 = y1; bz0 = z0; bz1 = z1; }
+        const int nyb = by1 - by0 + 1, nzb = bz1 - bz0 + 1;
+        const long n3 = 3L * lv.ni * (long)sizeof(S), nij3 = 3L * lv.nij * (long)sizeof(S);  // bytes of a row, of a plane
+        staged = bx1 - bx0 < cols && (long)nyb * nzb <= kTrajRows && n3 * nyb + nij3 * nzb < 0x7fff0000L;
+        if (staged) {
+          const char* b0 = (const char*)(f3 + 3 * ((bx0 - 1) + (long)(by0 - 1) * lv.ni + (long)bz0 * lv.nij));
+          const long left = (const char*)(uvw_d + 3L * P.nij * P.nk) + 16 - b0;  // (the array ends in 16 spare bytes)
+          const __amdgpu_buffer_rsrc_t rs = field_rsrc(b0, (unsigned)min(left, 0x7fff0000L));
+          const int quads = (3 * (bx1 - bx0 + 1) * (int)sizeof(S) + 15) / 16;
+          constexpr int kI = kWindPitch * (int)sizeof(S) / 1024;  // DMA instructions per row
+          for (int r = wv; r < nyb * nzb; r += kTrajWaves) {
+            const int zz = r / nyb, yy = r - zz * nyb;
+            const int off = yy * (int)n3 + zz * (int)nij3;
+  #pragma unroll
+            for (int h = 0; h < kI; h++) {
+              const int q = 64 * h + (int)lane;
+              __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                  rs, (__attribute__((address_space(3))) void*)(box + r * kWindPitch + h * (1024 / (int)sizeof(S))), 16,
+                  q < quads ? off + 16 * q : 0x7fff0000, 0, 0, 0);
+            }
           }
+          __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+          __syncthreads();
+        } else {
+          bx0 = kFar;  // nothing in LDS
         }
-        __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
-        __syncthreads();
-      } else {
-        bx0 = kFar;  // nothing in LDS
       }
     }
     double w3[3] = {__builtin_nan(""), __builtin_nan(""), __builtin_nan("")};
     if (ok) {
       double c[20];
       weights_ref(x, lv, c);
-      if (staged) {
+      if constexpr (FLAT) {
+        tricub3_ref<S>(f3 + 3 * x.off, c, 3L * lv.ni, 3L * lv.nij, x.zlinear, w3);
+      } else if (staged) {
         const int nyb = by1 - by0 + 1;
         const int b = ((x.iy - 1 - by0) + nyb * (x.pz - bz0)) * kWindPitch + 3 * (x.ix - 1 - bx0);
         const int o1 = x.zlinear ? 0 : nyb * kWindPitch, o2 = o1 + nyb * kWindPitch, o3 = o2 + o1;
@@ -356,8 +371,8 @@ __global__ void k_inittraj(S* __restrict__ pxyzm, double* __restrict__ wpxyz, Tr
 // Positions of the u and v grids (Adz_pmu, Adz_pmv: adz_interp_traj.F90:45-78) and of the
 // thermodynamic levels (Adz_pb: :80-174, and its part Adz_pt: :176-181) from the FP64 history
 // W, in one pass over it.  A lane takes kc consecutive levels of one column, the four levels of
-// the vertical stencil passing through its registers; a block's 64 columns by 4 rows share the
-// horizontal stencils in the first-level cache.
+// the vertical stencil passing through its registers; a block's 64 columns by 4 rows (fewer columns
+// by more rows where rows are short) share the horizontal stencils in the first-level cache.
 //
 // What bounds it: memory, 88 bytes of history, winds and positions per point at 2.8 TB/s, in
 // nine streams.  1024 x 512 x 84: 1.22 ms in one kernel (1.26 with an eighth of the tiles per
@@ -367,12 +382,13 @@ template <class S>
 __global__ __launch_bounds__(256) void k_sets(S* __restrict__ pmu, S* __restrict__ pmv, S* __restrict__ pb,
                                               S* __restrict__ pt, const double* __restrict__ W,
                                               const S* __restrict__ uvw_dep, const float* __restrict__ zdt0,
-                                              TrajParams P, double dtzD, double dtzA, int kc) {
-  const unsigned nbi = (P.ni + 63) / 64, nbj = (P.nj + 3) / 4, nbk = (P.nk + kc - 1) / kc;
+                                              TrajParams P, double dtzD, double dtzA, int kc, int ltw) {
+  const unsigned tw = 1u << ltw, tr = 256u >> ltw;  // columns and rows of a tile
+  const unsigned nbi = (P.ni + tw - 1) >> ltw, nbj = (P.nj + tr - 1) / tr, nbk = (P.nk + kc - 1) / kc;
   const long ntiles = (long)nbi * nbj * nbk, t = tile_of_block(ntiles, 0);
   if (t >= ntiles) return;
   const unsigned tk = (unsigned)(t / ((long)nbi * nbj)), tij = (unsigned)(t - (long)tk * nbi * nbj), tj = tij / nbi;
-  const int i = (int)(64 * (tij - tj * nbi) + (threadIdx.x & 63)) + 1, j = (int)(4 * tj + (threadIdx.x >> 6)) + 1;
+  const int i = (int)(tw * (tij - tj * nbi) + (threadIdx.x & (tw - 1))) + 1, j = (int)(tr * tj + (threadIdx.x >> ltw)) + 1;
   if (i > P.ni || j > P.nj) return;
   const int nk = P.nk, k1 = (int)tk * kc + 1, k2 = min(nk, k1 + kc - 1), kstart = max(P.k00i, 2);
   const bool onu = i >= P.i0u && i <= P.inu && j >= P.j0 && j <= P.jn;
@@ -505,7 +521,14 @@ void free_ctx(adz_ctx* c) {
 // as many rows as 256 lanes hold (at most 8, for the box), the one that leaves the fewest lanes
 // without a point.  (65 x 103 x 49, cold: 109 us per lane, 176 with tiles of 64 x 4 and a
 // whole tile for the last column, 112 with 33 x 7; 200 x 150 x 60, cold: 466 and 425.)
+// Rows of fewer than kFlatRow points would leave a quarter of the lanes and more without one, and
+// are taken flat.  The whole call, flat (in tiles), us: 8 x 800 x 60 115 (177), 16 x 800 x 60 159
+// (192), 20 x 600 x 60 143 (158), 24 x 600 x 60 164 (161); in FP64 170 (241), 244 (258), 219 (238),
+// 240 (243).
+constexpr int kFlatRow = 24;
 void traj_tile(int ni, int nj, unsigned* tw, unsigned* tr) {
+  *tw = *tr = 0;
+  if (ni < kFlatRow) return;
   long best = -1;
   for (int nt = (ni + 63) / 64; nt == (ni + 63) / 64 || (ni + nt - 1) / nt >= 32; nt++) {
     const int w = (ni + nt - 1) / nt, r = std::min(8, 256 / w);
@@ -530,16 +553,23 @@ int run_traject(adz_ctx* c, double dt, int advec, double bA_m, double bA, const 
   hipLaunchKernelGGL(k_prep_arr<S>, dim3(nb((long)P.ni * P.nj), std::min(P.nk, kMaxGridY)), dim3(256), 0, st, arr, arr + nint, arr + 2 * nint, ut0, vt0, zdt0, P);
   unsigned tw, tr;
   traj_tile(P.ni, P.nj, &tw, &tr);
-  const long tiles = (long)((P.ni + tw - 1) / tw) * ((P.nj + tr - 1) / tr) * ((P.nk - P.k00 + kTrajLevels) / kTrajLevels);
-  hipLaunchKernelGGL(k_traject<S>, tile_grid(tiles), dim3(64 * kTrajWaves), 0, st, (S*)c->pxyzm, c->wpxyz, (S*)c->uvw_dep,
-                     (S*)c->pm, (const S*)c->uvw_d, arr, arr + nint, arr + 2 * nint, c->zq->dev, P, c->niter, dtA, dtD, dtzA,
-                     dtzD, tw, tr);
+  const long points = (long)P.ni * P.nj * (P.nk - P.k00 + 1);
+  const long tiles =
+      tw ? (long)((P.ni + tw - 1) / tw) * ((P.nj + tr - 1) / tr) * ((P.nk - P.k00 + kTrajLevels) / kTrajLevels) : 0;
+  hipLaunchKernelGGL((tw ? k_traject<S, false> : k_traject<S, true>), tw ? tile_grid(tiles) : dim3(nb(points)),
+                     dim3(tw ? 64 * kTrajWaves : 256), 0, st, (S*)c->pxyzm, c->wpxyz, (S*)c->uvw_dep, (S*)c->pm,
+                     (const S*)c->uvw_d, arr, arr + nint, arr + 2 * nint, c->zq->dev, P, c->niter, dtA, dtD, dtzA, dtzD, tw,
+                     tr);
   c->niter = c->itraj;  // adz_traject.F90:120
   // levels per lane: as many as leave eight waves for every SIMD, at most 8
-  const long cols = (long)((P.ni + 63) / 64) * ((P.nj + 3) / 4);
+  // columns of a tile of k_sets: 64; in rows of up to 32 points as many as there are, rounded up (the
+  // call on 8 x 800 x 60 points 115 -> 80 us, 16 x 800 x 60 159 -> 138)
+  int ltw = 6;
+  while (ltw > 3 && P.ni <= (1 << (ltw - 1))) ltw--;
+  const long cols = (long)((P.ni + (1 << ltw) - 1) >> ltw) * ((P.nj + (256 >> ltw) - 1) / (256 >> ltw));
   const int kc = (int)std::min(8L, std::max(1L, cols * 4 * P.nk / (8 * 1024)));
   hipLaunchKernelGGL(k_sets<S>, tile_grid(cols * ((P.nk + kc - 1) / kc)), dim3(256), 0, st, (S*)c->pmu, (S*)c->pmv,
-                     (S*)c->pb, (S*)c->pt, c->wpxyz, (const S*)c->uvw_dep, zdt0, P, dtzD, dtzA, kc);
+                     (S*)c->pb, (S*)c->pt, c->wpxyz, (const S*)c->uvw_dep, zdt0, P, dtzD, dtzA, kc, ltw);
   ADZ_HIP_CHECK(hipGetLastError());
   return ADZ_OK;
 }
