@@ -30,9 +30,9 @@
 // Why every wait ends: the list order is a topological order of the waits, and an entry is
 // taken from the ticket counter only by a wave that is running, so the first entry not yet
 // visited is always held by a running wave that waits for nothing.  The waits are bounded all
-// the same: one that gives up raises a flag, every wave stops before its next window, and
-// k_il_finish visits what is left in list order with one wave, so the result is exact in
-// either case.
+// the same: one that gives up raises a flag and ends its wave, as does every wait that sees the
+// flag; windows whose waits are over are still visited, and k_il_finish visits what is left in
+// list order with one wave, so the result is exact in either case.
 //
 // The wave holds its window's surroundings, (4 + 2S) x (2S+1) x (2S+1) cells, in LDS: f, its
 // bounds and the air mass.  For each visit the lanes form the cube's masses, every lane adds
@@ -66,7 +66,8 @@ constexpr int kIlBlock = 256;
 constexpr int kIlScan = 1024;
 constexpr int kIlWin = 4;          // cells of a row per piece of work
 constexpr uint64_t kIlMask = (1ull << kIlWin) - 1;
-constexpr int kIlWaves = 512;      // most waves of the visiting launch
+constexpr int kIlWaves = 512;      // waves of the visiting launch
+constexpr int kIlFew = 128;        // those of them per tracer that visit in any case
 constexpr int kIlSpin = 1 << 22;   // polls of one wait (about 1 us each) before it gives up
 
 struct IlmcTr {
@@ -450,7 +451,12 @@ __device__ __forceinline__ int il_visit(const IlmcArgs& A, const IlmcTr& T, cons
 }
 
 // The visits: single-wave blocks take windows from the ticket counter until none is left or
-// a wait gave up.
+// a wait gave up.  128 waves per tracer, and where that is more, three for every window that the
+// values of t have on average, as many as their order lets run at a time; others would only poll.
+// ms, with 128 (256, 512, 1024) waves: two tracers of 384 x 288 x 84 with a front 7.3 (7.6, 8.0,
+// 8.7), one of 100 x 80 x 40 with 30 % of the cells out of bounds 2.2 (1.9, 3.3, 3.9), one of
+// 512 x 384 x 84 with 2 % 9.1 (4.8, 3.5, 4.2), with 30 % 98 (50, 34, 35; 61 as a launch per
+// hyperplane).
 template <int S, bool AB>
 __global__ __launch_bounds__(64) void k_il_visit(IlmcArgs A) {
   __shared__ IlBox<S, AB> L;
@@ -459,6 +465,7 @@ __global__ __launch_bounds__(64) void k_il_visit(IlmcArgs A) {
   K.init();
   const int lane = threadIdx.x;
   const long long total = A.off[A.nplanes];
+  if (blockIdx.x >= (long long)kIlFew * A.ntr && blockIdx.x >= 3 * total / A.nplanes) return;
   for (;;) {
     // through LDS and barriers: a readfirstlane here would hang on where the lanes reconverge
     // after the branches on lane 0
@@ -554,15 +561,14 @@ using namespace adz;
 struct adz_ilmc {
   IlmcArgs a;
   int sweep_max, autobar, min_max;
-  int visit_blocks;
   void* mem;
 };
 
 namespace {
 
 template <int S, bool AB>
-void launch_visits(const IlmcArgs& a, int blocks, int reset, hipStream_t st) {
-  hipLaunchKernelGGL((k_il_visit<S, AB>), dim3(blocks), dim3(64), 0, st, a);
+void launch_visits(const IlmcArgs& a, int reset, hipStream_t st) {
+  hipLaunchKernelGGL((k_il_visit<S, AB>), dim3(kIlWaves), dim3(64), 0, st, a);
   hipLaunchKernelGGL((k_il_finish<S, AB>), dim3(kIlWaves), dim3(64), 0, st, a, reset);
 }
 
@@ -579,8 +585,8 @@ int adz_ilmc_create(const adz_ilmc_tracer* tr, int ntr, const adz_ilmc_domain* d
   if (d.sweep_max < 1 || d.sweep_max > 4)
     return fail(ADZ_EINVAL, "adz_ilmc_create: ILMC_sweep_max must be 1..4 (the sweep arrays hold 400 cells)");
   const int ni = d.in - d.i0 + 1, nj = d.jn - d.j0 + 1, nkk = d.nk - d.k0 + 1;
-  // cell offsets are packed in 16 + 16 + 12 bits, tracers in the remaining 20; the row
-  // kernels launch one 256-lane block per row of the domain (at most 2^32 lanes)
+  // window and row offsets are packed in 16 bits each, levels in 12, tracers in the remaining 20;
+  // k_il_mark launches a 256-lane block for every few rows of the domain (at most 2^32 lanes)
   if (ni > 65535 || nj > 65535 || nkk > 4095 || ntr > 65535 || (long)nj * nkk > (1L << 24))
     return fail(ADZ_EINVAL, "adz_ilmc_create: domain or tracer count too large");
   std::vector<IlmcTr> h(ntr);
@@ -624,10 +630,6 @@ int adz_ilmc_create(const adz_ilmc_tracer* tr, int ntr, const adz_ilmc_domain* d
   adz_ilmc* r = new adz_ilmc;
   r->a = a;
   r->sweep_max = d.sweep_max; r->autobar = d.autobar != 0; r->min_max = d.min_max != 0;
-  // waves: 128 per tracer, as many as its chains of visits keep busy.  More only poll: the
-  // call on two tracers of 384 x 288 x 84 took 4.9 ms (dense front: 9.8) with 128 waves in
-  // all, 4.9 (7.9) with 256, 5.5 (12.0) with 512, 6.4 (14.0) with 1024
-  r->visit_blocks = (int)std::min((long)kIlWaves, 128L * ntr);
   r->mem = mem;
   *out = r;
   return ADZ_OK;
@@ -648,16 +650,16 @@ int adz_ilmc_lam(adz_ilmc* il, const void* air_m, long long* counts, adz_stream 
   hipLaunchKernelGGL(k_il_scan, dim3(1), dim3(kIlScan), 0, st, a);
   hipLaunchKernelGGL(k_il_fill, dim3((unsigned)(((long)nrows * a.wpr + kIlBlock - 1) / kIlBlock), (unsigned)a.ntr),
                      dim3(kIlBlock), 0, st, a);
-  const int nb = il->visit_blocks, reset = il->min_max;
+  const int reset = il->min_max;
   switch (il->sweep_max * 2 + il->autobar) {
-    case 2: launch_visits<1, false>(a, nb, reset, st); break;
-    case 3: launch_visits<1, true>(a, nb, reset, st); break;
-    case 4: launch_visits<2, false>(a, nb, reset, st); break;
-    case 5: launch_visits<2, true>(a, nb, reset, st); break;
-    case 6: launch_visits<3, false>(a, nb, reset, st); break;
-    case 7: launch_visits<3, true>(a, nb, reset, st); break;
-    case 8: launch_visits<4, false>(a, nb, reset, st); break;
-    default: launch_visits<4, true>(a, nb, reset, st); break;
+    case 2: launch_visits<1, false>(a, reset, st); break;
+    case 3: launch_visits<1, true>(a, reset, st); break;
+    case 4: launch_visits<2, false>(a, reset, st); break;
+    case 5: launch_visits<2, true>(a, reset, st); break;
+    case 6: launch_visits<3, false>(a, reset, st); break;
+    case 7: launch_visits<3, true>(a, reset, st); break;
+    case 8: launch_visits<4, false>(a, reset, st); break;
+    default: launch_visits<4, true>(a, reset, st); break;
   }
   ADZ_HIP_CHECK(hipGetLastError());
   return ADZ_OK;
