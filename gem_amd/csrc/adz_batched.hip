@@ -1085,6 +1085,9 @@ template <class TF, int W, int S> constexpr int dma_per_wave() { return (box_dma
 template <class TF, int W, int S> constexpr int box_elems() { return box_dma<TF, W, S>() * 1024 / (int)sizeof(TF); }
 static_assert(box_rows<float, 8, 4>() < 128 && box_rows<double, 8, 4>() < 128, "row split by a float reciprocal below");
 
+// What may pass a scheduling barrier that keeps memory operations in order: arithmetic alone.
+constexpr int kNoMemory = 0x40f;
+
 // s_waitcnt immediate (gfx9): at most n vector-memory operations outstanding, the other
 // counters not waited for
 constexpr int vmcnt_imm(int n) { return (n & 15) | (7 << 4) | (15 << 8) | ((n >> 4) << 14); }
@@ -1352,13 +1355,16 @@ __device__ __forceinline__ void dma_tile(const DevItem& it, const Fields& F, lon
   // wave's vector-memory operations retire in order, and every field adds its loads and then
   // kSt stores, so at the wait for field f only the stores of field f - 1 may be outstanding:
   // no wave waits for its stores.  (The first field has none before it: as many, out of range
-  // and therefore dropped, keep the count.)
+  // and therefore dropped, keep the count.)  The count is right only while no store is issued
+  // before the loads that precede it here: the scheduling barriers keep the compiler from moving
+  // one there.
   Ptr P;
   auto step = [&](int f, const TF* cur, TF* next) {
     __builtin_amdgcn_s_waitcnt(vmcnt_imm(kSt));
     __syncthreads();  // every wave's part of field f has landed, and nobody reads `next` any more
     const int half = half_of(SZ == 2 ? F.s(f) : nullptr);
     issue(P.s, f + 1 < f1, next);
+    __builtin_amdgcn_sched_barrier(kNoMemory);
     eval(P, half, cur);
     source(f + 2, &P);
     target(f + 1, &P);
@@ -1366,6 +1372,7 @@ __device__ __forceinline__ void dma_tile(const DevItem& it, const Fields& F, lon
   source(f0, &P);
   target(f0, &P);
   issue(P.s, true, boxA);
+  __builtin_amdgcn_sched_barrier(kNoMemory);
   {
     const __amdgpu_buffer_rsrc_t none = field_rsrc(P.d, 0u);
 #pragma unroll
