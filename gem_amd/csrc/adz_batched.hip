@@ -1759,6 +1759,11 @@ int tile_levels(int stage) { return stage == 7 ? 2 : stage == 8 ? 4 : 1; }
 unsigned plan_threads(int stage) {
   return stage == 3 ? kPCThreads : stage == 6 || stage == 7 ? 512 : stage == 8 ? 1024 : kTile;
 }
+// does a plan of this staging launch a block per tile (blocks_per_cu has no effect)?
+bool block_per_tile(int stage, int fdtype) {
+  const int rs = run_stage(stage, fdtype);
+  return rs >= 5 && one_tile(plan_threads(rs) / 64);
+}
 
 int device_cus() {
   static int cus = 0;
@@ -1912,7 +1917,8 @@ int adz_plan_execute(const adz_plan* p, adz_stream stream) {
   PlanArgs a = p->args;
   void* args[] = {&a};
   const unsigned nthr = plan_threads(rs);
-  ADZ_HIP_CHECK(hipLaunchKernel(kern, rs >= 5 && one_tile(nthr / 64) ? tile_grid(a.ntiles) : dim3(p->grid), dim3(nthr), args, 0, (hipStream_t)stream));
+  const dim3 grid = block_per_tile(p->tune.stage, p->fdtype) ? tile_grid(a.ntiles) : dim3(p->grid);
+  ADZ_HIP_CHECK(hipLaunchKernel(kern, grid, dim3(nthr), args, 0, (hipStream_t)stream));
   return ADZ_OK;
 }
 
@@ -1981,13 +1987,14 @@ int adz_plan_autotune(const adz_item* items, int nitems, int fdtype, int math, i
   const int nst = (fdtype == ADZ_F32 ? 8 : 6) - (math != ADZ_MATH_F32), nor = 7;
   // staging and tile order together first: the LDS-staged forms depend on the L2 reuse the
   // tile order gives, so one is not searched at the other's best value.  Each staging is
-  // timed at 4 blocks per CU, blocks of 16 waves at 1 (one of them is resident per CU).
+  // timed at 4 blocks per CU, blocks of 16 waves at 1 (one of them is resident per CU), those
+  // with a block per tile at the built-in 8, which they don't use.
   for (int s = 0; s < nst && rc == ADZ_OK; s++)
     for (int v = 0; v < nor && rc == ADZ_OK; v++) {
       adz_tune t = cur;
       t.stage = stages[s];
       t.level_inner = orders[v];
-      t.blocks_per_cu = plan_threads(run_stage(t.stage, fdtype)) >= 1024 ? 1 : 4;
+      t.blocks_per_cu = block_per_tile(t.stage, fdtype) ? 8 : plan_threads(run_stage(t.stage, fdtype)) >= 1024 ? 1 : 4;
       if (t.stage == cur.stage && t.level_inner == cur.level_inner && t.blocks_per_cu == cur.blocks_per_cu) continue;
       float ms = 0.f;
       rc = time_one(t, &ms);
@@ -1998,6 +2005,7 @@ int adz_plan_autotune(const adz_item* items, int nitems, int fdtype, int math, i
   const int coords[] = {2, 1, 3, 4, 5};
   for (int ci = 0; ci < 5 && rc == ADZ_OK; ci++) {
     const int coord = coords[ci];
+    if (coord == 3 && block_per_tile(cur.stage, fdtype)) continue;
     const int* vals = coord == 1 ? orders : coord == 2 ? fpps : coord == 3 ? bpcs : flags;
     int nv = coord == 1 ? nor : coord == 2 ? 11 : coord == 3 ? 6 : 2;
     for (int v = 0; v < nv && rc == ADZ_OK; v++) {
