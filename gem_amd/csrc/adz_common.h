@@ -189,11 +189,11 @@ __device__ __forceinline__ void weights_f32(const Index& x, const ZtabDev& lv, f
 // rows folded by fma, and the x stage accumulated column by column with fma
 // (Tricublin_zyxf3_inline AVX2 path, turbo_tricublin.c:1142-1257).  f points at the
 // stencil corner; ni3/nij3 are the element strides of a row / plane (3*ni, 3*nij).
-template <class TF, class I>
-__device__ __forceinline__ void tricub3_ref(const TF* __restrict__ f, const double* c, I ni3, I nij3,
+template <class TF>
+__device__ __forceinline__ void tricub3_ref(const TF* __restrict__ f, const double* c, long ni3, long nij3,
                                             int zlinear, double* out) {
-  const I o1 = zlinear ? 0 : nij3;
-  const I o2 = o1 + nij3, o3 = o2 + o1;
+  const long o1 = zlinear ? 0 : nij3;
+  const long o2 = o1 + nij3, o3 = o2 + o1;
   // rows outer, the 12 interleaved values of a row inner: only one row's values and the
   // 12 running sums are live at a time (each element keeps the same operation order)
   double dst[12];
