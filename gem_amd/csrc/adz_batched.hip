@@ -1050,7 +1050,9 @@ __device__ __forceinline__ void shared_tile(const DevItem& it, const Fields& F, 
 // What bounds it: 6 FP32 fields, no lin/min/max (stage 7): LDS reads (256 B per point-field),
 // FP32 arithmetic (100 instructions per field and 40 per field for the tile's indexes, weights
 // and box) and the texture unit's DMA, 58, 54 and 41 % of the cycles with 16 waves per CU,
-// none hidden completely behind another; with 24 waves 0.85 of that time.
+// none hidden completely behind another; with 24 waves 0.85 of that time.  20 fields with lin/min/max
+// of 2048 x 1024 x 84, ten at a time: vector instructions, 87 % of the cycles (201 per point-field);
+// LDS 58 %, 3.9 TB/s of HBM traffic, 1.2 bytes written for each byte of output.
 
 // elements per LDS row: whole rounds of the 32 banks
 template <class TF> constexpr int box_pitch() { return sizeof(TF) == 8 ? 80 : sizeof(TF) == 4 ? 96 : 128; }
@@ -1508,8 +1510,8 @@ __global__ __launch_bounds__(kTile) void k_hlt(DevItem it, InlineFields F) {
 // tile list.  One tile per block: the hardware fills a CU with the next ones as blocks end.
 // Measured against 64 x 8 x 1 tiles with 62 rows per box, where a third of the tiles of a
 // 200 x 150 grid and four fifths of a 512 x 384 one fitted: 3 fields of 200 x 150 x 60 in the
-// reference's arithmetic 63.7 -> 54.8 us; in FP32, 4 fields of 512 x 384 x 84 681 -> 550 us,
-// 8 of 2048 x 1024 x 84 13.4 -> 8.2 ms.
+// reference's arithmetic 63.7 -> 46.7 us; in FP32, 4 fields of 512 x 384 x 84 681 -> 399 us,
+// 8 of 2048 x 1024 x 84 13.4 -> 7.0 ms.
 // Tile order: super-columns of three tile rows, which read a source plane again while it is in
 // an XCD's L2; rows, then levels, where lin/min/max are stored, whose streams prefer it.  us,
 // super-columns (rows): 512 x 384 x 84, smooth positions, 4 FP64 fields 705 (735), 4 FP32 419
@@ -1688,17 +1690,18 @@ int field_bytes(int fdtype) { return fdtype == ADZ_F64 ? 8 : fdtype == ADZ_F32 ?
 // One field, which does not pay for a tile's extents and its first box?  By what was measured, us,
 // per-lane loads (staged boxes) of one field of 304 x 227 x 84, 512 x 384 x 84 and 1024 x 512 x 84;
 // two fields of 304 x 227 x 84 and more gain by staging in every form.  The call / a plan:
-//   FP32 arithmetic              61 (73), 198 (213), 535 (574)     / 64 (78), 201 (233), 560 (631)
-//     clipped                    61 (74), 204 (214), 546 (579)     / 68 (78), 213 (228), 596 (617)
-//     lin/min/max                77 (76), 281 (237), 749 (636)     / 83 (86), 283 (269), 812 (713)
-//   reference arithmetic         81 (89), 261 (250), 709 (682)     / 83 (92), 254 (266), 710 (723)
-//     clipped                    116 (126), 352 (364), 949 (987)   / 85 (128), 250 (379), 687 (1018)
-//     lin/min/max                115 (126), 383 (395), 1027 (1068) / 108 (135), 340 (417), 940 (1129)
-//   FP64                         112 (120), 377 (351), 995 (946)   / 116 (122), 359 (358), 1029 (949)
-//     clipped                    143 (141), 439 (417), 1156 (1122) / 122 (142), 362 (431), 1016 (1160)
-//     lin/min/max                168 (145), 554 (447), 1449 (1186) / 181 (151), 600 (458), 1630 (1225)
-//   BF16                         88 (87), 249 (233), 737 (667)     / 90 (92), 252 (257), 774 (725)
-//     lin/min/max                101 (93), 337 (270), 880 (737)    / 108 (103), 342 (300), 938 (809)
+//   FP32 arithmetic              61 (74), 199 (216), 535 (582)     / 64 (78), 201 (233), 560 (631)
+//     clipped                    61 (76), 204 (215), 535 (579)     / 68 (78), 213 (228), 596 (617)
+//     lin/min/max                77 (77), 259 (240), 713 (647)     / 83 (86), 283 (269), 812 (713)
+//   reference arithmetic         81 (90), 262 (252), 699 (685)     / 83 (92), 254 (266), 710 (723)
+//     clipped                    116 (127), 351 (367), 942 (991)   / 85 (128), 250 (379), 687 (1018)
+//     lin/min/max                116 (126), 376 (385), 996 (1041)  / 108 (135), 340 (417), 940 (1129)
+//   FP64                         112 (120), 378 (350), 996 (939)   / 116 (122), 359 (358), 1029 (949)
+//     clipped                    143 (141), 440 (414), 1162 (1101) / 122 (142), 362 (431), 1016 (1160)
+//     lin/min/max                169 (145), 543 (445), 1450 (1186) / 181 (151), 600 (458), 1630 (1225)
+//   BF16                         88 (87), 250 (232), 734 (661)     / 90 (92), 252 (257), 774 (725)
+//     clipped                    89 (93), 249 (250), 749 (707)
+//     lin/min/max                101 (92), 333 (268), 905 (734)    / 108 (103), 342 (300), 938 (809)
 bool few_fields(int fdtype, int math, int post, long targets, int fields, bool plan) {
   if (fields > 1 || fdtype == ADZ_BF16) return false;
   const bool few = targets < (1L << 23);
@@ -1710,15 +1713,15 @@ bool few_fields(int fdtype, int math, int post, long targets, int fields, bool p
 // Built-in tile parameters: ten fields per pass, LDS-staged boxes of tiles of 64 x 4 targets x
 // 2 levels (stage 7; its eight-wave blocks leave the most of them on a CU).  Times of stage 7
 // (of stage 5, stage 8, per-lane loads), ms:
-//   16 subdomains to 512 x 384 x 6 FP32 fields, FP32 arithmetic  3.84 (4.94, 5.09, 6.22)
-//   10 fields with lin/min/max, 1024 x 512 x 84                  3.51 (4.30, 3.70, 6.87)
-//   10 fields with lin/min/max, 2048 x 1024 x 84                14.2 (17.4, 14.7, 30.1)
-//   4 clipped FP32 fields, reference arithmetic, the same grid   8.73 (8.99, -, 11.1)
-//   4 FP64 fields, 511 x 385 x 84                                0.71 (1.02, -, 1.29)
-//   4 clipped BF16 fields, 600 x 400 x 60                        0.57 (0.65, 0.73, 1.07)
-// Tiles walk rows, then levels, where lin/min/max are stored (levels first, 3.95 and 15.5 ms
-// in lines two and three), else the levels of a column first (rows first 3.95 ms in line
-// one); FP64 fields super-columns of two tile rows (line five; rows first 0.77).
+//   16 subdomains to 512 x 384 x 6 FP32 fields, FP32 arithmetic  3.70 (4.90, 5.20, 6.26)
+//   10 fields with lin/min/max, 1024 x 512 x 84                  3.35 (4.31, 3.67, 7.20)
+//   10 fields with lin/min/max, 2048 x 1024 x 84                13.6 (17.6, 15.1, 33.1)
+//   4 clipped FP32 fields, reference arithmetic, the same grid   8.02 (8.27, -, 8.08)
+//   4 FP64 fields, 511 x 385 x 84                                0.71 (1.03, -, 1.32)
+//   4 clipped BF16 fields, 600 x 400 x 60                        0.48 (0.54, 0.63, 0.89)
+// Tiles walk rows, then levels, where lin/min/max are stored (levels first, 3.88 and 15.5 ms
+// in lines two and three), else the levels of a column first (rows first 3.87 ms in line
+// one); FP64 fields super-columns of two tile rows (line five; rows first 0.75).
 // Too few fields (few_fields), and plans of which every item is beyond 32-bit offsets: per-lane
 // loads (stage 2).  Such an item among others reads per lane in the staged kernel: six subdomains
 // of 64 x 48 to 512 x 384 and one more with a source of 2600 x 2600 x 84, 6 FP32 fields, 1.53 ms

@@ -38,9 +38,9 @@
 !   * With F_post present, tracers whose meta has mono == 1 are clipped to [min, max]
 !     inside the interpolation launch (the same operation adz_post_tr.F90:81-94 applies to
 !     the same box afterwards), so adz_post_tr(1|2) runs ILMC and registers the fixer's
-!     tracers only.  ILMC runs once for all mono = 2 tracers of a group (one launch per
-!     hyperplane for all of them); each tracer's result is the sequential loop's, as the
-!     tracers do not interact.
+!     tracers only.  ILMC runs once for all mono = 2 tracers of a group (one launch sequence
+!     for all of them); each tracer's result is the sequential loop's, as the tracers do not
+!     interact.
 !   * The carried mass deficits stay on the device from one Bermejo_Conde call to the
 !     next (Adz_bc_deficit).  They are read from F_bc(:)%mass_deficit on the first call and
 !     whenever Adz_bc_deficit_upload_L is set (after a restart), and written back into
