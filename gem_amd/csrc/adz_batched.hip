@@ -1168,9 +1168,11 @@ __device__ __forceinline__ void eval_rows(Acc at, const double* c, double* v, do
   }
 }
 
-template <class TF, int MATH, int POST, class TP, int TH, int TL, class Fields>
+// (the tile order is ORDER, or with -1 the argument)
+template <class TF, int MATH, int POST, class TP, int TH, int TL, int ORDER, class Fields>
 __device__ __forceinline__ void dma_tile(const DevItem& it, const Fields& F, long ptile, int f0, int f1, TF* boxA,
-                                         TF* boxB, int* red, unsigned nth, int level_inner) {
+                                         TF* boxB, int* red, unsigned nth, int order) {
+  const int level_inner = ORDER < 0 ? order : ORDER;
   constexpr int W = TH * TL;                  // waves of the block: one per target row and level
   constexpr int S = dma_waves(sizeof(TF), W, MATH, POST);  // waves per SIMD
   constexpr int kRows = box_rows<TF, W, S>(), kN = dma_per_wave<TF, W, S>();
@@ -1487,11 +1489,11 @@ __global__ __launch_bounds__(64 * TH * TL, dma_waves(sizeof(TF), TH * TL, MATH, 
     const long t = tile_of_block(A.ntiles, A.xcd_chunks);
     if (t >= A.ntiles) return;  // the whole block leaves: no barrier is reached
     const PlanTile P = plan_tile(A, t);
-    dma_tile<TF, MATH, POST, TP, TH, TL>(P.it, P.fields(), P.ptile, P.f0, P.f1, boxA, boxB, red, 0, A.level_inner);
+    dma_tile<TF, MATH, POST, TP, TH, TL, -1>(P.it, P.fields(), P.ptile, P.f0, P.f1, boxA, boxB, red, 0, A.level_inner);
   } else {
     unsigned nth = 0;
     each_tile(A, [&](const PlanTile& P) {
-      dma_tile<TF, MATH, POST, TP, TH, TL>(P.it, P.fields(), P.ptile, P.f0, P.f1, boxA, boxB, red, nth++,
+      dma_tile<TF, MATH, POST, TP, TH, TL, -1>(P.it, P.fields(), P.ptile, P.f0, P.f1, boxA, boxB, red, nth++,
                                            A.level_inner);
     });
   }
@@ -1512,21 +1514,15 @@ __global__ __launch_bounds__(kTile) void k_hlt(DevItem it, InlineFields F) {
 // 200 x 150 grid and four fifths of a 512 x 384 one fitted: 3 fields of 200 x 150 x 60 in the
 // reference's arithmetic 63.7 -> 46.7 us; in FP32, 4 fields of 512 x 384 x 84 681 -> 399 us,
 // 8 of 2048 x 1024 x 84 13.4 -> 7.0 ms.
-// Tile order: super-columns of three tile rows, which read a source plane again while it is in
-// an XCD's L2; rows, then levels, where lin/min/max are stored, whose streams prefer it.  us,
-// super-columns (rows): 512 x 384 x 84, smooth positions, 4 FP64 fields 705 (735), 4 FP32 419
-// (426), 2 FP32 with lin/min/max 355 (342); sheared by up to 0.8 cells per cell, 4 FP64 2276
-// (2899), 4 FP32 1299 (1686); 3 fields of 200 x 150 x 60, reference arithmetic, 52.4 (50.3).
-constexpr int hlt_order(int post) { return post & ADZ_POST_STORE ? 0 : 3; }
 constexpr int kHltTH = kTJ, kHltTL = 2;
 
-template <class TF, class TP, int MATH, int POST>
+template <class TF, class TP, int MATH, int POST, int ORDER>
 __global__ __launch_bounds__(64 * kHltTH * kHltTL,
                                   dma_waves(sizeof(TF), kHltTH * kHltTL, MATH, POST)) void k_hlt5(DevItem it, InlineFields F, long ntiles) {
   ADZ_BOXES(TF, kHltTH * kHltTL, dma_waves(sizeof(TF), kHltTH * kHltTL, MATH, POST))
   const long t = tile_of_block(ntiles, 1);
   if (t >= ntiles) return;  // the whole block leaves: no barrier is reached
-  dma_tile<TF, MATH, POST, TP, kHltTH, kHltTL>(it, F, t, 0, it.nf, boxA, boxB, red, 0, hlt_order(POST));
+  dma_tile<TF, MATH, POST, TP, kHltTH, kHltTL, ORDER>(it, F, t, 0, it.nf, boxA, boxB, red, 0, ORDER);
 }
 
 }  // namespace adz
@@ -1649,14 +1645,24 @@ void* pick_plan(int post, int stage) {
     default: return (void*)&k_plan<TF, TP, M, 3, 2>;
   }
 }
+// Tile order of the staged call (ORDER of k_hlt5): rows, then levels, where the eight or so planes
+// of all fields that a level's stencils span are at most four times an XCD's 4 MB of L2, and where
+// lin/min/max are stored, whose streams prefer it; else super-columns of three tile rows, which
+// read a source plane again while it is there.  Super-columns over rows, smooth positions: 8 FP32
+// fields of 304 x 227 x 84 (15 MB) 1.03, of 512 x 384 x 84 (45 MB) 0.95, 4 FP64 fields 1.03 and
+// 0.96, 2 FP32 fields of 512 x 384 x 84 with lin/min/max 1.04; positions sheared by up to 0.8 cells
+// per cell, 512 x 384 x 84, 4 FP64 fields 0.79, 4 FP32 0.77.
+int hlt_order(const DevItem& it, int fields, int size, int post) {
+  return (post & ADZ_POST_STORE) || (long)it.nx * it.ny * 8 * fields * size <= (16L << 20) ? 0 : 3;
+}
 template <class TF, class TP, int M>
-void* pick_hlt(int post, bool staged) {
+void* pick_hlt(int post, bool staged, int order) {
   if (staged) {
     switch (post) {
-      case 0: return (void*)&k_hlt5<TF, TP, M, 0>;
-      case 1: return (void*)&k_hlt5<TF, TP, M, 1>;
-      case 2: return (void*)&k_hlt5<TF, TP, M, 2>;
-      default: return (void*)&k_hlt5<TF, TP, M, 3>;
+      case 0: return order ? (void*)&k_hlt5<TF, TP, M, 0, 3> : (void*)&k_hlt5<TF, TP, M, 0, 0>;
+      case 1: return (void*)&k_hlt5<TF, TP, M, 1, 0>;
+      case 2: return order ? (void*)&k_hlt5<TF, TP, M, 2, 3> : (void*)&k_hlt5<TF, TP, M, 2, 0>;
+      default: return (void*)&k_hlt5<TF, TP, M, 3, 0>;
     }
   }
   switch (post) {
@@ -1668,8 +1674,8 @@ void* pick_hlt(int post, bool staged) {
 }
 
 template <bool PLAN>
-void* pick(int fdt, int pdt, int math, int post, int stage = 2) {
-#define P_(TF, TP, M) return PLAN ? pick_plan<TF, TP, M>(post, stage) : pick_hlt<TF, TP, M>(post, stage != 2)
+void* pick(int fdt, int pdt, int math, int post, int stage = 2, int order = 0) {
+#define P_(TF, TP, M) return PLAN ? pick_plan<TF, TP, M>(post, stage) : pick_hlt<TF, TP, M>(post, stage != 2, order)
   if (math == ADZ_MATH_REF) {
     if (fdt == ADZ_F64 && pdt == ADZ_F64) P_(double, double, ADZ_MATH_REF);
     if (fdt == ADZ_F64 && pdt == ADZ_F32) P_(double, float, ADZ_MATH_REF);
@@ -1811,9 +1817,10 @@ int adz_tricub_hlt(const adz_field* fld, int nptr, const void* xyz, int pdtype, 
     }
     const bool staged = stageable(it, field_bytes(fdtype)) &&
                         !few_fields(fdtype, math, post, (long)it.nx * it.ny * it.nz, nf, false);
-    void* kern = pick<false>(fdtype, pdtype, math, post, staged ? 7 : 2);
+    const int order = hlt_order(it, nf, field_bytes(fdtype), post);
+    void* kern = pick<false>(fdtype, pdtype, math, post, staged ? 7 : 2, order);
     if (staged) {  // k_hlt5: LDS-staged boxes, an eighth of the tile list per XCD
-      long ntiles = item_ptiles(it.nx, it.ny, it.nz, hlt_order(post), kTI, kHltTH, kHltTL);
+      long ntiles = item_ptiles(it.nx, it.ny, it.nz, order, kTI, kHltTH, kHltTL);
       void* args[] = {&it, &F, &ntiles};
       ADZ_HIP_CHECK(hipLaunchKernel(kern, tile_grid(ntiles), dim3(64 * kHltTH * kHltTL), args, 0, (hipStream_t)stream));
     } else {
